@@ -1,6 +1,8 @@
 // mkf_find.hip -- best-hit track finding on gfx950.
 //
-//   LayerOfHits build   k_hit_keys -> stable LSD radix sort (hipCUB) -> k_loh_gather, k_loh_fill
+//   LayerOfHits build   k_row_partition -> k_row_sort (hits by q row, then each row in LDS), or, for layers
+//                       of few q bins and many hits, k_hit_keys -> stable LSD radix sort (hipCUB) ->
+//                       k_loh_gather, k_loh_fill
 //   SelectHitIndices    k_select (per-operation entry point)
 //   FindTracksBestHit   k_find_best_hit: one lane per seed carries its track
 //                       through every layer with the state in VGPRs; hit
@@ -48,13 +50,16 @@ constexpr int kOffChunk = 256;
 struct OffsetsArg {
   int first, count;
   int off[kOffChunk + 1];
+  int tile[kOffChunk + 1];      // first tile of k_row_partition per layer
 };
 
-__global__ void k_set_offsets(OffsetsArg o, LayerDev* __restrict__ L) {
+__global__ void k_set_offsets(OffsetsArg o, LayerDev* __restrict__ L, int* __restrict__ tile_off) {
   const int l = threadIdx.x;
   if (l < o.count) {
     L[o.first + l].hit_off = o.off[l];
     L[o.first + l].n_hits = o.off[l + 1] - o.off[l];
+    tile_off[o.first + l] = o.tile[l];
+    if (l + 1 == o.count) tile_off[o.first + o.count] = o.tile[o.count];
   }
 }
 
@@ -62,12 +67,15 @@ __global__ void k_fill_i32(int* __restrict__ p, long n, int v) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = v;
 }
 
+// Hit::r of an endcap hit (Hit.h:64-80); the FMA is written out so that every kernel forms the same bits.
+__device__ __forceinline__ float hit_r(float x, float y) { return sqrtf(__builtin_fmaf(x, x, y * y)); }
+
 // Hit::phi and Hit::z (barrel) / Hit::r (endcap) of a hit (Hit.h:64-80).  Not
 // inlined: the key kernel and the fill kernel run this one piece of machine
 // code, so the phi and q stored with a sorted hit are bit for bit the values
 // its sort key was formed from.
 __device__ __noinline__ float2 hit_phi_q(float x, float y, float z, int is_barrel) {
-  return make_float2(atan2_cr(y, x), is_barrel ? z : sqrtf(x * x + y * y));
+  return make_float2(atan2_cr(y, x), is_barrel ? z : hit_r(x, y));
 }
 
 // Layer owning event hit i: the last one in [lo, hi] whose hit range starts at
@@ -184,6 +192,300 @@ k_loh_fill(int total, int pass, const uint32_t* __restrict__ keys_s, const int* 
     }
     for (int b = max(pb + 1, 1); b < nb; ++b) row[b] = make_int2(local + 1, local + 1);
   }
+}
+
+// ---- LayerOfHits by q rows ---------------------------------------------------
+// A layer's order is (q bin, fine phi bin, hit index), and its hits arrive in one
+// run.  k_row_partition deals each tile of kTile hits of a layer into the layer's
+// q rows in LDS and writes the tile's (phi, index) pairs row by row, with the
+// tile's row starts; k_row_sort takes one row per block, collects its pairs from
+// the layer's tiles, orders them in LDS by fine phi bin and index, and writes
+// everything the finders read: the hits, phi, q, ranks, the inverse map and the
+// row's bin ranges.  A hit moves 36 + 8 bytes in the first kernel and 8 + 36 + 52
+// in the second, against 36 + 8, four radix passes of 16, 8 + 36 + 44 and 8 + 16
+// for keys, sort, gather and fill.
+constexpr int kTile = 3072;          // hits per tile; also the LDS capacity of k_row_sort, so one tile's part
+constexpr int kRowCap = kTile;       // of a row always fits
+constexpr int kPartBlock = 512, kRowBlock = 256;
+constexpr int kFineBins = 1025;      // fine phi bins 0..1024 (1024: phi == +pi)
+static_assert(kTile % kPartBlock == 0 && kRowCap % kRowBlock == 0 && kTile <= 0xffff, "tile size");
+// Layers with more hits than this per q bin go through the radix sort: one block per row leaves the chip idle.
+constexpr size_t kRowMeanMax = 2 * kRowCap;
+
+struct RowPair {
+  float phi;
+  int idx;      // hit index in its layer
+};
+
+__device__ __forceinline__ int fine_bin_clamped(float phi) {
+  return min(max(phi_bin_fine(phi), 0), kFineBins - 1);
+}
+
+// Exclusive prefix sum of v over the block's threads; *total gets the sum.  `part` holds a word per wavefront.
+template <int BLOCK>
+__device__ __forceinline__ int block_exclusive(int v, int* part, int* total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int incl = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += u;
+  }
+  if (lane == 63) part[wave] = incl;
+  __syncthreads();
+  int before = 0, sum = 0;
+#pragma unroll
+  for (int w = 0; w < BLOCK / 64; ++w) {
+    const int p = part[w];
+    before += w < wave ? p : 0;
+    sum += p;
+  }
+  __syncthreads();
+  *total = sum;
+  return before + incl - v;
+}
+
+__global__ void __launch_bounds__(kPartBlock)
+k_row_partition(int n_layers, const int* __restrict__ tile_off, const LayerDev* __restrict__ L,
+                const float* __restrict__ hits, RowPair* __restrict__ pairs, unsigned short* __restrict__ pre,
+                int pre_stride) {
+  __shared__ RowPair out[kTile];
+  __shared__ int hist[kMaxQBins];
+  __shared__ int part[kPartBlock / 64];
+  __shared__ int s_layer;
+  const int t = threadIdx.x, tile = blockIdx.x;
+  if (t < 64) {
+    // The layer holding the tile: the last of the layers whose first tile is at or before it, found in two
+    // steps of 64 lanes (of MKF_MAX_EOH_LAYERS = 64 * 32 layers).
+    constexpr int kStep = MKF_MAX_EOH_LAYERS / 64;
+    const int c = t * kStep;
+    const int coarse = __popcll(__ballot(c < n_layers && tile_off[min(c, n_layers)] <= tile)) - 1;
+    const int l = coarse * kStep + t;
+    const int fine = __popcll(__ballot(t < kStep && l < n_layers && tile_off[min(l, n_layers)] <= tile)) - 1;
+    if (t == 0) s_layer = coarse * kStep + fine;
+  }
+  for (int q = t; q < kMaxQBins; q += kPartBlock) hist[q] = 0;
+  __syncthreads();
+  const LayerDev& d = L[s_layer];
+  const int first = (tile - tile_off[s_layer]) * kTile;       // in the layer
+  const int n = min(kTile, d.n_hits - first);
+  const float* __restrict__ src = hits + (size_t)(d.hit_off + first) * 9;
+  constexpr int kPer = kTile / kPartBlock;
+  float x[kPer], y[kPer], z[kPer];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int j = min(t + k * kPartBlock, n - 1);
+    x[k] = src[(size_t)j * 9];
+    y[k] = src[(size_t)j * 9 + 1];
+    z[k] = src[(size_t)j * 9 + 2];
+  }
+  const bool barrel = d.is_barrel != 0;
+  int qb[kPer], rank[kPer];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    if (t + k * kPartBlock < n) {
+      qb[k] = q_bin_checked(d, barrel ? z[k] : hit_r(x[k], y[k]));
+      rank[k] = atomicAdd(&hist[qb[k]], 1);
+    }
+  }
+  __syncthreads();
+  // row starts within the tile
+  static_assert(kMaxQBins == 2 * kPartBlock, "two rows per thread");
+  const int h0 = hist[2 * t], h1 = hist[2 * t + 1];
+  int total;
+  const int e0 = block_exclusive<kPartBlock>(h0 + h1, part, &total);
+  hist[2 * t] = e0;
+  hist[2 * t + 1] = e0 + h0;
+  unsigned short* __restrict__ row = pre + (size_t)tile * pre_stride;
+  if (2 * t <= d.nq) row[2 * t] = (unsigned short)e0;
+  if (2 * t + 1 <= d.nq) row[2 * t + 1] = (unsigned short)(e0 + h0);
+  if (t == 0 && d.nq == kMaxQBins) row[kMaxQBins] = (unsigned short)n;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int j = t + k * kPartBlock;
+    if (j < n) out[hist[qb[k]] + rank[k]] = RowPair{atan2_cr(y[k], x[k]), first + j};
+  }
+  __syncthreads();
+  RowPair* __restrict__ dst = pairs + d.hit_off + first;
+  for (int j = t; j < n; j += kPartBlock) dst[j] = out[j];
+}
+
+// One q row per block; see above.  The pairs of a row come in any order within a
+// tile's part, so the order inside a fine phi bin (one to three hits) is set by
+// comparing indices.  Rows beyond the LDS capacity go through it in runs of whole
+// fine bins, and a single bin beyond it tile by tile, whose indices ascend.
+__global__ void __launch_bounds__(kRowBlock)
+k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, const int* __restrict__ tile_off,
+           const unsigned short* __restrict__ pre, int pre_stride, const RowPair* __restrict__ pairs,
+           const float* __restrict__ hits, float* __restrict__ shits, float* __restrict__ phis,
+           float* __restrict__ qs, int* __restrict__ ranks, int* __restrict__ inv, int2* __restrict__ bins) {
+  __shared__ float s_phi[kRowCap];
+  __shared__ int s_idx[kRowCap];
+  __shared__ int cur[kFineBins + 1];     // fine bin starts, then (as cursors) the ends of the bins placed so far
+  __shared__ int part[kRowBlock / 64];
+  __shared__ int s_b1, s_cnt;
+  const int t = threadIdx.x;
+  const int row = xcd_major_block();
+  const LayerDev& d = L[row_layer[row]];
+  const int q = row - d.bin_off / kNPhi;
+  const int nt = (d.n_hits + kTile - 1) / kTile;
+  const unsigned short* __restrict__ rp = pre + (size_t)tile_off[row_layer[row]] * pre_stride + q;
+  const RowPair* __restrict__ src = pairs + d.hit_off;
+  const float* __restrict__ lhits = hits + (size_t)d.hit_off * 9;
+  int c = 0, before = 0;
+  for (int i = t; i < nt; i += kRowBlock) {
+    const int a = rp[(size_t)i * pre_stride];
+    before += a;
+    c += rp[(size_t)i * pre_stride + 1] - a;
+  }
+  int n, start;                          // hits of the row, its first position in the layer
+  block_exclusive<kRowBlock>(c, part, &n);
+  block_exclusive<kRowBlock>(before, part, &start);
+  int2* __restrict__ brow = bins + d.bin_off + q * kNPhi;
+  if (n == 0) {
+    brow[t] = make_int2(0, 0);
+    return;
+  }
+  for (int b = t; b <= kFineBins; b += kRowBlock) cur[b] = 0;
+  __syncthreads();
+  // every pair of the row, 16 lanes per tile's part
+  auto each_pair = [&](int i0, int i1, auto&& f) {
+    for (int i = i0 + (t >> 4); i < i1; i += kRowBlock / 16) {
+      const int lo = rp[(size_t)i * pre_stride], hi = rp[(size_t)i * pre_stride + 1];
+      for (int j = lo + (t & 15); j < hi; j += 16) f(src[(size_t)i * kTile + j]);
+    }
+  };
+  each_pair(0, nt, [&](const RowPair& p) { atomicAdd(&cur[fine_bin_clamped(p.phi)], 1); });
+  __syncthreads();
+  {
+    constexpr int kPer = (kFineBins + kRowBlock) / kRowBlock;
+    int h[kPer], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int b = t * kPer + k;
+      h[k] = b <= kFineBins ? cur[b] : 0;
+      sum += h[k];
+    }
+    int total;
+    int e = block_exclusive<kRowBlock>(sum, part, &total);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int b = t * kPer + k;
+      if (b <= kFineBins) cur[b] = e;
+      e += h[k];
+    }
+  }
+  __syncthreads();
+  const int gbase = d.hit_off + start;
+  const bool barrel = d.is_barrel != 0;
+  // m ordered hits in s_phi / s_idx to row positions base..
+  auto write_out = [&](int base, int m) {
+    struct F3 { float a, b, c; };
+    const int g0 = gbase + base;
+    for (int f = t; f < m * 3; f += kRowBlock) {
+      const int h = f / 3, w = f - h * 3;
+      F3 v;
+      __builtin_memcpy(&v, lhits + (size_t)s_idx[h] * 9 + w * 3, 12);
+      __builtin_memcpy(shits + (size_t)g0 * 9 + (size_t)f * 3, &v, 12);
+      if (w == 0) qs[g0 + h] = barrel ? v.c : hit_r(v.a, v.b);
+    }
+    for (int h = t; h < m; h += kRowBlock) {
+      const int idx = s_idx[h];
+      phis[g0 + h] = s_phi[h];
+      ranks[g0 + h] = idx;
+      inv[d.hit_off + idx] = g0 + h;
+    }
+  };
+  // Puts each of the m entries, whose equal-bin group lies at [lo(e), hi(e)), at its place by index.
+  auto order = [&](int m, auto&& group) {
+    constexpr int kPer = kRowCap / kRowBlock;
+    float phi[kPer];
+    int idx[kPer], pos[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int s = t + k * kRowBlock;
+      if (s < m) {
+        phi[k] = s_phi[s];
+        idx[k] = s_idx[s];
+        const int2 r = group(phi[k]);
+        int p = r.x;
+        for (int i = r.x; i < r.y; ++i) p += s_idx[i] < idx[k];
+        pos[k] = p;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      if (t + k * kRowBlock < m) {
+        s_phi[pos[k]] = phi[k];
+        s_idx[pos[k]] = idx[k];
+      }
+    }
+    __syncthreads();
+  };
+  for (int b0 = 0; b0 < kFineBins;) {
+    const int base = cur[b0];
+    int b1 = kFineBins;
+    if (n > kRowCap) {                   // the longest run of bins from b0 that fits
+      if (t == 0) s_b1 = b0;
+      __syncthreads();
+      for (int b = b0 + 1 + t; b <= kFineBins; b += kRowBlock)
+        if (cur[b] - base <= kRowCap) atomicMax(&s_b1, b);
+      __syncthreads();
+      b1 = s_b1;
+      __syncthreads();
+    }
+    if (b1 > b0) {
+      const int m = cur[b1] - base;      // cur[kFineBins] == n
+      __syncthreads();
+      each_pair(0, nt, [&](const RowPair& p) {
+        const int b = fine_bin_clamped(p.phi);
+        if (b >= b0 && b < b1) {
+          const int s = atomicAdd(&cur[b], 1) - base;
+          s_phi[s] = p.phi;
+          s_idx[s] = p.idx;
+        }
+      });
+      __syncthreads();
+      order(m, [&](float phi) {
+        const int b = fine_bin_clamped(phi);
+        return make_int2((b > b0 ? cur[b - 1] : base) - base, cur[b] - base);
+      });
+      write_out(base, m);
+      b0 = b1;
+    } else {                             // one bin beyond the capacity
+      int done = 0;
+      for (int i = 0; i < nt; ++i) {
+        if (t == 0) s_cnt = 0;
+        __syncthreads();
+        each_pair(i, i + 1, [&](const RowPair& p) {
+          if (fine_bin_clamped(p.phi) == b0) {
+            const int s = atomicAdd(&s_cnt, 1);
+            s_phi[s] = p.phi;
+            s_idx[s] = p.idx;
+          }
+        });
+        __syncthreads();
+        const int m = s_cnt;
+        order(m, [&](float) { return make_int2(0, m); });
+        write_out(base + done, m);
+        done += m;
+        __syncthreads();
+      }
+      if (t == 0) cur[b0] = base + done;
+      ++b0;
+    }
+    __syncthreads();
+  }
+  // Bin ranges (HitStructures.cc:146-171), as k_loh_fill's two passes leave them: an empty bin 1..255 of a row
+  // with hits below phi = +pi holds its insertion point, and the phi = +pi run takes over bin 0.
+  auto end_of = [&](int b) { return b < 0 ? 0 : cur[b]; };
+  const int lo = end_of(4 * t - 1), hi = end_of(4 * t + 3), regular = end_of(1023);
+  int2 r = make_int2(start + lo, start + hi);
+  if (regular == 0 || (t == 0 && hi == 0)) r = make_int2(0, 0);
+  if (t == 0 && n > regular) r = make_int2(start + regular, start + n);
+  brow[t] = r;
 }
 
 // The iteration's hit mask in sorted order: mask_s[inv[j]] = mask[j] for every event hit j.
@@ -380,41 +682,43 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
 namespace {
 
 void free_hit_arrays(mkf_event_of_hits* h) {
-  void* ps[] = {h->d_keys, h->d_keys_s, h->d_vals, h->d_vals_s,
-                h->d_phis, h->d_qs,     h->d_shits, h->d_ranks, h->d_inv,   h->d_temp};
+  void* ps[] = {h->d_phis, h->d_qs, h->d_shits, h->d_ranks, h->d_inv};
   for (void* p : ps)
     if (p) (void)hipFree(p);
-  h->d_keys = h->d_keys_s = nullptr;
-  h->d_vals = h->d_vals_s = h->d_ranks = h->d_inv = nullptr;
+  h->d_ranks = h->d_inv = nullptr;
   h->d_phis = h->d_qs = h->d_shits = nullptr;
-  h->d_temp = nullptr;
-  h->temp_bytes = 0;
   h->cap = 0;
 }
 
-int grow(mkf_event_of_hits* h, size_t total, hipStream_t st) {
-  if (total <= h->cap && h->d_temp) return MKF_OK;
+void free_sort_arrays(mkf_event_of_hits* h) {
+  if (h->d_sort) (void)hipFree(h->d_sort);
+  h->d_sort = nullptr;
+  h->sort_bytes = 0;
+}
+
+int grow(mkf_event_of_hits* h, size_t total, size_t sort_bytes, hipStream_t st) {
+  if (total <= h->cap && h->cap && sort_bytes <= h->sort_bytes) return MKF_OK;
   HIP_TRY(hipStreamSynchronize(st));
   HIP_TRY(hipDeviceSynchronize());
-  free_hit_arrays(h);
-  const size_t cap = std::max<size_t>(total, 1024);
-  HIP_TRY(hipMalloc(&h->d_keys, cap * 4));
-  HIP_TRY(hipMalloc(&h->d_keys_s, cap * 4));
-  HIP_TRY(hipMalloc(&h->d_vals, cap * 4));
-  HIP_TRY(hipMalloc(&h->d_vals_s, cap * 4));
-  HIP_TRY(hipMalloc(&h->d_phis, cap * 4));
-  HIP_TRY(hipMalloc(&h->d_qs, cap * 4));
-  HIP_TRY(hipMalloc(&h->d_ranks, cap * 4));
-  HIP_TRY(hipMalloc(&h->d_inv, cap * 4));
-  HIP_TRY(hipMalloc(&h->d_shits, cap * 9 * 4));
-  size_t tb = 0;
-  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, h->d_keys, h->d_keys_s, h->d_vals, h->d_vals_s, (int)cap,
-                                             0, 32, st));
-  HIP_TRY(hipMalloc(&h->d_temp, tb));
-  h->temp_bytes = tb;
-  h->cap = cap;
+  if (total > h->cap || !h->cap) {
+    free_hit_arrays(h);
+    const size_t cap = std::max<size_t>(total, 1024);
+    HIP_TRY(hipMalloc(&h->d_phis, cap * 4));
+    HIP_TRY(hipMalloc(&h->d_qs, cap * 4));
+    HIP_TRY(hipMalloc(&h->d_ranks, cap * 4));
+    HIP_TRY(hipMalloc(&h->d_inv, cap * 4));
+    HIP_TRY(hipMalloc(&h->d_shits, cap * 9 * 4));
+    h->cap = cap;
+  }
+  if (sort_bytes > h->sort_bytes) {
+    free_sort_arrays(h);
+    HIP_TRY(hipMalloc(&h->d_sort, sort_bytes));
+    h->sort_bytes = sort_bytes;
+  }
   return MKF_OK;
 }
+
+size_t aligned(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 int blocks_for(size_t n, int block) { return (int)std::max<size_t>(1, (n + block - 1) / block); }
 
@@ -462,8 +766,19 @@ int mkf_event_of_hits_create(mkf_context* c, int n_layers, const mkf_layer_desc*
   h->n_layers = n_layers;
   h->layers = L;
   h->total_bins = bin_off;
+  std::vector<int> row_layer(bin_off / kNPhi);              // layer of each q row
+  for (int l = 0; l < n_layers; ++l) {
+    std::fill_n(row_layer.begin() + L[l].bin_off / kNPhi, L[l].nq, l);
+    h->max_nq = std::max(h->max_nq, L[l].nq);
+  }
   hipError_t e = hipMalloc(&h->d_layers, sizeof(LayerDev) * n_layers);
   if (e == hipSuccess) e = hipMemcpy(h->d_layers, L.data(), sizeof(LayerDev) * n_layers, hipMemcpyHostToDevice);
+  // first tile per layer (set by each load), then the rows' layers
+  if (e == hipSuccess) e = hipMalloc(&h->d_tile_off, sizeof(int) * (n_layers + 1 + row_layer.size()));
+  if (e == hipSuccess) {
+    h->d_row_layer = h->d_tile_off + n_layers + 1;
+    e = hipMemcpy(h->d_row_layer, row_layer.data(), sizeof(int) * row_layer.size(), hipMemcpyHostToDevice);
+  }
 
   if (e == hipSuccess) e = hipMalloc(&h->d_bins, sizeof(int2) * (size_t)bin_off);
   if (e != hipSuccess) {
@@ -480,6 +795,8 @@ int mkf_event_of_hits_destroy(mkf_event_of_hits* h) {
   (void)hipSetDevice(h->device);
   (void)hipDeviceSynchronize();
   free_hit_arrays(h);
+  free_sort_arrays(h);
+  if (h->d_tile_off) (void)hipFree(h->d_tile_off);
   if (h->d_ce_nodes) (void)hipFree(h->d_ce_nodes);
   if (h->d_mask_s) (void)hipFree(h->d_mask_s);
   if (h->d_charge_s) (void)hipFree(h->d_charge_s);
@@ -504,41 +821,80 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
   if (total >= ((size_t)1 << 31) - 1) return fail(MKF_ERR_INVALID_ARG, "too many hits in one event of hits");
   if (total) CHECK(check_dev(hits, total * 9 * 4, "hits"));
   hipStream_t st = (hipStream_t)stream;
-  CHECK(grow(h, total, st));
+  // Which way the hits are sorted: by q rows, unless a layer has so few q bins for its hits that one block per
+  // row would take longer than the radix sort of all.
+  bool rows = true;
+  int tiles = 0;
+  for (int l = 0; l < L; ++l) {
+    const size_t nl = (size_t)hit_offset[l + 1] - hit_offset[l];
+    rows = rows && nl <= kRowMeanMax * h->layers[l].nq;
+    tiles += (int)((nl + kTile - 1) / kTile);
+  }
+  const int pre_stride = h->max_nq + 1;
+  const size_t items = std::max<size_t>(total, 1024);
+  size_t temp = 0, need;
+  if (rows) {
+    need = aligned(items * sizeof(RowPair)) + (size_t)tiles * pre_stride * sizeof(unsigned short);
+  } else {
+    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, temp, (uint32_t*)nullptr, (uint32_t*)nullptr, (int*)nullptr,
+                                               (int*)nullptr, (int)items, 0, 32, st));
+    need = 4 * aligned(items * 4) + temp;
+  }
+  CHECK(grow(h, total, need, st));
   h->has_mask = false;
   h->has_charge = false;
   for (int l = 0; l < L; ++l) {
     h->layers[l].hit_off = hit_offset[l];
     h->layers[l].n_hits = hit_offset[l + 1] - hit_offset[l];
   }
-  for (int f = 0; f < L; f += kOffChunk) {
+  for (int f = 0, tile = 0; f < L; f += kOffChunk) {
     OffsetsArg o;
     o.first = f;
     o.count = std::min(kOffChunk, L - f);
-    for (int l = 0; l <= o.count; ++l) o.off[l] = hit_offset[f + l];
-    hipLaunchKernelGGL(k_set_offsets, dim3(1), dim3(kOffChunk), 0, st, o, h->d_layers);
+    for (int l = 0; l <= o.count; ++l) {
+      o.off[l] = hit_offset[f + l];
+      o.tile[l] = tile;
+      if (l < o.count) tile += (h->layers[f + l].n_hits + kTile - 1) / kTile;
+    }
+    hipLaunchKernelGGL(k_set_offsets, dim3(1), dim3(kOffChunk), 0, st, o, h->d_layers, h->d_tile_off);
     HIP_TRY(hipGetLastError());
   }
-  const int* bins_i = reinterpret_cast<const int*>(h->d_bins);
-  hipLaunchKernelGGL(k_fill_i32, dim3(std::min(blocks_for((size_t)h->total_bins * 2, 256), 4096)), dim3(256), 0, st,
-                     const_cast<int*>(bins_i), (long)h->total_bins * 2, 0);
-  HIP_TRY(hipGetLastError());
-  if (total) {
-    const int nt = (int)total;
-    hipLaunchKernelGGL(k_hit_keys, dim3(blocks_for(total, 256)), dim3(256), 0, st, nt, L, hits, h->d_layers,
-                       h->d_keys, h->d_vals);
-    HIP_TRY(hipGetLastError());
-    size_t tb = h->temp_bytes;
-    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(h->d_temp, tb, h->d_keys, h->d_keys_s, h->d_vals, h->d_vals_s, nt, 0,
-                                               32, st));
-    hipLaunchKernelGGL(k_loh_gather, dim3(blocks_for(total, 256)), dim3(256), 0, st, nt, h->d_keys_s, h->d_vals_s,
-                       h->d_layers, hits, h->d_shits, h->d_phis, h->d_qs);
-    HIP_TRY(hipGetLastError());
-    for (int pass = 0; pass < 2; ++pass) {
-      hipLaunchKernelGGL(k_loh_fill, dim3(blocks_for(total, 256)), dim3(256), 0, st, nt, pass, h->d_keys_s,
-                         h->d_vals_s, h->d_layers, h->d_ranks, h->d_inv, h->d_bins);
+  const int n_rows = h->total_bins / kNPhi;
+  if (rows) {
+    RowPair* pairs = static_cast<RowPair*>(h->d_sort);
+    unsigned short* pre = reinterpret_cast<unsigned short*>(static_cast<char*>(h->d_sort) +
+                                                            aligned(items * sizeof(RowPair)));
+    if (tiles) {
+      hipLaunchKernelGGL(k_row_partition, dim3(tiles), dim3(kPartBlock), 0, st, L, h->d_tile_off, h->d_layers, hits,
+                         pairs, pre, pre_stride);
       HIP_TRY(hipGetLastError());
     }
+    hipLaunchKernelGGL(k_row_sort, dim3(n_rows), dim3(kRowBlock), 0, st, h->d_row_layer, h->d_layers, h->d_tile_off,
+                       pre, pre_stride, pairs, hits, h->d_shits, h->d_phis, h->d_qs, h->d_ranks, h->d_inv, h->d_bins);
+    HIP_TRY(hipGetLastError());
+    h->loaded = true;
+    return MKF_OK;
+  }
+  hipLaunchKernelGGL(k_fill_i32, dim3(std::min(blocks_for((size_t)h->total_bins * 2, 256), 4096)), dim3(256), 0, st,
+                     reinterpret_cast<int*>(h->d_bins), (long)h->total_bins * 2, 0);
+  HIP_TRY(hipGetLastError());
+  const int nt = (int)total;
+  char* scr = static_cast<char*>(h->d_sort);
+  uint32_t* keys = reinterpret_cast<uint32_t*>(scr);
+  uint32_t* keys_s = reinterpret_cast<uint32_t*>(scr + aligned(items * 4));
+  int* vals = reinterpret_cast<int*>(scr + 2 * aligned(items * 4));
+  int* vals_s = reinterpret_cast<int*>(scr + 3 * aligned(items * 4));
+  hipLaunchKernelGGL(k_hit_keys, dim3(blocks_for(total, 256)), dim3(256), 0, st, nt, L, hits, h->d_layers, keys, vals);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(scr + 4 * aligned(items * 4), temp, keys, keys_s, vals, vals_s, nt, 0, 32,
+                                             st));
+  hipLaunchKernelGGL(k_loh_gather, dim3(blocks_for(total, 256)), dim3(256), 0, st, nt, keys_s, vals_s, h->d_layers,
+                     hits, h->d_shits, h->d_phis, h->d_qs);
+  HIP_TRY(hipGetLastError());
+  for (int pass = 0; pass < 2; ++pass) {
+    hipLaunchKernelGGL(k_loh_fill, dim3(blocks_for(total, 256)), dim3(256), 0, st, nt, pass, keys_s, vals_s,
+                       h->d_layers, h->d_ranks, h->d_inv, h->d_bins);
+    HIP_TRY(hipGetLastError());
   }
   h->loaded = true;
   return MKF_OK;

@@ -286,17 +286,16 @@ struct mkf_event_of_hits {
   int total_bins = 0;
   int2* d_bins = nullptr;
   size_t cap = 0;                 // hit capacity of the arrays below
-  uint32_t* d_keys = nullptr;
-  uint32_t* d_keys_s = nullptr;
-  int* d_vals = nullptr;
-  int* d_vals_s = nullptr;
+  int max_nq = 0;                 // most q bins of a layer
+  int* d_tile_off = nullptr;      // first hit tile of each layer, as of the last load
+  int* d_row_layer = nullptr;     // layer of each q row
   float* d_phis = nullptr;
   float* d_qs = nullptr;
   float* d_shits = nullptr;
   int* d_ranks = nullptr;
   int* d_inv = nullptr;           // event hit index -> sorted position (inverse of ranks)
-  void* d_temp = nullptr;
-  size_t temp_bytes = 0;
+  void* d_sort = nullptr;         // a load's scratch: pairs and row starts, or keys and radix sort buffers
+  size_t sort_bytes = 0;
   bool loaded = false;
   void* d_ce_nodes = nullptr;     // clone-engine HitOnTrack node store, then its best short candidates
   size_t ce_node_cap = 0;         // in 16-byte units

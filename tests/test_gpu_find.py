@@ -376,3 +376,82 @@ def test_hit_mask_matches_oracle(gpu_device):
     for k in a:
         assert np.array_equal(a[k], plain_bh[k]), k
     ctx.close()
+
+
+def _rows_of_keys(key, nq):
+    """Bin ranges of a layer from its hits' keys, as LayerOfHits::SuckInHits leaves them: the phi == +pi run
+    (fine bin 1024) of a row overwrites coarse bin 0."""
+    ks = np.sort(key)
+    bins = np.zeros((nq * 256, 2), np.int64)
+    for q in range(nq):
+        edge = np.searchsorted(ks, (q << 16) + np.append(np.arange(0, 1024, 4), [1024, 1025]))
+        for b in range(256):
+            if edge[b] < edge[b + 1]:
+                bins[q * 256 + b] = edge[b], edge[b + 1]
+        if edge[256] < edge[257]:
+            bins[q * 256] = edge[256], edge[257]
+    return bins
+
+
+@pytest.mark.parametrize("q_bin,is_barrel", [(0.15, 1), (2.0, 1), (30.0, 1), (120.0, 1), (1.5, 0), (60.0, 0)])
+def test_loh_order_for_row_and_tile_sizes(gpu_device, q_bin, is_barrel):
+    """Sizes around the tile and row capacity (3072 hits) and one hit or none, from 800 q bins down to one: rows
+    sorted in one go, rows beyond the capacity, and layers whose few bins send the load through the radix sort."""
+    import torch
+    rng = np.random.default_rng(int(q_bin * 100) + is_barrel)
+    sizes = [0, 1, 3071, 3072, 3073, 0, 9000, 40000, 2]
+    descs, hits = [], []
+    for n in sizes:
+        r = 20.0 if is_barrel else rng.uniform(2.0, 55.0, n)
+        phi = rng.uniform(-np.pi, np.pi, n)
+        z = rng.uniform(-62.0, 62.0, n) if is_barrel else np.full(n, 30.0)
+        if n > 1000:
+            phi[:200] = np.pi                              # fine bin 1024
+            phi[200:600] = phi[600]                        # one crowded fine bin
+        h = np.zeros((n, 9), np.float32)
+        h[:, 0], h[:, 1], h[:, 2] = r * np.cos(phi), r * np.sin(phi), z
+        h[:200, 1] = np.where(np.arange(len(h[:200])) % 2 == 0, 0.0, h[:200, 1]) if n > 1000 else h[:200, 1]
+        h[:, 3:] = rng.uniform(0.0, 1.0, (n, 6))
+        hits.append(h[rng.permutation(n)] if n > 1000 else h)
+        descs.append(dict(is_barrel=is_barrel, rin=2.0 if not is_barrel else 19.99, rout=50.0 if not is_barrel else 20.01,
+                          zmin=-60.0 if is_barrel else 29.99, zmax=60.0 if is_barrel else 30.01,
+                          propagate_to=20.0 if is_barrel else 30.0, q_bin=q_bin, min_dphi=0.002, max_dphi=0.1, min_dq=0.3,
+                          max_dq=2.0, c_dp_sf=1.1, c_dq_sf=1.1, c_c2_sf=1.1))
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    flat = np.concatenate(hits)
+    ctx = mk.Context(bfield=3.8)
+    eoh = mk.EventOfHits(ctx, descs)
+    eoh.load(off, torch.from_numpy(flat).to(gpu_device))
+    for l, h in enumerate(hits):
+        ranks, bins, phis, qs, nq = eoh.layer_views(l)
+        assert sorted(ranks.tolist()) == list(range(len(h)))
+        phi = np.empty_like(phis); phi[ranks] = phis
+        q = np.empty_like(qs); q[ranks] = qs
+        assert np.array_equal(phi, np.arctan2(h[:, 1].astype(np.float64), h[:, 0].astype(np.float64)).astype(np.float32))
+        r2 = h[:, 0].astype(np.float64) ** 2 + h[:, 1].astype(np.float64) ** 2
+        assert np.array_equal(q, h[:, 2]) if is_barrel else np.allclose(q, np.sqrt(r2), rtol=2e-7, atol=0)
+        d = descs[l]
+        lo, hi = np.float32(d["zmin"] if is_barrel else d["rin"]), np.float32(d["zmax"] if is_barrel else d["rout"])
+        extra = np.float32(0.5) * (np.float32(nq) * np.float32(q_bin) - (hi - lo))
+        qb = np.clip(((q - (lo - extra)) * (np.float32(nq) / (hi - lo))).astype(np.int64), 0, nq - 1)
+        key = np.floor(F_PHI_FINE * (phi + np.float32(np.pi))).astype(np.int64) + (qb << 16)
+        assert np.array_equal(ranks, np.argsort(key, kind="stable")), (l, len(h))
+        want = _rows_of_keys(key, nq)
+        full = want[:, 0] < want[:, 1]
+        assert np.array_equal(bins[full], want[full]) and np.all(bins[~full, 0] == bins[~full, 1]), (l, len(h))
+    # the sorted hits and the inverse map, through a selection mask: every hit masked but one stays found as itself
+    keep = int(off[-1]) - 1
+    mask = np.ones(off[-1], np.uint8); mask[keep] = 0
+    eoh.set_hit_mask(torch.from_numpy(mask).to(gpu_device))
+    last, n = len(sizes) - 1, 1
+    x, y, z = flat[keep, :3]
+    if abs(z) < 60.0:
+        par = np.array([[x], [y], [z], [0.5], [np.arctan2(y, x)], [1.2]], np.float32)
+        err = np.zeros((21, 1), np.float32)
+        err[[0, 2, 5, 9, 14, 20], 0] = 1e-4
+        t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu_device)
+        xs, xa, w = t(np.zeros(1, np.int32)), t(np.zeros((16, 1), np.int32)), t(np.zeros(1, np.int32))
+        eoh.select_hit_indices(last, t(par), t(err), xs, xa, w)
+        assert xs.item() == 1 and xa[0, 0].item() == sizes[last] - 1
+    eoh.close()
+    ctx.close()
