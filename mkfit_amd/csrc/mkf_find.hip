@@ -313,8 +313,11 @@ k_row_partition(int n_layers, const int* __restrict__ tile_off, const LayerDev* 
 
 // One q row per block; see above.  The pairs of a row come in any order within a
 // tile's part, so the order inside a fine phi bin (one to three hits) is set by
-// comparing indices.  Rows beyond the LDS capacity go through it in runs of whole
-// fine bins, and a single bin beyond it tile by tile, whose indices ascend.
+// comparing indices.  A row that fits the LDS is read once; what it reads from
+// memory is issued in batches, as the block waits on memory for most of its time.
+// Rows beyond the LDS capacity (or of layers with more tiles than threads) go
+// through it in runs of whole fine bins, and a single bin beyond it tile by tile,
+// whose indices ascend.
 __global__ void __launch_bounds__(kRowBlock)
 k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, const int* __restrict__ tile_off,
            const unsigned short* __restrict__ pre, int pre_stride, const RowPair* __restrict__ pairs,
@@ -323,42 +326,37 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
   __shared__ float s_phi[kRowCap];
   __shared__ int s_idx[kRowCap];
   __shared__ int cur[kFineBins + 1];     // fine bin starts, then (as cursors) the ends of the bins placed so far
+  __shared__ int s_seg[kRowBlock];       // each tile's part: first place in the tile << 16 | length
+  __shared__ int s_dst[kRowBlock];       // and the place of its first pair among the row's
   __shared__ int part[kRowBlock / 64];
   __shared__ int s_b1, s_cnt;
   const int t = threadIdx.x;
   const int row = xcd_major_block();
-  const LayerDev& d = L[row_layer[row]];
+  const int layer = row_layer[row];
+  const LayerDev& d = L[layer];
   const int q = row - d.bin_off / kNPhi;
   const int nt = (d.n_hits + kTile - 1) / kTile;
-  const unsigned short* __restrict__ rp = pre + (size_t)tile_off[row_layer[row]] * pre_stride + q;
+  const unsigned short* __restrict__ rp = pre + (size_t)tile_off[layer] * pre_stride + q;
   const RowPair* __restrict__ src = pairs + d.hit_off;
   const float* __restrict__ lhits = hits + (size_t)d.hit_off * 9;
+  for (int b = t; b <= kFineBins; b += kRowBlock) cur[b] = 0;
   int c = 0, before = 0;
   for (int i = t; i < nt; i += kRowBlock) {
-    const int a = rp[(size_t)i * pre_stride];
+    const int a = rp[(size_t)i * pre_stride], len = rp[(size_t)i * pre_stride + 1] - a;
     before += a;
-    c += rp[(size_t)i * pre_stride + 1] - a;
+    c += len;
+    s_seg[t] = a << 16 | len;
   }
   int n, start;                          // hits of the row, its first position in the layer
-  block_exclusive<kRowBlock>(c, part, &n);
+  s_dst[t] = block_exclusive<kRowBlock>(c, part, &n);
   block_exclusive<kRowBlock>(before, part, &start);
   int2* __restrict__ brow = bins + d.bin_off + q * kNPhi;
   if (n == 0) {
     brow[t] = make_int2(0, 0);
     return;
   }
-  for (int b = t; b <= kFineBins; b += kRowBlock) cur[b] = 0;
-  __syncthreads();
-  // every pair of the row, 16 lanes per tile's part
-  auto each_pair = [&](int i0, int i1, auto&& f) {
-    for (int i = i0 + (t >> 4); i < i1; i += kRowBlock / 16) {
-      const int lo = rp[(size_t)i * pre_stride], hi = rp[(size_t)i * pre_stride + 1];
-      for (int j = lo + (t & 15); j < hi; j += 16) f(src[(size_t)i * kTile + j]);
-    }
-  };
-  each_pair(0, nt, [&](const RowPair& p) { atomicAdd(&cur[fine_bin_clamped(p.phi)], 1); });
-  __syncthreads();
-  {
+  // cur: counts to starts
+  auto scan_bins = [&]() {
     constexpr int kPer = (kFineBins + kRowBlock) / kRowBlock;
     int h[kPer], sum = 0;
 #pragma unroll
@@ -375,20 +373,30 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
       if (b <= kFineBins) cur[b] = e;
       e += h[k];
     }
-  }
-  __syncthreads();
+    __syncthreads();
+  };
   const int gbase = d.hit_off + start;
   const bool barrel = d.is_barrel != 0;
   // m ordered hits in s_phi / s_idx to row positions base..
   auto write_out = [&](int base, int m) {
     struct F3 { float a, b, c; };
     const int g0 = gbase + base;
-    for (int f = t; f < m * 3; f += kRowBlock) {
-      const int h = f / 3, w = f - h * 3;
-      F3 v;
-      __builtin_memcpy(&v, lhits + (size_t)s_idx[h] * 9 + w * 3, 12);
-      __builtin_memcpy(shits + (size_t)g0 * 9 + (size_t)f * 3, &v, 12);
-      if (w == 0) qs[g0 + h] = barrel ? v.c : hit_r(v.a, v.b);
+    constexpr int kBatch = 6;
+    for (int f0 = t; f0 < m * 3; f0 += kRowBlock * kBatch) {
+      F3 v[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int f = min(f0 + u * kRowBlock, m * 3 - 1), h = f / 3;
+        __builtin_memcpy(&v[u], lhits + (size_t)s_idx[h] * 9 + (f - h * 3) * 3, 12);
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int f = f0 + u * kRowBlock, h = f / 3;
+        if (f < m * 3) {
+          __builtin_memcpy(shits + (size_t)g0 * 9 + (size_t)f * 3, &v[u], 12);
+          if (f == h * 3) qs[g0 + h] = barrel ? v[u].c : hit_r(v[u].a, v[u].b);
+        }
+      }
     }
     for (int h = t; h < m; h += kRowBlock) {
       const int idx = s_idx[h];
@@ -397,7 +405,97 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
       inv[d.hit_off + idx] = g0 + h;
     }
   };
-  // Puts each of the m entries, whose equal-bin group lies at [lo(e), hi(e)), at its place by index.
+  auto write_bins = [&](auto&& start_of) {
+    // Bin ranges (HitStructures.cc:146-171), as k_loh_fill's two passes leave them: an empty bin 1..255 of a row
+    // with hits below phi = +pi holds its insertion point, and the phi = +pi run takes over bin 0.
+    const int lo = start_of(4 * t), hi = start_of(4 * t + 4), regular = start_of(1024);
+    int2 r = make_int2(start + lo, start + hi);
+    if (regular == 0 || (t == 0 && hi == 0)) r = make_int2(0, 0);
+    if (t == 0 && n > regular) r = make_int2(start + regular, start + n);
+    brow[t] = r;
+  };
+  if (n <= kRowCap && nt <= kRowBlock) {
+    // 32 lanes per tile's part, four parts' loads in flight
+    constexpr int kGroups = kRowBlock / 32, kSegs = 4;
+    const int g = t >> 5, gl = t & 31;
+    for (int i0 = g; i0 < nt; i0 += kGroups * kSegs) {
+      RowPair p[kSegs];
+      int len[kSegs], dst[kSegs];
+#pragma unroll
+      for (int u = 0; u < kSegs; ++u) {
+        const int i = i0 + u * kGroups;
+        const int seg = i < nt ? s_seg[i] : 0;
+        len[u] = seg & 0xffff;
+        dst[u] = i < nt ? s_dst[i] : 0;
+        if (gl < len[u]) p[u] = src[(size_t)i * kTile + (seg >> 16) + gl];
+      }
+#pragma unroll
+      for (int u = 0; u < kSegs; ++u) {
+        if (gl < len[u]) {
+          s_phi[dst[u] + gl] = p[u].phi;
+          s_idx[dst[u] + gl] = p[u].idx;
+        }
+        for (int j = gl + 32; j < len[u]; j += 32) {
+          const int i = i0 + u * kGroups;
+          const RowPair r = src[(size_t)i * kTile + (s_seg[i] >> 16) + j];
+          s_phi[dst[u] + j] = r.phi;
+          s_idx[dst[u] + j] = r.idx;
+        }
+      }
+    }
+    __syncthreads();
+    constexpr int kPer = kRowCap / kRowBlock;
+    float phi[kPer];
+    int idx[kPer], at[kPer];             // at: fine bin << 16 | place in it; then the place in the row
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int s = t + k * kRowBlock;
+      if (s < n) {
+        phi[k] = s_phi[s];
+        idx[k] = s_idx[s];
+        const int b = fine_bin_clamped(phi[k]);
+        at[k] = b << 16 | atomicAdd(&cur[b], 1);
+      }
+    }
+    __syncthreads();
+    scan_bins();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (t + k * kRowBlock < n) s_idx[cur[at[k] >> 16] + (at[k] & 0xffff)] = idx[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      if (t + k * kRowBlock < n) {
+        const int lo = cur[at[k] >> 16], hi = cur[(at[k] >> 16) + 1];
+        int p = lo;
+        for (int i = lo; i < hi; ++i) p += s_idx[i] < idx[k];
+        at[k] = p;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      if (t + k * kRowBlock < n) {
+        s_phi[at[k]] = phi[k];
+        s_idx[at[k]] = idx[k];
+      }
+    }
+    __syncthreads();
+    write_out(0, n);
+    write_bins([&](int b) { return cur[b]; });
+    return;
+  }
+  // every pair of the row, 16 lanes per tile's part
+  auto each_pair = [&](int i0, int i1, auto&& f) {
+    for (int i = i0 + (t >> 4); i < i1; i += kRowBlock / 16) {
+      const int lo = rp[(size_t)i * pre_stride], hi = rp[(size_t)i * pre_stride + 1];
+      for (int j = lo + (t & 15); j < hi; j += 16) f(src[(size_t)i * kTile + j]);
+    }
+  };
+  each_pair(0, nt, [&](const RowPair& p) { atomicAdd(&cur[fine_bin_clamped(p.phi)], 1); });
+  __syncthreads();
+  scan_bins();
+  // Puts each of the m entries, whose equal-bin group lies at [x, y) = group(phi), at its place by index.
   auto order = [&](int m, auto&& group) {
     constexpr int kPer = kRowCap / kRowBlock;
     float phi[kPer];
@@ -426,16 +524,13 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
   };
   for (int b0 = 0; b0 < kFineBins;) {
     const int base = cur[b0];
-    int b1 = kFineBins;
-    if (n > kRowCap) {                   // the longest run of bins from b0 that fits
-      if (t == 0) s_b1 = b0;
-      __syncthreads();
-      for (int b = b0 + 1 + t; b <= kFineBins; b += kRowBlock)
-        if (cur[b] - base <= kRowCap) atomicMax(&s_b1, b);
-      __syncthreads();
-      b1 = s_b1;
-      __syncthreads();
-    }
+    // the longest run of bins from b0 that fits
+    if (t == 0) s_b1 = b0;
+    __syncthreads();
+    for (int b = b0 + 1 + t; b <= kFineBins; b += kRowBlock)
+      if (cur[b] - base <= kRowCap) atomicMax(&s_b1, b);
+    __syncthreads();
+    const int b1 = s_b1;
     if (b1 > b0) {
       const int m = cur[b1] - base;      // cur[kFineBins] == n
       __syncthreads();
@@ -478,14 +573,7 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
     }
     __syncthreads();
   }
-  // Bin ranges (HitStructures.cc:146-171), as k_loh_fill's two passes leave them: an empty bin 1..255 of a row
-  // with hits below phi = +pi holds its insertion point, and the phi = +pi run takes over bin 0.
-  auto end_of = [&](int b) { return b < 0 ? 0 : cur[b]; };
-  const int lo = end_of(4 * t - 1), hi = end_of(4 * t + 3), regular = end_of(1023);
-  int2 r = make_int2(start + lo, start + hi);
-  if (regular == 0 || (t == 0 && hi == 0)) r = make_int2(0, 0);
-  if (t == 0 && n > regular) r = make_int2(start + regular, start + n);
-  brow[t] = r;
+  write_bins([&](int b) { return b > 0 ? cur[b - 1] : 0; });
 }
 
 // The iteration's hit mask in sorted order: mask_s[inv[j]] = mask[j] for every event hit j.
