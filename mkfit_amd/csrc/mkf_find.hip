@@ -212,6 +212,11 @@ static_assert(kTile % kPartBlock == 0 && kRowCap % kRowBlock == 0 && kTile <= 0x
 // Layers with more hits than this per q bin go through the radix sort: one block per row leaves the chip idle.
 constexpr size_t kRowMeanMax = 2 * kRowCap;
 
+// Beyond this many hits the sorted copies are stored past the caches: the 256 MB last-level cache no longer keeps
+// them for the finder (best-hit step, stored past / through the caches: 562 / 516 us at 2.8M hits, 723 / 742 at
+// 5.7M, 1517 / 1559 at 22.7M).
+constexpr size_t kStreamHits = 4000000;
+
 struct RowPair {
   float phi;
   int idx;      // hit index in its layer
@@ -324,6 +329,7 @@ k_row_partition(int n_layers, const int* __restrict__ tile_off, const LayerDev* 
 // Rows beyond the LDS capacity (or of layers with more tiles than threads) go
 // through it in runs of whole fine bins, and a single bin beyond it tile by tile,
 // whose indices ascend.
+template <bool NT>
 __global__ void __launch_bounds__(kRowBlock)
 k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, const int* __restrict__ tile_off,
            const unsigned short* __restrict__ pre, int pre_stride, const RowPair* __restrict__ pairs,
@@ -384,6 +390,10 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
   };
   const int gbase = d.hit_off + start;
   const bool barrel = d.is_barrel != 0;
+  auto put_out = [](float* p, float v) {
+    if (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+  };
   // m ordered hits in s_phi / s_idx to row positions base..
   auto write_out = [&](int base, int m) {
     struct F3 { float a, b, c; };
@@ -401,16 +411,16 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
         const int f = f0 + u * kRowBlock, h = f / 3;
         if (f < m * 3) {
           float* o = shits + (size_t)g0 * 9 + (size_t)f * 3;
-          __builtin_nontemporal_store(v[u].a, o);
-          __builtin_nontemporal_store(v[u].b, o + 1);
-          __builtin_nontemporal_store(v[u].c, o + 2);
-          if (f == h * 3) __builtin_nontemporal_store(barrel ? v[u].c : hit_r(v[u].a, v[u].b), qs + g0 + h);
+          put_out(o, v[u].a);
+          put_out(o + 1, v[u].b);
+          put_out(o + 2, v[u].c);
+          if (f == h * 3) put_out(qs + g0 + h, barrel ? v[u].c : hit_r(v[u].a, v[u].b));
         }
       }
     }
     for (int h = t; h < m; h += kRowBlock) {
       const int idx = s_idx[h];
-      __builtin_nontemporal_store(s_phi[h], phis + g0 + h);
+      put_out(phis + g0 + h, s_phi[h]);
       ranks[g0 + h] = idx;
     }
   };
@@ -665,7 +675,7 @@ k_select(LayerDev d, int n, const float* __restrict__ par, const float* __restri
 // ---- FindTracksBestHit -------------------------------------------------------
 
 struct FindArgs {
-  int n, n_layers, first_layer, eoh_layers;
+  int n, n_layers, first_layer, eoh_layers, spw;
   const int* __restrict__ layer_base;
   float chi2_cut;
   int pflags, prop_to_hit, intra_pflags;
@@ -686,34 +696,58 @@ struct FindArgs {
   const int* __restrict__ ranks;
 };
 
-// The reference's block loop (MkBuilder.cc:1395-1478) per lane.  A lane that
-// stops leaves the loop with the state it had at that point, which is the
-// state the reference outputs for it (OutputTrackAndHitIdx at stop time).
-// HitOnTrack bookkeeping as MkFinder::add_hit (MkFinder.h:312-354); with at
-// most MKF_MAX_FIND_LAYERS layers a track never exceeds Config::nMaxTrkHits.
-// Two waves per SIMD: 2.33 ms per 50 events, against 2.45 ms at three waves (168 VGPRs, 94 spilled)
-// and 2.70 ms at four.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) k_find_best_hit(FindArgs a) {
-  __shared__ int s_cand[kHitIdxMax][256];     // each thread's window hits of the layer, in scan order
-  const int stride = gridDim.x * blockDim.x;
+// The reference's block loop (MkBuilder.cc:1395-1478), one wavefront per workgroup
+// and one lane per seed for everything but the hits.  A lane that stops keeps the
+// state it had at that point, which is the state the reference outputs for it
+// (OutputTrackAndHitIdx at stop time).  HitOnTrack bookkeeping as
+// MkFinder::add_hit (MkFinder.h:312-354); with at most MKF_MAX_FIND_LAYERS layers
+// a track never exceeds Config::nMaxTrkHits.
+//
+// The windows' hits are scanned by the whole wavefront (wave_scan) and their chi2
+// evaluated as (seed, hit) pairs spread over its lanes, so a layer waits for a few
+// batches of loads instead of one per hit of the fullest window.  A wavefront
+// carries `spw` seeds: 64 when there are enough to fill the chip, fewer otherwise,
+// since the lanes without a seed still share the scan and the pairs.
+struct BestHitLds {
+  ScanLds scan;
+  float c2[64][kHitIdxMax];
+  int pre[64];
+  unsigned char owner[64 * kHitIdxMax];
+};
+constexpr size_t kBestHitWaves = 2048;
+constexpr int kRowW = 29;    // words of a lane's staged state: par, err, charge << 1 | barrel; odd stride
+static_assert(sizeof(ScanLds::desc) >= 64 * kRowW * sizeof(float), "the staged states fit the scan's work list");
+
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_find_best_hit(FindArgs a) {
+  __shared__ BestHitLds S;
+  float* __restrict__ X = reinterpret_cast<float*>(S.scan.desc);   // free between two scans
   const size_t n = (size_t)a.n;
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < a.n; t += stride) {
-    const int base = a.layer_base ? a.layer_base[t] : 0;   // first layer of the seed's event
-    if (base < 0 || base > a.eoh_layers - a.n_layers) continue;
-    const LayerDev* __restrict__ lays = a.layers + base;
-    float par[6], err[21];
+  const int lane = threadIdx.x;
+  const int t = blockIdx.x * a.spw + lane;
+  bool alive = lane < a.spw && t < a.n;
+  const int base = (alive && a.layer_base) ? a.layer_base[t] : 0;   // first layer of the seed's event
+  const bool valid = alive && base >= 0 && base <= a.eoh_layers - a.n_layers;
+  alive = valid;
+  const LayerDev* __restrict__ lays = a.layers + (valid ? base : 0);
+  float par[6], err[21];
+  int chg = 1;
+  float chi2 = 0.f;
+  int nfound = 0, ninside = 0, ntail = 0, stop = a.n_layers;
+  if (valid) {
 #pragma unroll
     for (int e = 0; e < 6; ++e) par[e] = a.par[e * n + t];
 #pragma unroll
     for (int e = 0; e < 21; ++e) err[e] = a.err[e * n + t];
-    int chg = a.chg[t];
-    float chi2 = a.chi2[t];
-    int nfound = 0, ninside = 0, ntail = 0;
+    chg = a.chg[t];
+    chi2 = a.chi2[t];
     for (int l = 0; l < a.first_layer; ++l) nfound += a.hot[l * n + t] >= 0;
-    int layer = a.first_layer;
-    for (; layer < a.n_layers; ++layer) {
-      const LayerDev& d = lays[layer];
-      float pp[6], pe[21];
+  }
+  for (int layer = a.first_layer; layer < a.n_layers && __any(alive); ++layer) {
+    const LayerDev& d = lays[layer];
+    float pp[6], pe[21];
+    Window w;
+    w.wsr = MKF_WSR_OUTSIDE;
+    if (alive) {
 #pragma unroll
       for (int e = 0; e < 6; ++e) pp[e] = par[e];
 #pragma unroll
@@ -723,86 +757,114 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
       else
         propagate_to_z(pp, pe, chg, d.propagate_to, a.pflags, false, a.bfield, a.mat);
       // Tracks that cannot reach a barrel layer stop here (MkBuilder.cc:1431-1455).
-      if (d.is_barrel && pp[0] * pp[0] + pp[1] * pp[1] < d.rin * d.rin) break;
-      Window w;
-      hit_window(d, pp, pe, w);
-      float mp[3] = {pp[0], pp[1], pp[2]};
-      float me[6] = {666.f, 0.f, 666.f, 0.f, 0.f, 666.f};   // fake hit (MkFinder.cc:776-800)
-      int code = -9;
-      if (w.wsr != MKF_WSR_OUTSIDE) {
-        float min_c2 = dyn_chi2_cut(d, a.chi2_cut, pp[3], pp[5]);
-        int best = -1;
-        // The window's hits first (the scan keeps several loads in flight), then
-        // their chi2 in scan order, one copy of the evaluation.
-        int nc = 0;
-        scan_window(d, w, a.bins, a.phis, a.qs, a.mask, [&](int gi) { s_cand[nc++][threadIdx.x] = gi; });
-        for (int hc = 0; hc < nc; ++hc) {
-          const int gi = s_cand[hc][threadIdx.x];
-          float hp[3], he[6];
-          load_hit9(a.shits + (size_t)gi * 9, hp, he);
-          float q[6], qe[21];
-#pragma unroll
-          for (int e = 0; e < 6; ++e) q[e] = pp[e];
-#pragma unroll
-          for (int e = 0; e < 21; ++e) qe[e] = pe[e];
-          if (a.prop_to_hit) {                                // kalmanPropagateAndComputeChi2
-            if (d.is_barrel)
-              propagate_to_r(q, qe, chg, hypot_ref(hp[0], hp[1]), a.intra_pflags, false, a.bfield, a.mat);
-            else
-              propagate_to_z(q, qe, chg, hp[2], a.intra_pflags, false, a.bfield, a.mat);
-          }
-          const float c2 = fabsf(d.is_barrel ? kalman_barrel<true, false>(q, qe, hp, he)
-                                             : kalman_endcap<true, false>(q, qe, hp, he));
-          if (c2 < min_c2) {
-            min_c2 = c2;
-            best = gi;
-          }
-        }
-        if (best >= 0) {
-          load_hit9(a.shits + (size_t)best * 9, mp, me);
-          chi2 += min_c2;
-          code = a.ranks[best];
-          ++nfound;
-          ninside += ntail;
-          ntail = 0;
-        } else {
-          code = w.wsr == MKF_WSR_EDGE ? -3 : (ninside + ntail ? -2 : -1);
-          ntail += code == -1;
-        }
-      }
-      a.hot[layer * n + t] = code;
-      if (a.prop_to_hit) {                                    // kalmanPropagateAndUpdate
-        if (d.is_barrel)
-          propagate_to_r(pp, pe, chg, hypot_ref(mp[0], mp[1]), a.intra_pflags, false, a.bfield, a.mat);
-        else
-          propagate_to_z(pp, pe, chg, mp[2], a.intra_pflags, false, a.bfield, a.mat);
-      }
-      if (d.is_barrel)
-        kalman_barrel<false, true>(pp, pe, mp, me);
-      else
-        kalman_endcap<false, true>(pp, pe, mp, me);
-      if (pp[3] < 0.f) {                                      // KalmanUtilsMPlex.cc:497-504
-        chg = -chg;
-        pp[3] = -pp[3];
-      }
-#pragma unroll
-      for (int e = 0; e < 6; ++e) par[e] = pp[e];
-#pragma unroll
-      for (int e = 0; e < 21; ++e) err[e] = pe[e];
-      if (code == -2) {                                       // MkBuilder.cc:1465-1473
-        ++layer;
-        break;
+      if (d.is_barrel && pp[0] * pp[0] + pp[1] * pp[1] < d.rin * d.rin) {
+        alive = false;
+        stop = layer;
+      } else {
+        hit_window(d, pp, pe, w);
       }
     }
-    for (; layer < a.n_layers; ++layer) a.hot[layer * n + t] = -9;
+    const int nc = wave_scan(alive && w.wsr != MKF_WSR_OUTSIDE, d, w, a.bins, a.phis, a.qs, a.mask, S.scan);
+    int incl = nc;
 #pragma unroll
-    for (int e = 0; e < 6; ++e) a.par[e * n + t] = par[e];
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    const int total = __shfl(incl, 63, 64);
+    S.pre[lane] = incl - nc;
+    if (nc) {
+      float* xs = X + lane * kRowW;
+      for (int k = 0; k < nc; ++k) S.owner[incl - nc + k] = (unsigned char)lane;
 #pragma unroll
-    for (int e = 0; e < 21; ++e) a.err[e * n + t] = err[e];
-    a.chg[t] = chg;
-    a.chi2[t] = chi2;
-    a.n_found[t] = nfound;
+      for (int e = 0; e < 6; ++e) xs[e] = pp[e];
+#pragma unroll
+      for (int e = 0; e < 21; ++e) xs[6 + e] = pe[e];
+      xs[27] = __int_as_float(chg);
+      xs[28] = __int_as_float(d.is_barrel);
+    }
+    __syncthreads();
+    for (int j = lane; j < total; j += 64) {
+      const int o = S.owner[j], k = j - S.pre[o];
+      const float* xs = X + o * kRowW;
+      float hp[3], he[6];
+      load_hit9(a.shits + (size_t)S.scan.list[o][k] * 9, hp, he);
+      const bool barrel = __float_as_int(xs[28]) != 0;
+      float q[6], qe[21];
+#pragma unroll
+      for (int e = 0; e < 6; ++e) q[e] = xs[e];
+#pragma unroll
+      for (int e = 0; e < 21; ++e) qe[e] = xs[6 + e];
+      if (a.prop_to_hit) {                                    // kalmanPropagateAndComputeChi2
+        const int c = __float_as_int(xs[27]);
+        if (barrel)
+          propagate_to_r(q, qe, c, hypot_ref(hp[0], hp[1]), a.intra_pflags, false, a.bfield, a.mat);
+        else
+          propagate_to_z(q, qe, c, hp[2], a.intra_pflags, false, a.bfield, a.mat);
+      }
+      S.c2[o][k] = fabsf(barrel ? kalman_barrel<true, false>(q, qe, hp, he) : kalman_endcap<true, false>(q, qe, hp, he));
+    }
+    __syncthreads();
+    if (!alive) continue;
+    float mp[3] = {pp[0], pp[1], pp[2]};
+    float me[6] = {666.f, 0.f, 666.f, 0.f, 0.f, 666.f};       // fake hit (MkFinder.cc:776-800)
+    int code = -9;
+    if (w.wsr != MKF_WSR_OUTSIDE) {
+      float min_c2 = dyn_chi2_cut(d, a.chi2_cut, pp[3], pp[5]);
+      int best = -1;
+      for (int k = 0; k < nc; ++k) {
+        const float c2 = S.c2[lane][k];
+        if (c2 < min_c2) {
+          min_c2 = c2;
+          best = k;
+        }
+      }
+      if (best >= 0) {
+        const int gi = S.scan.list[lane][best];
+        load_hit9(a.shits + (size_t)gi * 9, mp, me);
+        chi2 += min_c2;
+        code = a.ranks[gi];
+        ++nfound;
+        ninside += ntail;
+        ntail = 0;
+      } else {
+        code = w.wsr == MKF_WSR_EDGE ? -3 : (ninside + ntail ? -2 : -1);
+        ntail += code == -1;
+      }
+    }
+    a.hot[layer * n + t] = code;
+    if (a.prop_to_hit) {                                      // kalmanPropagateAndUpdate
+      if (d.is_barrel)
+        propagate_to_r(pp, pe, chg, hypot_ref(mp[0], mp[1]), a.intra_pflags, false, a.bfield, a.mat);
+      else
+        propagate_to_z(pp, pe, chg, mp[2], a.intra_pflags, false, a.bfield, a.mat);
+    }
+    if (d.is_barrel)
+      kalman_barrel<false, true>(pp, pe, mp, me);
+    else
+      kalman_endcap<false, true>(pp, pe, mp, me);
+    if (pp[3] < 0.f) {                                        // KalmanUtilsMPlex.cc:497-504
+      chg = -chg;
+      pp[3] = -pp[3];
+    }
+#pragma unroll
+    for (int e = 0; e < 6; ++e) par[e] = pp[e];
+#pragma unroll
+    for (int e = 0; e < 21; ++e) err[e] = pe[e];
+    if (code == -2) {                                         // MkBuilder.cc:1465-1473
+      alive = false;
+      stop = layer + 1;
+    }
   }
+  if (!valid) return;
+  for (int layer = max(stop, a.first_layer); layer < a.n_layers; ++layer) a.hot[layer * n + t] = -9;
+#pragma unroll
+  for (int e = 0; e < 6; ++e) a.par[e * n + t] = par[e];
+#pragma unroll
+  for (int e = 0; e < 21; ++e) a.err[e * n + t] = err[e];
+  a.chg[t] = chg;
+  a.chi2[t] = chi2;
+  a.n_found[t] = nfound;
 }
 
 }  // namespace
@@ -1002,7 +1064,7 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
                          pairs, pre, pre_stride);
       HIP_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_row_sort, dim3(n_rows), dim3(kRowBlock), 0, st, h->d_row_layer, h->d_layers, h->d_tile_off,
+    hipLaunchKernelGGL((total > kStreamHits ? k_row_sort<true> : k_row_sort<false>), dim3(n_rows), dim3(kRowBlock), 0, st, h->d_row_layer, h->d_layers, h->d_tile_off,
                        pre, pre_stride, pairs, hits, h->d_shits, h->d_phis, h->d_qs, h->d_ranks, place, h->d_bins);
     HIP_TRY(hipGetLastError());
     if (tiles) {
@@ -1215,7 +1277,9 @@ int mkf_find_tracks_best_hit(mkf_context* c, mkf_event_of_hits* h, const mkf_fin
   a.bins = h->d_bins;
   a.phis = h->d_phis; a.qs = h->d_qs; a.shits = h->d_shits; a.ranks = h->d_ranks;
   a.mask = h->mask();
-  hipLaunchKernelGGL(k_find_best_hit, dim3(blocks_for(N, 256)), dim3(256), 0, (hipStream_t)stream, a);
+  a.spw = 64;
+  while (a.spw > 4 && N < (size_t)a.spw * kBestHitWaves) a.spw /= 2;
+  hipLaunchKernelGGL(k_find_best_hit, dim3(blocks_for(N, a.spw)), dim3(64), 0, (hipStream_t)stream, a);
   HIP_TRY(hipGetLastError());
   return MKF_OK;
 }

@@ -195,6 +195,129 @@ __device__ __forceinline__ int scan_window(const LayerDev& d, const Window& w, c
   return cnt;
 }
 
+// ---- the same scan for a wavefront's windows ---------------------------------
+// Lane l's window (active) is scanned by the whole wavefront: the windows' bin runs
+// are cut into chunks of kChunk hits, numbered over the lanes, and each group of
+// kChunk lanes takes one chunk at a time, so a load instruction reads a few whole
+// lines rather than 64 scattered words and no lane idles while the fullest window
+// is read.  Chunks of a window are consecutive, so a hit's place in its window's
+// list is the window's count so far plus the passing hits of the groups before it;
+// the lists hold the same hits in the same order as scan_window's.  One wavefront
+// per workgroup.
+constexpr int kChunk = 8, kChunkGroups = 64 / kChunk;
+constexpr int kScanDescs = 1024;
+constexpr int kScanBatch = 4;                 // chunks per group whose loads are in flight together
+constexpr int kScanRows = 4;                  // q rows whose bin ranges are read together
+struct ScanLds {
+  int2 desc[kScanDescs];                      // a chunk: {first sorted position, lane | hits << 6 | chunk << 10}
+  float4 win[64];                             // q, phi, dq, dphi
+  int cnt[64];
+  int list[64][kHitIdxMax];                   // the hits' sorted positions
+};
+
+__device__ __forceinline__ int wave_scan(bool active, const LayerDev& d, const Window& w,
+                                         const int2* __restrict__ bins, const float* __restrict__ phis,
+                                         const float* __restrict__ qs, const unsigned char* __restrict__ mask,
+                                         ScanLds& S) {
+  const int lane = threadIdx.x & 63, group = lane / kChunk, gl = lane % kChunk;
+  // Runs of the window's bins that avoid bin 0, or bin 0 itself, in scan order: run(first position, hits).
+  auto each_run = [&](auto&& run) {
+    for (int qi = w.qb1; qi < w.qb2; ++qi) {
+      const int2* __restrict__ row = bins + d.bin_off + qi * kNPhi;
+      for (int pi = w.pb1; pi < w.pb2;) {
+        const int b = pi & 0xff;
+        const int b2 = b == 0 ? 0 : min(kNPhi - 1, b + (w.pb2 - 1 - pi));
+        const int lo = row[b].x, hi = row[b2].y;
+        pi += b2 - b + 1;
+        if (hi > lo) run(d.hit_off + lo, hi - lo);
+      }
+    }
+  };
+  const int b1 = w.pb1 & 0xff;
+  // One run per row and few rows: all their ranges are read at once and kept.
+  const bool plain = active && w.qb2 - w.qb1 <= kScanRows && b1 > 0 && b1 + (w.pb2 - w.pb1) <= kNPhi;
+  int lo[kScanRows], len[kScanRows], nch = 0;
+#pragma unroll
+  for (int r = 0; r < kScanRows; ++r) {
+    lo[r] = len[r] = 0;
+    if (plain && w.qb1 + r < w.qb2 && w.pb2 > w.pb1) {
+      const int2* __restrict__ row = bins + d.bin_off + (w.qb1 + r) * kNPhi + b1;
+      lo[r] = row[0].x;
+      len[r] = row[w.pb2 - w.pb1 - 1].y;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kScanRows; ++r) {
+    len[r] = max(len[r] - lo[r], 0);
+    lo[r] += d.hit_off;
+    nch += (len[r] + kChunk - 1) / kChunk;
+  }
+  if (active && !plain) each_run([&](int, int h) { nch += (h + kChunk - 1) / kChunk; });
+  int incl = nch;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += v;
+  }
+  const int total = __shfl(incl, 63, 64), first = incl - nch;
+  __syncthreads();
+  if (active) S.win[lane] = make_float4(w.q, w.phi, w.dq, w.dphi);
+  S.cnt[lane] = 0;
+  for (int r0 = 0; r0 < total; r0 += kScanDescs) {
+    if (active) {
+      int id = first - r0, k = 0;
+      auto add = [&](int at, int hits) {
+        for (int h = 0; h < hits; h += kChunk, ++id, ++k)
+          if (id >= 0 && id < kScanDescs) S.desc[id] = make_int2(at + h, lane | min(kChunk, hits - h) << 6 | min(k, kChunkGroups) << 10);
+      };
+      if (plain) {
+#pragma unroll
+        for (int r = 0; r < kScanRows; ++r) add(lo[r], len[r]);
+      } else {
+        each_run(add);
+      }
+    }
+    __syncthreads();
+    const int m = min(kScanDescs, total - r0);
+    for (int c0 = 0; c0 < m; c0 += kChunkGroups * kScanBatch) {
+      int2 dd[kScanBatch];
+      float hq[kScanBatch], hp[kScanBatch];
+      bool taken[kScanBatch];
+#pragma unroll
+      for (int u = 0; u < kScanBatch; ++u) {
+        const int c = c0 + u * kChunkGroups + group;
+        dd[u] = c < m ? S.desc[c] : make_int2(0, 0);
+        const bool in = gl < ((dd[u].y >> 6) & 0xf);
+        hq[u] = in ? qs[dd[u].x + gl] : 0.f;
+        hp[u] = in ? phis[dd[u].x + gl] : 0.f;
+        taken[u] = in && mask && mask[dd[u].x + gl];
+      }
+#pragma unroll
+      for (int u = 0; u < kScanBatch; ++u) {
+        const int wl = dd[u].y & 63, hits = (dd[u].y >> 6) & 0xf, k = dd[u].y >> 10;
+        const float4 v = S.win[wl];
+        const float ddq = fabsf(v.x - hq[u]);
+        const float ddphi = cdist(fabsf(v.y - hp[u]));
+        const bool pass = gl < hits && !(ddq >= v.z || ddphi >= v.w) && !taken[u];
+        const uint64_t all = __ballot(pass);
+        const int g0 = max(group - k, 0);                    // this window's first group in the step
+        const uint64_t mine = all >> (g0 * kChunk) << (g0 * kChunk);
+        const int before = S.cnt[wl];
+        const int at = before + __popcll(mine & ((1ull << lane) - 1));
+        if (pass && at < kHitIdxMax) S.list[wl][at] = dd[u].x + gl;
+        // the window's last group in the step adds up
+        const int next = __shfl_down(dd[u].y, kChunk, 64);
+        if (gl == 0 && hits && (group == kChunkGroups - 1 || ((next >> 6) & 0xf) == 0 || next >> 10 == 0))
+          S.cnt[wl] = before + __popcll(mine & (~0ull >> (64 - (group + 1) * kChunk)));
+        __syncthreads();
+      }
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  return active ? min(S.cnt[lane], kHitIdxMax) : 0;
+}
+
 // getHitSelDynamicChi2Cut (MkFinder.cc:202-220)
 __device__ __forceinline__ float dyn_chi2_cut(const LayerDev& d, float cut_min, float invpt, float theta_in) {
   const float theta = fabsf(theta_in - kPIOver2);
