@@ -714,7 +714,11 @@ struct BestHitLds {
   int pre[64];
   unsigned char owner[64 * kHitIdxMax];
 };
-constexpr size_t kBestHitWaves = 2048;
+// Seeds per wavefront are halved from 64 until there are this many wavefronts, one per SIMD: below, SIMDs idle;
+// above, wavefronts of half-used lanes take turns (best-hit step at 512 / 1024 / 2048 / 4096 wavefronts: one 10k-seed
+// event 357 / 342 / 432 / 432 us, 4 events - / 858 / 933 / 1020 us, 12 events - / 1950 / 2077 / 2311 us; at 500
+// seeds 1, 2, 4, 8, 16 seeds per wavefront: 286, 292, 298, 313, 345 us).
+constexpr size_t kBestHitWaves = 1024;
 constexpr int kRowW = 29;    // words of a lane's staged state: par, err, charge << 1 | barrel; odd stride
 static_assert(sizeof(ScanLds::desc) >= 64 * kRowW * sizeof(float), "the staged states fit the scan's work list");
 
@@ -1278,7 +1282,7 @@ int mkf_find_tracks_best_hit(mkf_context* c, mkf_event_of_hits* h, const mkf_fin
   a.phis = h->d_phis; a.qs = h->d_qs; a.shits = h->d_shits; a.ranks = h->d_ranks;
   a.mask = h->mask();
   a.spw = 64;
-  while (a.spw > 4 && N < (size_t)a.spw * kBestHitWaves) a.spw /= 2;
+  while (a.spw > 1 && N < (size_t)a.spw * kBestHitWaves) a.spw /= 2;
   hipLaunchKernelGGL(k_find_best_hit, dim3(blocks_for(N, a.spw)), dim3(64), 0, (hipStream_t)stream, a);
   HIP_TRY(hipGetLastError());
   return MKF_OK;
