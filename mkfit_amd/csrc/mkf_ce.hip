@@ -8,10 +8,11 @@
 //       each hit's chi2 (after propagating to the hit, as the reference does
 //       with finding_requires_propagation_to_hit_pos); accepted hits and the
 //       invalid-hit entry go to LDS as IdxChi2List records;
-//   (b) one lane per seed keeps the best max_cands records (a stable top-K by
-//       score in the reference's generation order) and lays out the seed's
-//       next candidate list -- records interleaved with held-back extras, the
-//       best short candidate set aside (CandCloner::ProcessSeedRange);
+//   (b) the seed's lanes rank its records (each lane offers its best remaining
+//       one, max_cands times: a stable top-K by score in the reference's
+//       generation order) and one of them lays out the seed's next candidate
+//       list -- records interleaved with held-back extras, the best short
+//       candidate set aside (CandCloner::ProcessSeedRange);
 //   (c) every lane builds its new candidate from its parent's state (exchanged
 //       through LDS), appends the HitOnTrack node and, for a real hit, applies
 //       the Kalman update after propagating to the hit (UpdateWithLastHit).
@@ -53,11 +54,37 @@ constexpr int kW = 37;                // LDS words per exchanged candidate (36 u
 // propagated phi and theta.  Word 36, which put / get leave alone, holds
 // the score of the lane's invalid-hit record from (a) to the new candidates (c).
 constexpr int kXCut = 28, kXPre = 29, kXOff = 30, kXBar = 31, kXTrig = 32, kXScore = 36;
-// A kept accepted-hit record is {hit_cnt << kPosBits | position in the layer}.
-constexpr int kPosBits = 28;
-constexpr int kPosMask = (1 << kPosBits) - 1;
+constexpr int kMaxLayerHits = (1 << 28) - 1;   // hits per layer the finders take
 constexpr int kBsW = 40;              // words per seed of the best short candidate store (36 used)
-static_assert(kHitIdxMax <= 16, "hit_cnt must fit above the position bits");
+
+// Ranking key of an entry: its score, then the earlier place in the reference's
+// generation order.  Held back (standard finding): place = slot; a record: kSMax + hit_cnt * kSMax
+// + slot; an invalid-hit entry: after every record.  0: no entry.  Scores are finite; adding 0 makes
+// -0 equal to +0.
+constexpr int kGenRec = kSMax, kGenFake = kSMax + kHitIdxMax * kSMax, kGenEnd = kGenFake + kSMax;
+__device__ __forceinline__ uint64_t rank_key(float score, int gen) {
+  const unsigned b = __float_as_uint(score + 0.f);
+  const unsigned o = b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
+  return (uint64_t)o << 32 | (unsigned)(kGenEnd - gen);
+}
+__device__ __forceinline__ float key_score(uint64_t key) {
+  const unsigned o = (unsigned)(key >> 32);
+  return __uint_as_float(o ^ ((o >> 31) ? 0x80000000u : 0xffffffffu));
+}
+__device__ __forceinline__ int key_gen(uint64_t key) { return kGenEnd - (int)(unsigned)key; }
+
+// The greatest key of the lane's seed group (lanes g*KS .. g*KS + KS - 1).
+template <int KS>
+__device__ __forceinline__ uint64_t group_max(uint64_t key, int group_lane0, int c) {
+  uint64_t best = key;
+#pragma unroll
+  for (int o = 1; o < KS; ++o) {
+    const int from = group_lane0 + (c + o >= KS ? c + o - KS : c + o);
+    const uint64_t k = __shfl(key, from, 64);
+    best = k > best ? k : best;
+  }
+  return best;
+}
 
 struct Cand {
   float par[6], err[21];
@@ -193,15 +220,13 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
   // 19.9 KB (kS = 6) / 20.4 KB (kS = 8): eight workgroups per CU, as many as
   // the VGPRs allow.
   __shared__ float X[kLanes * kW];          // candidate state exchange (and the kX* words in (a))
-  __shared__ int Gh[kLanes][kHitIdxMax];    // each lane's window hits (positions in the layer), in scan
-                                            // order; from (a3) on its kept records, first ecnt
-  __shared__ float Gc[kLanes][kHitIdxMax];  // their chi2 if accepted, else -1; then the kept records'
-  __shared__ float Es[kLanes][kS];          // the kept records' scores
+  __shared__ int Gh[kLanes][kHitIdxMax];    // each lane's window hits (positions in the layer), in scan order
+  __shared__ float Gc[kLanes][kHitIdxMax];  // their chi2 if accepted, else -1
+  __shared__ float Es[kLanes][kS];          // (a2) the pairs' owners; (b) row g*kS + r: the seed's r-th ranked entry
   __shared__ float Gp[STD ? kLanes : 1][kHitIdxMax];   // STD: pT of each accepted hit's updated state
-  __shared__ unsigned char ecnt[kLanes];    // kept records
   __shared__ signed char fcode[kLanes];     // invalid-hit record's hit code, 0 = none
   __shared__ unsigned char xkind[kLanes];   // 1 = held back unchanged, 2 = stopped replica
-  __shared__ int D[kGA][kS];                // next candidates: kind | parent slot << 2 | record << 5
+  __shared__ int D[kGA][kS];                // next candidates: kind | parent slot << 2 | rank << 5 | hit_cnt << 8
   __shared__ float s_bsc[kGA];              // score of the best short candidate (the candidate: a.bs)
   __shared__ int s_nnodes[kGA];
   __shared__ unsigned char s_bs[kGA], s_state[kGA], s_ncand[kGA], s_any[kGA], s_nnew[kGA], s_merge[kGA];
@@ -253,7 +278,6 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
       if (s_state[g] == 0 && layer - 1 == a.first_layer - 1) s_state[g] = 1;
       s_any[g] = 0;
     }
-    ecnt[lane] = 0;
     fcode[lane] = 0;
     xkind[lane] = 0;
     __syncthreads();
@@ -377,9 +401,12 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
       }
     }
     __syncthreads();
-    // (a3) records of the accepted hits, in scan order
+    // (a3) the lane's best K records, sorted by score, in scan order among equals: the seed's top K never takes
+    // a record that K records of its own lane beat
+    float rs[kS];
+    int rh[kS], ne = 0;
     if (search) {
-      int ne = 0, nacc = 0;
+      int nacc = 0;
       for (int hc = 0; hc < nh; ++hc) {
         const float c2 = Gc[lane][hc];
         if (!(c2 >= 0.f)) continue;
@@ -387,41 +414,22 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
         const float tot = st.chi2 + c2;
         const float sc = score_calc(st.nfound + 1, 0, 0, st.ninside + st.ntail, tot < 0 ? 0.f : tot,
                                     STD ? Gp[lane][hc] : pt_l, true);
-        const int rec = hc << kPosBits | Gh[lane][hc];
-        // Keep only this lane's best K records, in hit order.  The seed's
-        // top K (by score, earlier generation first on ties) never takes a
-        // record that K records of its own lane beat, so the merge below
-        // sees every record it can select.  Worst kept = lowest score, the
-        // latest of equals; the new record comes after all kept ones, so it
-        // replaces the worst only with a strictly higher score.  The kept
-        // records go to the front of Gh / Gc in place: slot ne <= hc, and
-        // every slot past hc is still unread.
-        if (ne < K) {
-          Es[lane][ne] = sc;
-          Gh[lane][ne] = rec;
-          Gc[lane][ne] = c2;
-          ++ne;
-        } else {
-          int wk = 0;
-          float ws = Es[lane][0];
-          for (int kk = 1; kk < K; ++kk)
-            if (!(Es[lane][kk] > ws)) {
-              wk = kk;
-              ws = Es[lane][kk];
-            }
-          if (sc > ws) {
-            for (int kk = wk; kk < K - 1; ++kk) {
-              Es[lane][kk] = Es[lane][kk + 1];
-              Gh[lane][kk] = Gh[lane][kk + 1];
-              Gc[lane][kk] = Gc[lane][kk + 1];
-            }
-            Es[lane][K - 1] = sc;
-            Gh[lane][K - 1] = rec;
-            Gc[lane][K - 1] = c2;
-          }
+        int pos = 0;                                    // kept records with score >= sc
+#pragma unroll
+        for (int q = 0; q < kS; ++q) pos += (q < ne && !(rs[q] < sc)) ? 1 : 0;
+        if (pos >= K) continue;
+#pragma unroll
+        for (int q = kS - 1; q > 0; --q) {
+          rs[q] = q > pos ? rs[q - 1] : rs[q];
+          rh[q] = q > pos ? rh[q - 1] : rh[q];
         }
+#pragma unroll
+        for (int q = 0; q < kS; ++q) {
+          rs[q] = q == pos ? sc : rs[q];
+          rh[q] = q == pos ? hc : rh[q];
+        }
+        if (ne < K) ++ne;
       }
-      ecnt[lane] = ne;
       if (gap && nacc == 0) {      // dead module, no hit taken: -7, which is no hole (MkFinder.cc:1092-1096, 1263-1267)
         fcode[lane] = -7;
         X[lane * kW + kXScore] = score_calc(st.nfound, st.ntail, 0, st.ninside, st.chi2 < 0 ? 0.f : st.chi2, pt_l, true);
@@ -434,125 +442,90 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
     else
       put(&X[lane * kW], st);
     __syncthreads();
-    // ---- (b) CandCloner::ProcessSeedRange, one lane per seed
+    // ---- (b) CandCloner::ProcessSeedRange.  Each lane's entries are its records, its invalid-hit record and (STD,
+    // where find_tracks_handle_missed_layers runs before FindCandidates) itself when held back; K times the group
+    // takes the best of the lanes' best remaining ones.
+    {
+      const int l0 = g * kS;
+      const int fc = fcode[lane];
+      uint64_t fake = 0;                             // the lane's one entry beside its records
+      if (fc && !(STD && fc == -2)) fake = rank_key(X[lane * kW + kXScore], kGenFake + c);
+      if (STD && xkind[lane] == 1) fake = rank_key(X[lane * kW + 29], c);
+      const int rounds = g < kG ? K : 0;
+      for (int r = 0; r < K; ++r) {
+        const uint64_t rec = ne > 0 ? rank_key(rs[0], kGenRec + rh[0] * kSMax + c) : 0;
+        const uint64_t own = rec > fake ? rec : fake;
+        const uint64_t best = group_max<kS>(own, l0, c);
+        if (r < rounds && c == 0) {                  // the r-th ranked entry; word 1: 0 when there is none
+          Es[l0 + r][0] = best ? key_score(best) : 0.f;
+          Es[l0 + r][1] = __int_as_float(best ? key_gen(best) + 1 : 0);
+        }
+        if (own && own == best) {
+          if (rec > fake) {
+#pragma unroll
+            for (int q = 0; q + 1 < kS; ++q) {
+              rs[q] = rs[q + 1];
+              rh[q] = rh[q + 1];
+            }
+            --ne;
+          } else {
+            fake = 0;
+          }
+        }
+      }
+      if (STD) {
+        // the first entry with a -2 hit in ranked order: a stopped replica or a -2 invalid-hit entry
+        uint64_t shrt = 0;
+        if (xkind[lane] == 2) shrt = rank_key(X[lane * kW + 29], c);
+        else if (fc == -2) shrt = rank_key(X[lane * kW + kXScore], kGenFake + c);
+        shrt = group_max<kS>(shrt, l0, c);
+        if (c == 0 && g < kG) {
+          Es[l0][2] = shrt ? key_score(shrt) : 0.f;
+          Es[l0][3] = __int_as_float(shrt ? key_gen(shrt) + 1 : 0);
+        }
+      }
+    }
+    __syncthreads();
+    // One lane per seed lays out the next candidates.
     if (c == 0 && s_merge[g]) {
-      // The seed's best K so far, by score; a new entry goes after the kept
-      // ones of equal score.  Entry info: kind | slot << 2 | v << 5 with v the
-      // record in the slot lane's list (kind 2) or minus the hit code (kind 3).
-      // Every array index is a compile-time constant, so the lists stay in
-      // registers.
+      const int l0 = g * kS;
       float tsc[kS];
-      int ti[kS];
-      int nt = 0, nent = 0;
-      auto insert = [&](float sc, int info) {
-        ++nent;
-        int pos = 0;                                  // kept entries with score >= sc
+      int tg[kS];                                    // generation places of the ranked entries, -1 past the last
+      int nt = 0;
 #pragma unroll
-        for (int q = 0; q < kS; ++q) pos += (q < nt && !(tsc[q] < sc)) ? 1 : 0;
-        if (pos >= K) return;
-#pragma unroll
-        for (int q = kS - 1; q > 0; --q)
-          if (q > pos) {
-            tsc[q] = tsc[q - 1];
-            ti[q] = ti[q - 1];
-          }
-#pragma unroll
-        for (int q = 0; q < kS; ++q)
-          if (q == pos) {
-            tsc[q] = sc;
-            ti[q] = info;
-          }
-        if (nt < K) ++nt;
+      for (int q = 0; q < kS; ++q) {
+        const bool in = q < K;
+        tsc[q] = in ? Es[l0 + q][0] : 0.f;
+        tg[q] = in ? __float_as_int(Es[l0 + q][1]) - 1 : -1;
+        nt += tg[q] >= 0 ? 1 : 0;
+      }
+      // D's word of the ranked entry q
+      auto entry = [&](int gen, int q) {
+        if (gen < kGenRec) return 1 | gen << 2;
+        if (gen < kGenFake) return 2 | (gen & (kSMax - 1)) << 2 | q << 5 | (gen - kGenRec) / kSMax << 8;
+        return 3 | (gen & (kSMax - 1)) << 2;
       };
-      // STD: the first entry with a -2 hit in ranked order (highest score, earliest generated among equals)
-      // and its generation rank: held back 0..kS-1, records kS + hit_cnt * kS + slot, invalid-hit entries
-      // after every record.
-      float bsc = kScoreWorst;
-      int binfo = -1, bgen = 0;
-      auto consider_short = [&](float sc, int info, int gen) {
-        if (binfo < 0 || sc > bsc) {
-          bsc = sc;
-          binfo = info;
-          bgen = gen;
-        }
-      };
-      if (STD) {              // find_tracks_handle_missed_layers runs before FindCandidates
-        for (int s = 0; s < kS; ++s) {
-          const int l = g * kS + s;
-          if (xkind[l] == 1) insert(X[l * kW + 29], 1 | s << 2);
-          else if (xkind[l] == 2) consider_short(X[l * kW + 29], 1 | s << 2, s);
-        }
-      }
-      // Generation order: hit_cnt, then lane.  Each slot's records are in
-      // increasing hit_cnt, so the records are merged by always taking the
-      // slot whose next record has the lowest hit_cnt (the lowest slot among
-      // equals); a slot with none left reads kHitIdxMax.
-      int ptr[kS], cur[kS];
-#pragma unroll
-      for (int s = 0; s < kS; ++s) {
-        const int l = g * kS + s;
-        ptr[s] = 0;
-        cur[s] = ecnt[l] > 0 ? (int)((unsigned)Gh[l][0] >> kPosBits) : kHitIdxMax;
-      }
-      while (true) {
-        int sb = 0, hb = cur[0], pb = ptr[0];
-#pragma unroll
-        for (int s = 1; s < kS; ++s)
-          if (cur[s] < hb) {
-            hb = cur[s];
-            sb = s;
-            pb = ptr[s];
-          }
-        if (hb >= kHitIdxMax) break;
-        const int l = g * kS + sb;
-        insert(Es[l][pb], 2 | sb << 2 | pb << 5);
-        const int nx = pb + 1 < ecnt[l] ? (int)((unsigned)Gh[l][pb + 1] >> kPosBits) : kHitIdxMax;
-#pragma unroll
-        for (int s = 0; s < kS; ++s)
-          if (s == sb) {
-            ptr[s] = pb + 1;
-            cur[s] = nx;
-          }
-      }
-      for (int s = 0; s < kS; ++s) {
-        const int l = g * kS + s;
-        if (STD && fcode[l] == -2)
-          consider_short(X[l * kW + kXScore], 3 | s << 2 | 2 << 5, kS + kHitIdxMax * kS + s);
-        else if (fcode[l])
-          insert(X[l * kW + kXScore], 3 | s << 2 | -fcode[l] << 5);
-      }
+      static_assert((kGenRec & (kSMax - 1)) == 0 && (kGenFake & (kSMax - 1)) == 0, "the slot is gen's low bits");
       if (STD) {
         // MkBuilder.cc:1776-1828: the kept entries in ranked order become the next candidates; the first -2
         // entry is met if it ranks before the K-th of them
         int np = 0;
-        float sK = 0.f;
-        int iK = 0;
-        for (int ih = 0; ih < nt; ++ih) {
-          float sc = tsc[0];
-          int info = ti[0];
 #pragma unroll
-          for (int q = 1; q < kS; ++q)
-            if (q == ih) {
-              sc = tsc[q];
-              info = ti[q];
-            }
-          D[g][np++] = (info & 3) == 2 ? info : (info & 31);
-          sK = sc;
-          iK = info;
-        }
-        if (binfo >= 0) {
+        for (int q = 0; q < kS; ++q)
+          if (tg[q] >= 0) D[g][np++] = entry(tg[q], q);
+        const float bsc = Es[l0][2];
+        const int bgen = __float_as_int(Es[l0][3]) - 1;
+        if (bgen >= 0) {
           bool met = nt < K;
           if (!met) {
-            const int kind = iK & 3, slot = (iK >> 2) & 7;
-            const int gen = kind == 1 ? slot
-                          : kind == 2 ? kS + (int)((unsigned)Gh[g * kS + slot][iK >> 5] >> kPosBits) * kS + slot
-                                      : kS + kHitIdxMax * kS + slot;
-            met = bsc > sK || (bsc == sK && bgen < gen);
+            const float sK = Es[l0 + K - 1][0];
+            const int gK = __float_as_int(Es[l0 + K - 1][1]) - 1;
+            met = bsc > sK || (bsc == sK && bgen < gK);
           }
           if (met && bsc > s_bsc[g]) {                   // best short candidate
             Cand b;
-            get(&X[(g * kS + ((binfo >> 2) & 7)) * kW], b);
-            if ((binfo & 3) == 3) {                      // an invalid-hit entry; a stopped replica has its -2
+            get(&X[(l0 + (bgen & (kSMax - 1))) * kW], b);
+            if (bgen >= kGenFake) {                      // an invalid-hit entry; a stopped replica has its -2
               const int k = append_node(a, seed, &s_nnodes[g], -2, layer, b.last);
               if (k >= 0) b.last = k;
               add_hit_counts(b, -2, 0.f);
@@ -563,7 +536,7 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
             s_bs[g] = 1;
           }
         }
-        if (nent == 0 && binfo < 0)                      // no entry at all: the candidates stay
+        if (nt == 0 && bgen < 0)                         // no entry at all: the candidates stay
           for (int i = 0; i < s_ncand[g]; ++i) D[g][np++] = 1 | i << 2;
         s_nnew[g] = np;
       } else {
@@ -571,26 +544,22 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
       unsigned xm = 0;                                // held-back slots, lowest first
       for (int s = 0; s < kS; ++s)
         if (xkind[g * kS + s]) xm |= 1u << s;
-      if (nent == 0) {
+      if (nt == 0) {
         for (; xm; xm &= xm - 1) {
           D[g][np] = 1 | (__ffs(xm) - 1) << 2;
           ++np;
         }
       } else {
-        for (int ih = 0; ih < nt; ++ih) {
-          float sc = tsc[0];
-          int info = ti[0];
+        bool full = false;
 #pragma unroll
-          for (int q = 1; q < kS; ++q)
-            if (q == ih) {
-              sc = tsc[q];
-              info = ti[q];
-            }
-          const int kind = info & 3, slot = (info >> 2) & 7;
-          if (kind == 3 && (info >> 5) == 2) {        // hit code -2: a short candidate
+        for (int q = 0; q < kS; ++q) {
+          if (tg[q] < 0 || full) continue;
+          const float sc = tsc[q];
+          const int slot = tg[q] & (kSMax - 1);
+          if (tg[q] >= kGenFake && fcode[l0 + slot] == -2) {   // a short candidate
             if (sc > s_bsc[g]) {                      // best short candidate
               Cand b;
-              get(&X[(g * kS + slot) * kW], b);
+              get(&X[(l0 + slot) * kW], b);
               const int k = append_node(a, seed, &s_nnodes[g], -2, layer, b.last);
               if (k >= 0) b.last = k;
               add_hit_counts(b, -2, 0.f);
@@ -601,13 +570,16 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
             }
             continue;
           }
-          while (xm && X[(g * kS + __ffs(xm) - 1) * kW + 29] > sc && np < K) {
+          while (xm && X[(l0 + __ffs(xm) - 1) * kW + 29] > sc && np < K) {
             D[g][np] = 1 | (__ffs(xm) - 1) << 2;
             ++np;
             xm &= xm - 1;
           }
-          if (np >= K) break;
-          D[g][np] = kind == 2 ? info : (info & 31);
+          if (np >= K) {
+            full = true;
+            continue;
+          }
+          D[g][np] = entry(tg[q], q);
           ++np;
         }
         for (; xm && np < K; xm &= xm - 1) {
@@ -623,16 +595,16 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
     if (s_merge[g] && gvalid) {
       if (c < s_nnew[g]) {
         const int dd = D[g][c];
-        const int kind = dd & 3, l = g * kS + ((dd >> 2) & 7), ri = dd >> 5;
+        const int kind = dd & 3, l = g * kS + ((dd >> 2) & 7), rank = (dd >> 5) & 7, hc = dd >> 8;
         get(&X[l * kW], st);
         if (kind != 1) {
-          // kind 2: the slot lane's kept record ri; kind 3: its invalid-hit record
-          const int val = kind == 2 ? d.hit_off + (Gh[l][ri] & kPosMask) : fcode[l];
+          // kind 2: the slot lane's window hit hc; kind 3: its invalid-hit record
+          const int val = kind == 2 ? d.hit_off + Gh[l][hc] : fcode[l];
           const int hit = kind == 2 ? a.ranks[val] : val;
           const int k = append_node(a, seed, &s_nnodes[g], hit, layer, st.last);
           if (k >= 0) st.last = k;
-          add_hit_counts(st, hit, kind == 2 ? Gc[l][ri] : 0.f);
-          st.score = kind == 2 ? Es[l][ri] : X[l * kW + kXScore];
+          add_hit_counts(st, hit, kind == 2 ? Gc[l][hc] : 0.f);
+          st.score = kind == 2 ? Es[g * kS + rank][0] : X[l * kW + kXScore];
           if (kind == 2) {
             float mp[3], me[6];
             load_hit9(a.shits + (size_t)val * 9, mp, me);
@@ -741,8 +713,9 @@ int find_combinatorial(mkf_context* c, mkf_event_of_hits* h, const mkf_ce_batch*
   if (h->ctx != c) return fail(MKF_ERR_INVALID_ARG, "event of hits belongs to another context");
   if (!h->loaded) return fail(MKF_ERR_INVALID_ARG, "event of hits not loaded");
   if (b->n_seeds < 0) return fail(MKF_ERR_INVALID_ARG, "n_seeds < 0");
-  for (const LayerDev& ld : h->layers)                      // hit records carry 28-bit layer positions
-    if (ld.n_hits > kPosMask) return fail(MKF_ERR_INVALID_ARG, "a layer holds %d hits, above %d", ld.n_hits, kPosMask);
+  for (const LayerDev& ld : h->layers)                      
+    if (ld.n_hits > kMaxLayerHits)
+      return fail(MKF_ERR_INVALID_ARG, "a layer holds %d hits, above %d", ld.n_hits, kMaxLayerHits);
   const int LE = b->n_layers ? b->n_layers : h->n_layers;   // layers per event
   if (LE < 1 || LE > h->n_layers || LE > MKF_MAX_FIND_LAYERS)
     return fail(MKF_ERR_INVALID_ARG, "n_layers %d outside [1, min(%d, %d)]", LE, h->n_layers, MKF_MAX_FIND_LAYERS);
