@@ -902,8 +902,8 @@ int grow(mkf_event_of_hits* h, size_t total, size_t sort_bytes, hipStream_t st) 
   if (total > h->cap || !h->cap) {
     free_hit_arrays(h);
     const size_t cap = std::max<size_t>(total, 1024);
-    HIP_TRY(hipMalloc(&h->d_phis, cap * 4));
-    HIP_TRY(hipMalloc(&h->d_qs, cap * 4));
+    HIP_TRY(hipMalloc(&h->d_phis, (cap + kScanUnroll) * 4));   // the scans read whole kScanUnroll runs
+    HIP_TRY(hipMalloc(&h->d_qs, (cap + kScanUnroll) * 4));
     HIP_TRY(hipMalloc(&h->d_ranks, cap * 4));
     HIP_TRY(hipMalloc(&h->d_inv, cap * 4));
     HIP_TRY(hipMalloc(&h->d_shits, cap * 9 * 4));

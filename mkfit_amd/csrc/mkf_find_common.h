@@ -146,6 +146,18 @@ __device__ __forceinline__ void hit_window(const LayerDev& d, const float (&par)
 // is read on its own.  The hits visited, and their order, are the bin-by-bin
 // scan's.
 constexpr int kScanUnroll = 8;
+// n consecutive floats from a 4-byte aligned address, as one wide load where the compiler can.
+template <int N>
+__device__ __forceinline__ void load_run(const float* __restrict__ p, float (&v)[N]) {
+  struct F4 { float f[4]; };
+#pragma unroll
+  for (int i = 0; i < N; i += 4) {
+    F4 t;
+    __builtin_memcpy(&t, p + i, 16);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[i + k] = t.f[k];
+  }
+}
 // mask: per sorted hit, nonzero for a hit taken by an earlier iteration (MkFinder.cc:476-482), or NULL;
 // such a hit is passed over and does not count toward the kHitIdxMax.
 template <class F>
@@ -173,12 +185,8 @@ __device__ __forceinline__ int scan_window(const LayerDev& d, const Window& w, c
       for (int h = lo; h < hi && cnt < kHitIdxMax; h += kScanUnroll) {
         const int gi = d.hit_off + h;
         float hq[kScanUnroll], hp[kScanUnroll];
-#pragma unroll
-        for (int u = 0; u < kScanUnroll; ++u) {
-          const bool in = h + u < hi;
-          hq[u] = in ? qs[gi + u] : 0.f;
-          hp[u] = in ? phis[gi + u] : 0.f;
-        }
+        load_run(qs + gi, hq);
+        load_run(phis + gi, hp);
 #pragma unroll
         for (int u = 0; u < kScanUnroll; ++u) {
           if (h + u >= hi || cnt >= kHitIdxMax) break;
