@@ -86,6 +86,8 @@ __device__ __forceinline__ uint64_t group_max(uint64_t key, int group_lane0, int
   return best;
 }
 
+constexpr int kCeWavesPerCu = 8, kStdWavesPerCu = 6;   // workgroups whose LDS fits a CU
+
 struct Cand {
   float par[6], err[21];
   int chg;
@@ -157,7 +159,7 @@ __device__ __forceinline__ void get(const float* X, Cand& c) {
 }
 
 struct CeArgs {
-  int n, n_layers, first_layer, eoh_layers;
+  int n, n_layers, first_layer, eoh_layers, spw;
   const int* __restrict__ layer_base;
   int max_cands, max_holes, max_consec, prop_to_hit, intra_pflags, inter_pflags;
   float chi2_cut, bfield;
@@ -206,9 +208,9 @@ __device__ __forceinline__ void propagate(bool barrel, float (&p)[6], float (&e)
     propagate_to_z(p, e, chg, target, pflags, false, a.bfield, a.mat, trig);
 }
 
-// KS candidate slots per seed (max_cands <= KS): KS = 6 packs 10 seeds into the
-// wavefront's 64 lanes (4 idle), KS = 8 packs 8.  Lanes past the last whole
-// seed group (g == kG) take no part.  STD: standard finding (see the top).
+// KS candidate slots per seed (max_cands <= KS): KS = 6 packs up to 10 seeds into
+// the wavefront's 64 lanes (4 idle), KS = 8 up to 8; a.spw of them are used.  Lanes past the last
+// seed group take no part.  STD: standard finding (see the top).
 // WAVES: waves per SIMD the registers are allotted for.  Left to itself the compiler spends all 512
 // registers of a lane on one wave; two measured 21.0 against 29.7 ms for the standard form and 15.3
 // against 28.1 ms for the clone engine (50 events).  mkf_autotune_find picks KS and WAVES by timing.
@@ -234,8 +236,8 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
 
   const int lane = threadIdx.x;
   const int g = lane / kS, c = lane % kS;
-  const int seed = blockIdx.x * kG + g;
-  const bool gin = g < kG && seed < a.n;
+  const int seed = blockIdx.x * a.spw + g;
+  const bool gin = g < a.spw && seed < a.n;
   const int base = (gin && a.layer_base) ? a.layer_base[seed] : 0;   // first layer of the seed's event
   const bool gvalid = gin && base >= 0 && base <= a.eoh_layers - a.n_layers;
   const LayerDev* __restrict__ lays = a.layers + (gvalid ? base : 0);
@@ -786,7 +788,14 @@ int find_combinatorial(mkf_context* c, mkf_event_of_hits* h, const mkf_ce_batch*
   const mkf_find_shape sh = c->find_shape[standard ? 1 : 0];
   const int slots = sh.slots ? sh.slots : (b->max_cands <= 6 ? 6 : 8);
   if (slots < b->max_cands) return fail(MKF_ERR_INVALID_ARG, "find shape: %d slots < max_cands %d", slots, b->max_cands);
-  const int grid = (int)((N + kLanes / slots - 1) / (kLanes / slots));
+  // Seeds per wavefront: as few as put every wavefront on the chip at once.  A lone wavefront leaves its SIMD waiting
+  // for its own results half of the time and its phases grow with its seeds' windows and pairs, but one more than
+  // fit wait for a whole launch (one 10k-seed event, 10 / 9 / 6 / 5 / 4 / 2 seeds per wavefront: 704 / 692 / 627 /
+  // 612 / 889 / 1093 us; standard finding of 5003 seeds, 10 / 4 / 3 / 2: 660 / 594 / 886 / 842 us; 500 seeds, 10 / 1:
+  // 607 / 432 us).
+  const size_t resident = (size_t)c->num_cus * std::min(4 * sh.waves_per_simd, standard ? kStdWavesPerCu : kCeWavesPerCu);
+  a.spw = (int)std::min<size_t>(kLanes / slots, (N + resident - 1) / resident);
+  const int grid = (int)((N + a.spw - 1) / a.spw);
   const int sel = (slots == 8 ? 4 : 0) | (standard ? 2 : 0) | (sh.waves_per_simd == 1 ? 1 : 0);
   switch (sel) {
 #define MKF_CE_CASE(I, KS, STD, W)                                                                   \
