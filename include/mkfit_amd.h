@@ -169,8 +169,10 @@ int mkf_num_batched_variants(void);
  *   alignment  layer l's hits are moved by d_rphi (cm) along their local r-phi
  *              direction and d_z (cm) along z before the propagation and update:
  *              x' = x - d_rphi y/r, y' = y + d_rphi x/r, z' = z + d_z.
- * The forward states are kept only every `checkpoint_every` layers and are
- * recomputed within each segment on the way back. */
+ * The forward states are kept at least every `checkpoint_every` layers and are
+ * recomputed between on the way back; more of them are kept (down to every
+ * layer, which recomputes none) while the scratch stays within 512 MiB (or
+ * what earlier calls on the context took).  The results do not depend on it. */
 typedef struct mkf_adjoint_batch {
   int n_tracks, n_layers;
   const float* seed_par;  /* [6][n] */
@@ -182,7 +184,7 @@ typedef struct mkf_adjoint_batch {
   const float* theta;     /* [n_layers][3] device */
   int pflags;             /* MKF_PF_APPLY_MATERIAL: material from theta (MKF_PF_USE_PARAM_B_FIELD unsupported) */
   float xi_per_x0;        /* energy-loss scale per unit x/X0 (GeV) */
-  int checkpoint_every;   /* layers per recomputed segment, >= 1 */
+  int checkpoint_every;   /* most layers per recomputed segment, >= 1 */
   float* chi2;            /* [n] out: the track's total chi2 */
   float* grad;            /* [n_layers][3] out: d(sum over tracks of chi2)/d theta */
   int fp64;               /* 0: the FP32 fit model (as mkf_fit_batched computes it); 1: the same model in FP64,

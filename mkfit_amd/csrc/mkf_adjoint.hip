@@ -227,8 +227,26 @@ static __device__ __align__(256) unsigned char scratch[kAdjNoallocBytes];
 
 namespace {
 
-// Checks the batch; returns through `need` the scratch bytes the call takes and through `sum_bytes` the
-// 256-byte aligned size of the sums' partials at its front.
+// Scratch of a batch that keeps every `every`-th state: the sums' partials (sum_bytes, 256-byte aligned),
+// checkpoints, per-track gradient rows.
+size_t adjoint_bytes(const mkf_adjoint_batch* b, int every, size_t sum_bytes) {
+  const size_t N = b->n_tracks, L = b->n_layers, n_ck = (L + every - 1) / every, word = b->fp64 ? 8 : 4;
+  return sum_bytes + (n_ck * 27 + L * 3) * N * word;
+}
+
+// The spacing a call uses: one, so that the reverse sweep recomputes no state, when the scratch for it stays within
+// `limit`; else the shortest that does, and the caller's at least.  The gradient does not depend on it.  Recomputing
+// the states of five-layer segments is two of the seven forward steps' worth of work per layer (100k tracks, 25
+// layers: 804 us at a spacing of 5, 496 us at 1), while a state's store and load are 216 bytes.
+int adjoint_spacing(const mkf_adjoint_batch* b, size_t sum_bytes, size_t limit) {
+  int every = 1;
+  while (every < b->checkpoint_every && adjoint_bytes(b, every, sum_bytes) > limit) ++every;
+  return every;
+}
+constexpr size_t kAdjScratchFree = (size_t)512 << 20;
+
+// Checks the batch; returns through `need` the scratch bytes the call takes at the caller's spacing and through
+// `sum_bytes` the 256-byte aligned size of the sums' partials at its front.
 int adjoint_check(const mkf_adjoint_batch* b, size_t& need, size_t& sum_bytes) {
   if (!b) return fail(MKF_ERR_INVALID_ARG, "batch is NULL");
   if (b->n_tracks < 0 || b->n_layers <= 0 || b->n_layers > 1024)
@@ -250,17 +268,15 @@ int adjoint_check(const mkf_adjoint_batch* b, size_t& need, size_t& sum_bytes) {
   CHECK(check_dev(b->hit_err, L * 6 * N * 4, "hit_err"));
   CHECK(check_dev(b->n_hits, N * 4, "n_hits"));
   CHECK(check_dev(b->chi2, N * 4, "chi2"));
-  const size_t n_ck = (L + b->checkpoint_every - 1) / b->checkpoint_every;
-  const size_t word = b->fp64 ? 8 : 4;
-  // scratch: the sums' partials (256-byte aligned size), checkpoints, per-track gradient rows
   sum_bytes = (L * 3 * kSumParts * sizeof(double) + 255) / 256 * 256;
-  need = sum_bytes + (n_ck * 27 + L * 3) * N * word;
+  need = adjoint_bytes(b, b->checkpoint_every, sum_bytes);
   return MKF_OK;
 }
 
-// The forward fit, reverse sweep and sums of a checked batch, with `scratch` holding at least the bytes
-// adjoint_check asked for.  Every byte of the scratch that a kernel reads is written earlier in the same call.
-int adjoint_launch(const mkf_context* c, const mkf_adjoint_batch* b, void* scr, size_t sum_bytes, hipStream_t st) {
+// The forward fit, reverse sweep and sums of a checked batch, states kept every `every` layers, with `scr` holding
+// at least adjoint_bytes.  Every byte of the scratch that a kernel reads is written earlier in the same call.
+int adjoint_launch(const mkf_context* c, const mkf_adjoint_batch* b, int every, void* scr, size_t sum_bytes,
+                   hipStream_t st) {
   const size_t N = b->n_tracks, L = b->n_layers;
   if (N == 0) {
     hipLaunchKernelGGL(k_sum_rows, dim3((unsigned)((L * 3 + 255) / 256)), dim3(256), 0, st, (const double*)nullptr,
@@ -268,12 +284,12 @@ int adjoint_launch(const mkf_context* c, const mkf_adjoint_batch* b, void* scr, 
     HIP_TRY(hipGetLastError());
     return MKF_OK;
   }
-  const size_t n_ck = (L + b->checkpoint_every - 1) / b->checkpoint_every;
+  const size_t n_ck = (L + every - 1) / every;
   const size_t word = b->fp64 ? 8 : 4;
   AdjArgs a;
   a.n = b->n_tracks;
   a.n_layers = b->n_layers;
-  a.ck = b->checkpoint_every;
+  a.ck = every;
   a.pflags = b->pflags;
   a.xi_per_x0 = b->xi_per_x0;
   a.bfield = c->bfield;
@@ -332,18 +348,27 @@ extern "C" int mkf_fit_adjoint(mkf_context* c, const mkf_adjoint_batch* b, void*
   size_t need = 0, sum_bytes = 0;
   CHECK(adjoint_check(b, need, sum_bytes));
   hipStream_t st = (hipStream_t)stream;
-  if (b->n_tracks == 0) return adjoint_launch(c, b, nullptr, 0, st);
+  if (b->n_tracks == 0) return adjoint_launch(c, b, 1, nullptr, 0, st);
   std::lock_guard<std::mutex> lk(c->mu);
   CHECK(scratch_acquire(c->adj_done, st));
-  if (need > c->adj_bytes) {
+  int every = adjoint_spacing(b, sum_bytes, std::max(kAdjScratchFree, c->adj_bytes));
+  const size_t want = adjoint_bytes(b, every, sum_bytes);
+  if (want > c->adj_bytes) {
     HIP_TRY(hipDeviceSynchronize());
     if (c->adj_scratch) HIP_TRY(hipFree(c->adj_scratch));
     c->adj_scratch = nullptr;
     c->adj_bytes = 0;
-    HIP_TRY(hipMalloc(&c->adj_scratch, need));
-    c->adj_bytes = need;
+    size_t got = want;
+    if (hipMalloc(&c->adj_scratch, want) != hipSuccess) {   // a full device: the caller's spacing
+      (void)hipGetLastError();
+      c->adj_scratch = nullptr;
+      every = b->checkpoint_every;
+      got = need;
+      HIP_TRY(hipMalloc(&c->adj_scratch, need));
+    }
+    c->adj_bytes = got;
   }
-  CHECK(adjoint_launch(c, b, c->adj_scratch, sum_bytes, st));
+  CHECK(adjoint_launch(c, b, every, c->adj_scratch, sum_bytes, st));
   return scratch_release(c->adj_done, st);
 }
 
@@ -356,5 +381,6 @@ extern "C" int mkf_fit_adjoint_noalloc(mkf_context* c, const mkf_adjoint_batch* 
     return fail(MKF_ERR_INVALID_ARG,
                 "batch needs %zu bytes of adjoint scratch; mkf_fit_adjoint_noalloc has %zu (fewer tracks, or a "
                 "larger checkpoint_every)", need, c->adj_static_bytes);
-  return adjoint_launch(c, b, c->adj_static, sum_bytes, (hipStream_t)stream);
+  return adjoint_launch(c, b, adjoint_spacing(b, sum_bytes, c->adj_static_bytes), c->adj_static, sum_bytes,
+                        (hipStream_t)stream);
 }

@@ -110,6 +110,20 @@ def test_checkpointing_does_not_change_the_result(setup, gpu_device, fp64):
         assert np.array_equal(c, out[0][0]) and np.array_equal(g, out[0][1])
 
 
+@pytest.mark.parametrize("n,fp64", [(79000, False), (27000, False), (20000, True), (39000, True)])
+def test_kept_and_recomputed_states_agree(gpu_device, n, fp64):
+    """The 64 MiB scratch makes the first form keep every second to fifth state; the second keeps all of them."""
+    import torch
+    ev, geo, th = make_event(n, seed=n)
+    ctx = mk.Context(bfield=3.8)
+    data = mk.AlignmentData(ctx, ev, gpu_device, checkpoint_every=5, fp64=fp64)
+    theta = _theta(th, gpu_device)
+    few, every = data.run(theta, noalloc=True), data.run(theta)
+    assert torch.isfinite(every[0]).all() and torch.isfinite(every[1]).all()
+    assert torch.equal(few[0], every[0]) and torch.equal(few[1], every[1])
+    ctx.close()
+
+
 def test_autograd_harness(setup, gpu_device):
     import torch
     from mkfit_amd.autograd import fit_chi2
