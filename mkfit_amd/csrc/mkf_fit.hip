@@ -175,10 +175,25 @@ __device__ __forceinline__ void load_hit(const FitArgs& a, const FitBufs& b, int
 // flags a negative or NaN variance or a covariance beyond what the variances
 // allow by more than rounding, C_ij^2 > (1 + 1e-5) C_ii C_jj, with the
 // products formed in double (exact for float factors).
+//
+// A first look in FP32 clears nearly every track: with d_i = fl(1.000005 C_ii), fma(C_ij, C_ij, -fl(d_i C_jj)) <= 0
+// implies C_ij^2 <= 1.000005 (1 + 3 2^-24) C_ii C_jj < 1.00001 C_ii C_jj while the products stay in the normal range,
+// which variances within [1e-15, 1e15] ensure (a C_ij^2 that underflows is then far below the product).  Otherwise
+// the products are formed in double.  Healthy covariances exceed 1 by up to 6e-7 through rounding.
 __device__ __forceinline__ bool ill_conditioned(const float (&C)[21]) {
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < 6; ++i) bad |= !(C[S(i, i)] >= 0.f);
+  float excess = 0.f, lo = C[0], hi = C[0];
+#pragma unroll
+  for (int i = 1; i < 6; ++i) {
+    const float d = C[S(i, i)] * 1.000005f;
+    lo = fminf(lo, C[S(i, i)]);
+    hi = fmaxf(hi, C[S(i, i)]);
+#pragma unroll
+    for (int j = 0; j < i; ++j) excess = fmaxf(excess, __builtin_fmaf(C[S(i, j)], C[S(i, j)], -(d * C[S(j, j)])));
+  }
+  if (!(excess > 0.f) && lo >= 1e-15f && hi <= 1e15f) return bad;
 #pragma unroll
   for (int i = 1; i < 6; ++i)
 #pragma unroll
