@@ -647,29 +647,37 @@ k_charge_sorted(int total, const int* __restrict__ inv, const unsigned char* __r
   if (j < total) charge_s[inv[j]] = code[j];
 }
 
-__global__ void __launch_bounds__(256)
-k_select(LayerDev d, int n, const float* __restrict__ par, const float* __restrict__ err,
+// One wavefront per workgroup, `lanes` of its lanes with a window each, scanned by all of them (25 -> 14 us for 30k
+// lanes, against one window per lane scanned by that lane).
+__global__ void __launch_bounds__(64)
+k_select(LayerDev d, int n, int lanes, const float* __restrict__ par, const float* __restrict__ err,
          const int2* __restrict__ bins, const float* __restrict__ phis, const float* __restrict__ qs,
          const unsigned char* __restrict__ mask, const int* __restrict__ ranks, int* __restrict__ xsize,
          int* __restrict__ xarr, int* __restrict__ wsr) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  float p[6], e[21];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) p[k] = par[(size_t)k * n + t];
-#pragma unroll
-  for (int k = 0; k < 21; ++k) e[k] = err[(size_t)k * n + t];
+  __shared__ ScanLds S;
+  const int lane = threadIdx.x, t = blockIdx.x * lanes + lane;
+  const bool valid = lane < lanes && t < n;
   Window w;
-  hit_window(d, p, e, w);
-  wsr[t] = w.wsr;
-  int cnt = -1;
-  if (w.wsr != MKF_WSR_OUTSIDE) {
-    int c = 0;
-    scan_window(d, w, bins, phis, qs, mask, [&](int gi) { xarr[(size_t)(c++) * n + t] = ranks[gi]; });
-    cnt = c;
+  w.wsr = MKF_WSR_OUTSIDE;
+  if (valid) {
+    float p[6], e[21];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) p[k] = par[(size_t)k * n + t];
+#pragma unroll
+    for (int k = 0; k < 21; ++k) e[k] = err[(size_t)k * n + t];
+    hit_window(d, p, e, w);
   }
-  xsize[t] = cnt;
-  for (int k = max(cnt, 0); k < kHitIdxMax; ++k) xarr[(size_t)k * n + t] = -1;
+  const bool search = valid && w.wsr != MKF_WSR_OUTSIDE;
+  const int cnt = wave_scan(search, d, w, bins, phis, qs, mask, S);
+  if (valid) {
+    wsr[t] = w.wsr;
+    xsize[t] = search ? cnt : -1;
+  }
+  // the lists, rows of `lanes` entries by all lanes
+  for (int j = lane; j < lanes * kHitIdxMax; j += 64) {
+    const int o = j % lanes, k = j / lanes, to = blockIdx.x * lanes + o;
+    if (to < n) xarr[(size_t)k * n + to] = k < min(S.cnt[o], kHitIdxMax) ? ranks[S.list[o][k]] : -1;
+  }
 }
 
 // ---- FindTracksBestHit -------------------------------------------------------
@@ -714,11 +722,6 @@ struct BestHitLds {
   int pre[64];
   unsigned char owner[64 * kHitIdxMax];
 };
-// Seeds per wavefront are halved from 64 until there are this many wavefronts, one per SIMD: below, SIMDs idle;
-// above, wavefronts of half-used lanes take turns (best-hit step at 512 / 1024 / 2048 / 4096 wavefronts: one 10k-seed
-// event 357 / 342 / 432 / 432 us, 4 events - / 858 / 933 / 1020 us, 12 events - / 1950 / 2077 / 2311 us; at 500
-// seeds 1, 2, 4, 8, 16 seeds per wavefront: 286, 292, 298, 313, 345 us).
-constexpr size_t kBestHitWaves = 1024;
 constexpr int kRowW = 29;    // words of a lane's staged state: par, err, charge << 1 | barrel; odd stride
 static_assert(sizeof(ScanLds::desc) >= 64 * kRowW * sizeof(float), "the staged states fit the scan's work list");
 
@@ -769,12 +772,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
       }
     }
     const int nc = wave_scan(alive && w.wsr != MKF_WSR_OUTSIDE, d, w, a.bins, a.phis, a.qs, a.mask, S.scan);
-    int incl = nc;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
-    }
+    const int incl = wave_inclusive(nc);
     const int total = __shfl(incl, 63, 64);
     S.pre[lane] = incl - nc;
     if (nc) {
@@ -1231,8 +1229,9 @@ int mkf_select_hit_indices(mkf_event_of_hits* h, int layer, int n, const float* 
   CHECK(check_dev(xsize, N * 4, "xsize"));
   CHECK(check_dev(xarr, kHitIdxMax * N * 4, "xarr"));
   CHECK(check_dev(wsr, N * 4, "wsr"));
-  hipLaunchKernelGGL(k_select, dim3(blocks_for(N, 256)), dim3(256), 0, (hipStream_t)stream, h->layers[layer], n, par,
-                     err, h->d_bins, h->d_phis, h->d_qs, h->mask(), h->d_ranks, xsize, xarr, wsr);
+  const int lanes = lanes_per_wave(N);
+  hipLaunchKernelGGL(k_select, dim3(blocks_for(N, lanes)), dim3(64), 0, (hipStream_t)stream, h->layers[layer], n, lanes,
+                     par, err, h->d_bins, h->d_phis, h->d_qs, h->mask(), h->d_ranks, xsize, xarr, wsr);
   HIP_TRY(hipGetLastError());
   return MKF_OK;
 }
@@ -1281,8 +1280,7 @@ int mkf_find_tracks_best_hit(mkf_context* c, mkf_event_of_hits* h, const mkf_fin
   a.bins = h->d_bins;
   a.phis = h->d_phis; a.qs = h->d_qs; a.shits = h->d_shits; a.ranks = h->d_ranks;
   a.mask = h->mask();
-  a.spw = 64;
-  while (a.spw > 1 && N < (size_t)a.spw * kBestHitWaves) a.spw /= 2;
+  a.spw = lanes_per_wave(N);
   hipLaunchKernelGGL(k_find_best_hit, dim3(blocks_for(N, a.spw)), dim3(64), 0, (hipStream_t)stream, a);
   HIP_TRY(hipGetLastError());
   return MKF_OK;

@@ -203,6 +203,17 @@ __device__ __forceinline__ int scan_window(const LayerDev& d, const Window& w, c
   return cnt;
 }
 
+// Inclusive prefix sum over a wavefront.
+__device__ __forceinline__ int wave_inclusive(int v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(v, o, 64);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
+
 // ---- the same scan for a wavefront's windows ---------------------------------
 // Lane l's window (active) is scanned by the whole wavefront: the windows' bin runs
 // are cut into chunks of kChunk hits, numbered over the lanes, and each group of
@@ -261,12 +272,7 @@ __device__ __forceinline__ int wave_scan(bool active, const LayerDev& d, const W
     nch += (len[r] + kChunk - 1) / kChunk;
   }
   if (active && !plain) each_run([&](int, int h) { nch += (h + kChunk - 1) / kChunk; });
-  int incl = nch;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += v;
-  }
+  const int incl = wave_inclusive(nch);
   const int total = __shfl(incl, 63, 64), first = incl - nch;
   __syncthreads();
   if (active) S.win[lane] = make_float4(w.q, w.phi, w.dq, w.dphi);
@@ -324,6 +330,16 @@ __device__ __forceinline__ int wave_scan(bool active, const LayerDev& d, const W
   }
   __syncthreads();
   return active ? min(S.cnt[lane], kHitIdxMax) : 0;
+}
+
+// Lanes of a one-wavefront workgroup given a seed (or candidate): halved from 64 until there is a wavefront per
+// SIMD.  Below, SIMDs idle; above, wavefronts of half-used lanes take turns (best-hit step at 512 / 1024 / 2048 /
+// 4096 wavefronts: one 10k-seed event 357 / 342 / 432 / 432 us, 4 events - / 858 / 933 / 1020 us, 12 events
+// - / 1950 / 2077 / 2311 us; at 500 seeds 1, 2, 4, 8, 16 seeds per wavefront: 286, 292, 298, 313, 345 us).
+inline int lanes_per_wave(size_t n) {
+  int lanes = 64;
+  while (lanes > 1 && n < (size_t)lanes * 1024) lanes /= 2;
+  return lanes;
 }
 
 // getHitSelDynamicChi2Cut (MkFinder.cc:202-220)

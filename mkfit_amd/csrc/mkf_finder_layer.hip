@@ -26,7 +26,7 @@ namespace {
 
 struct LayerStepArgs {
   LayerDev d;
-  int n;
+  int n, lanes;
   float chi2_cut, bfield;
   int prop_to_hit, prop_pflags, max_holes, max_consec;
   Material mat;
@@ -107,31 +107,95 @@ __device__ __forceinline__ void update_with(const LayerStepArgs& a, float (&p)[6
   }
 }
 
-__global__ void __launch_bounds__(256) k_add_best_hit(LayerStepArgs a) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.n) return;
+// ---- the hits of a wavefront's lists -----------------------------------------
+// A workgroup is one wavefront with a.lanes candidates, one per lane.  Their listed
+// hits are numbered over the lanes and evaluated 64 at a time, each by the next free
+// lane from the owner's state in LDS, so that the wavefront does not wait for the
+// longest list hit by hit.  c2[o][k]: hit k of lane o's list, its |chi2|, or -1 for an
+// entry that is not a hit of the layer (STRIP: or that a candidate may not take).
+constexpr int kStateW = 29;      // words of a staged state: par, err, charge; odd stride
+struct ListLds {
+  float x[64 * kStateW];
+  float c2[64][kHitIdxMax];
+  float cut[64];                 // STRIP: the lane's chi2 cut
+  int pre[64];
+  unsigned char owner[64 * kHitIdxMax];
+};
+
+template <bool STRIP>
+__device__ __forceinline__ void eval_lists(const LayerStepArgs& a, int xs, const float (&pp)[6], const float (&pe)[21],
+                                           int chg, float cut, ListLds& S) {
+  const int lane = threadIdx.x;
+  const size_t n = (size_t)a.n;
+  const int incl = wave_inclusive(xs);
+  const int total = __shfl(incl, 63, 64);
+  S.pre[lane] = incl - xs;
+  for (int k = 0; k < xs; ++k) S.owner[incl - xs + k] = (unsigned char)lane;
+  if (xs) {
+    float* x = S.x + lane * kStateW;
+#pragma unroll
+    for (int e = 0; e < 6; ++e) x[e] = pp[e];
+#pragma unroll
+    for (int e = 0; e < 21; ++e) x[6 + e] = pe[e];
+    x[27] = __int_as_float(chg);
+    if (STRIP) S.cut[lane] = cut;
+  }
+  __syncthreads();
+  for (int j = lane; j < total; j += 64) {
+    const int o = S.owner[j], k = j - S.pre[o];
+    const int pos = hit_pos(a, a.xarr[k * n + blockIdx.x * a.lanes + o]);
+    float c2 = -1.f;
+    if (pos >= 0) {
+      const float* x = S.x + o * kStateW;
+      float p[6], e[21], mp[3], me[6], q[6];
+      load_hit9(a.shits + (size_t)pos * 9, mp, me);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) p[i] = x[i];
+#pragma unroll
+      for (int i = 0; i < 21; ++i) e[i] = x[6 + i];
+      c2 = hit_chi2(a, p, e, __float_as_int(x[27]), mp, me, q);
+      if (STRIP) {
+        const bool barrel = a.d.is_barrel != 0;
+        if (!(c2 < S.cut[o] && strip_q_compatible(barrel, e, q, mp, me) &&
+              (!a.charge || pass_strip_charge(barrel, a.charge[pos], q, me))))
+          c2 = -1.f;
+      }
+    }
+    S.c2[o][k] = c2;
+  }
+  __syncthreads();
+}
+
+__global__ void __launch_bounds__(64) k_add_best_hit(LayerStepArgs a) {
+  __shared__ ListLds S;
+  const int lane = threadIdx.x, t = blockIdx.x * a.lanes + lane;
+  const bool valid = lane < a.lanes && t < a.n;
   const size_t n = (size_t)a.n;
   float pp[6], pe[21];
-  load_lane(a, t, pp, pe);
-  int chg = a.chg[t];
+  int chg = 1;
+  int xs = 0;
+  if (valid) {
+    load_lane(a, t, pp, pe);
+    chg = a.chg[t];
+    xs = max(min(a.xsize[t], kHitIdxMax), 0);
+  }
+  eval_lists<false>(a, xs, pp, pe, chg, 0.f, S);
+  if (!valid) return;
   float chi2 = a.chi2[t];
   int nfound = a.n_found[t], ninside = a.n_inside[t], ntail = a.n_tail[t];
-  const int xs = min(a.xsize[t], kHitIdxMax);
   const int w = a.wsr[t];
   float min_c2 = dyn_chi2_cut(a.d, a.chi2_cut, pp[3], pp[5]);
   int best = -1, best_pos = -1;
   for (int k = 0; k < xs; ++k) {                              // MkFinder.cc:725-765
-    const int idx = a.xarr[k * n + t];
-    const int pos = hit_pos(a, idx);
-    if (pos < 0) continue;
-    float hp[3], he[6], q[6];
-    load_hit9(a.shits + (size_t)pos * 9, hp, he);
-    const float c2 = hit_chi2(a, pp, pe, chg, hp, he, q);
-    if (c2 < min_c2) {
+    const float c2 = S.c2[lane][k];
+    if (!(c2 < 0.f) && c2 < min_c2) {
       min_c2 = c2;
-      best = idx;
-      best_pos = pos;
+      best = k;
     }
+  }
+  if (best >= 0) {
+    best = a.xarr[best * n + t];
+    best_pos = hit_pos(a, best);
   }
   float mp[3] = {pp[0], pp[1], pp[2]};
   float me[6] = {666.f, 0.f, 666.f, 0.f, 0.f, 666.f};          // fake hit (MkFinder.cc:776-800)
@@ -159,46 +223,45 @@ __global__ void __launch_bounds__(256) k_add_best_hit(LayerStepArgs a) {
   a.hit_code[t] = code;
 }
 
-__global__ void __launch_bounds__(256) k_find_candidates(LayerStepArgs a) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.n) return;
+__global__ void __launch_bounds__(64) k_find_candidates(LayerStepArgs a) {
+  __shared__ ListLds S;
+  const int lane = threadIdx.x, t = blockIdx.x * a.lanes + lane;
+  const bool valid = lane < a.lanes && t < a.n;
   const size_t n = (size_t)a.n;
   float pp[6], pe[21];
-  load_lane(a, t, pp, pe);
-  const int chg = a.chg[t];
+  int chg = 1, xs = 0;
+  float cut = 0.f;
+  if (valid) {
+    load_lane(a, t, pp, pe);
+    chg = a.chg[t];
+    xs = max(min(a.xsize[t], kHitIdxMax), 0);
+    cut = dyn_chi2_cut(a.d, a.chi2_cut, pp[3], pp[5]);
+  }
+  eval_lists<true>(a, xs, pp, pe, chg, cut, S);
+  if (!valid) return;
   const float chi2 = a.chi2[t];
   const int nfound = a.n_found[t], ninside = a.n_inside[t], ntail = a.n_tail[t];
-  const int xs = min(a.xsize[t], kHitIdxMax);
   const int w = a.wsr[t];
-  const float max_c2 = dyn_chi2_cut(a.d, a.chi2_cut, pp[3], pp[5]);
   const float pt = fabsf(1.0f / pp[3]);
-  const bool barrel = a.d.is_barrel != 0;
   mkf_idx_chi2* out = a.entries + (size_t)t * MKF_CE_ENTRIES_PER_LANE;
   int ne = 0;
   for (int k = 0; k < xs; ++k) {
-    const int idx = a.xarr[k * n + t];
-    const int pos = hit_pos(a, idx);
-    if (pos < 0) continue;
-    float mp[3], me[6], q[6];
-    load_hit9(a.shits + (size_t)pos * 9, mp, me);
-    const float c2 = hit_chi2(a, pp, pe, chg, mp, me, q);
-    if (c2 < max_c2 && strip_q_compatible(barrel, pe, q, mp, me) &&
-        (!a.charge || pass_strip_charge(barrel, a.charge[pos], q, me))) {
-      mkf_idx_chi2 r;
-      r.trk_idx = t;
-      r.hit_idx = idx;
-      r.module = 0u;
-      r.nhits = nfound + 1;
-      r.ntailholes = 0;
-      r.noverlaps = 0;
-      r.nholes = ninside + ntail;
-      r.pt = pt;
-      r.chi2 = chi2 + c2;
-      r.chi2_hit = c2;
-      r.score = score_calc(r.nhits, 0, 0, r.nholes, r.chi2 < 0 ? 0.f : r.chi2, pt, true);
-      r.xhit_pos = k;
-      out[ne++] = r;
-    }
+    const float c2 = S.c2[lane][k];
+    if (!(c2 >= 0.f)) continue;
+    mkf_idx_chi2 r;
+    r.trk_idx = t;
+    r.hit_idx = a.xarr[k * n + t];
+    r.module = 0u;
+    r.nhits = nfound + 1;
+    r.ntailholes = 0;
+    r.noverlaps = 0;
+    r.nholes = ninside + ntail;
+    r.pt = pt;
+    r.chi2 = chi2 + c2;
+    r.chi2_hit = c2;
+    r.score = score_calc(r.nhits, 0, 0, r.nholes, r.chi2 < 0 ? 0.f : r.chi2, pt, true);
+    r.xhit_pos = k;
+    out[ne++] = r;
   }
   if (w != MKF_WSR_OUTSIDE) {                                 // the invalid-hit record
     int fake = (ninside + ntail < a.max_holes && ntail < a.max_consec) ? -1 : -2;
@@ -309,7 +372,8 @@ int mkf_add_best_hit(mkf_context* c, mkf_event_of_hits* h, int layer, const mkf_
   a.prop_to_hit = prop_to_hit;
   a.prop_pflags = intra_pflags;
   a.hit_code = hit_code;
-  hipLaunchKernelGGL(k_add_best_hit, dim3(blocks_for(ln->n, 256)), dim3(256), 0, (hipStream_t)stream, a);
+  a.lanes = lanes_per_wave(ln->n);
+  hipLaunchKernelGGL(k_add_best_hit, dim3(blocks_for(ln->n, a.lanes)), dim3(64), 0, (hipStream_t)stream, a);
   HIP_TRY(hipGetLastError());
   return MKF_OK;
 }
@@ -332,7 +396,8 @@ int mkf_find_candidates_clone_engine(mkf_context* c, mkf_event_of_hits* h, int l
   a.max_consec = max_consec_holes;
   a.n_entries = n_entries;
   a.entries = entries;
-  hipLaunchKernelGGL(k_find_candidates, dim3(blocks_for(ln->n, 256)), dim3(256), 0, (hipStream_t)stream, a);
+  a.lanes = lanes_per_wave(ln->n);
+  hipLaunchKernelGGL(k_find_candidates, dim3(blocks_for(ln->n, a.lanes)), dim3(64), 0, (hipStream_t)stream, a);
   HIP_TRY(hipGetLastError());
   return MKF_OK;
 }
