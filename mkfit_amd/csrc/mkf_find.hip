@@ -335,7 +335,6 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
            const unsigned short* __restrict__ pre, int pre_stride, const RowPair* __restrict__ pairs,
            const float* __restrict__ hits, float* __restrict__ shits, float* __restrict__ phis,
            float* __restrict__ qs, int* __restrict__ ranks, int* __restrict__ place, int2* __restrict__ bins) {
-  __shared__ float s_phi[kRowCap];
   __shared__ int s_idx[kRowCap];
   __shared__ int cur[kFineBins + 1];     // fine bin starts, then (as cursors) the ends of the bins placed so far
   __shared__ int s_seg[kRowBlock];       // each tile's part: first place in the tile << 16 | length
@@ -394,8 +393,8 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
     if (NT) __builtin_nontemporal_store(v, p);
     else *p = v;
   };
-  // m ordered hits in s_phi / s_idx to row positions base..
-  auto write_out = [&](int base, int m) {
+  // m hits, ordered in s_idx, to row positions base..
+  auto write_hits = [&](int base, int m) {
     struct F3 { float a, b, c; };
     const int g0 = gbase + base;
     constexpr int kBatch = 6;
@@ -418,11 +417,7 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
         }
       }
     }
-    for (int h = t; h < m; h += kRowBlock) {
-      const int idx = s_idx[h];
-      put_out(phis + g0 + h, s_phi[h]);
-      ranks[g0 + h] = idx;
-    }
+    for (int h = t; h < m; h += kRowBlock) ranks[g0 + h] = s_idx[h];
   };
   auto write_bins = [&](auto&& start_of) {
     // Bin ranges (HitStructures.cc:146-171), as k_loh_fill's two passes leave them: an empty bin 1..255 of a row
@@ -434,83 +429,59 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
     brow[t] = r;
   };
   if (n <= kRowCap && nt <= kRowBlock) {
-    // 32 lanes per tile's part, four parts' loads in flight
-    constexpr int kGroups = kRowBlock / 32, kSegs = 4;
-    const int g = t >> 5, gl = t & 31;
-    for (int i0 = g; i0 < nt; i0 += kGroups * kSegs) {
-      RowPair p[kSegs];
-      int len[kSegs], dst[kSegs];
-#pragma unroll
-      for (int u = 0; u < kSegs; ++u) {
-        const int i = i0 + u * kGroups;
-        const int seg = i < nt ? s_seg[i] : 0;
-        len[u] = seg & 0xffff;
-        dst[u] = i < nt ? s_dst[i] : 0;
-        if (gl < len[u]) p[u] = src[(size_t)i * kTile + (seg >> 16) + gl];
-      }
-#pragma unroll
-      for (int u = 0; u < kSegs; ++u) {
-        if (gl < len[u]) {
-          s_phi[dst[u] + gl] = p[u].phi;
-          s_idx[dst[u] + gl] = p[u].idx;
-        }
-        for (int j = gl + 32; j < len[u]; j += 32) {
-          const int i = i0 + u * kGroups;
-          const RowPair r = src[(size_t)i * kTile + (s_seg[i] >> 16) + j];
-          s_phi[dst[u] + j] = r.phi;
-          s_idx[dst[u] + j] = r.idx;
-        }
-      }
+    // the positions of the row's pairs, 32 lanes per tile's part
+    constexpr int kGroups = kRowBlock / 32;
+    for (int i = t >> 5; i < nt; i += kGroups) {
+      const int seg = s_seg[i], len = seg & 0xffff, dst = s_dst[i], from = i * kTile + (seg >> 16);
+      for (int j = t & 31; j < len; j += 32) s_idx[dst + j] = from + j;
     }
     __syncthreads();
     constexpr int kPer = kRowCap / kRowBlock;
-    float phi[kPer];
-    int idx[kPer], at[kPer];             // at: fine bin << 16 | place in it; then the place in the row
+    RowPair pr[kPer];
+    int at[kPer];                        // fine bin << 16 | place in it; then the place in the row
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (t + k * kRowBlock < n) pr[k] = src[s_idx[t + k * kRowBlock]];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const int s = t + k * kRowBlock;
-      if (s < n) {
-        phi[k] = s_phi[s];
-        idx[k] = s_idx[s];
-        const int b = fine_bin_clamped(phi[k]);
+      if (t + k * kRowBlock < n) {
+        const int b = fine_bin_clamped(pr[k].phi);
         at[k] = b << 16 | atomicAdd(&cur[b], 1);
       }
     }
     __syncthreads();
     scan_bins();
+    int at0[kPer];                       // the pairs' positions, kept to write their places there
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) at0[k] = t + k * kRowBlock < n ? s_idx[t + k * kRowBlock] : 0;
+    __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPer; ++k)
-      if (t + k * kRowBlock < n) s_idx[cur[at[k] >> 16] + (at[k] & 0xffff)] = idx[k];
+      if (t + k * kRowBlock < n) s_idx[cur[at[k] >> 16] + (at[k] & 0xffff)] = pr[k].idx;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
       if (t + k * kRowBlock < n) {
         const int lo = cur[at[k] >> 16], hi = cur[(at[k] >> 16) + 1];
         int p = lo;
-        for (int i = lo; i < hi; ++i) p += s_idx[i] < idx[k];
+        for (int i = lo; i < hi; ++i) p += s_idx[i] < pr[k].idx;
         at[k] = p;
+        lplace[at0[k]] = gbase + p;
       }
-    }
-    __syncthreads();
-    // the pairs' places, back in the order they were read in (s_idx: place, s_phi: phi by place)
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      if (t + k * kRowBlock < n) {
-        s_idx[t + k * kRowBlock] = gbase + at[k];
-        s_phi[at[k]] = phi[k];
-      }
-    }
-    __syncthreads();
-    for (int i = g; i < nt; i += kGroups) {
-      const int seg = s_seg[i], len = seg & 0xffff, dst = s_dst[i];
-      for (int j = gl; j < len; j += 32) lplace[(size_t)i * kTile + (seg >> 16) + j] = s_idx[dst + j];
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPer; ++k)
-      if (t + k * kRowBlock < n) s_idx[at[k]] = idx[k];
+      if (t + k * kRowBlock < n) s_idx[at[k]] = pr[k].idx;
     __syncthreads();
-    write_out(0, n);
+    write_hits(0, n);
+    __syncthreads();
+    float* s_phi = reinterpret_cast<float*>(s_idx);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (t + k * kRowBlock < n) s_phi[at[k]] = pr[k].phi;
+    __syncthreads();
+    for (int h = t; h < n; h += kRowBlock) put_out(phis + gbase + h, s_phi[h]);
     write_bins([&](int b) { return cur[b]; });
     return;
   }
@@ -524,39 +495,40 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
   each_pair(0, nt, [&](const RowPair& p, int) { atomicAdd(&cur[fine_bin_clamped(p.phi)], 1); });
   __syncthreads();
   scan_bins();
-  // Puts each of the m entries (s_idx: hit index, s_phi: the pair's position), whose equal-bin group lies at
-  // [x, y) = group(phi), at its place by index, from row position `base` on, and then its phi in s_phi.
+  // Puts each of the m entries (s_idx: the pairs' positions), whose equal-bin group lies at [x, y) = group(phi), at
+  // its place by index, from row position `base` on; then s_idx holds hit indices.
   auto order = [&](int base, int m, auto&& group) {
     constexpr int kPer = kRowCap / kRowBlock;
-    float phi[kPer];
-    int idx[kPer], pos[kPer];
+    RowPair pr[kPer];
+    int at[kPer], pos[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const int s = t + k * kRowBlock;
-      if (s < m) {
-        const int at = __float_as_int(s_phi[s]);
-        phi[k] = src[at].phi;
-        idx[k] = s_idx[s];
-        const int2 r = group(phi[k]);
-        int p = r.x;
-        for (int i = r.x; i < r.y; ++i) p += s_idx[i] < idx[k];
-        pos[k] = p;
-        lplace[at] = gbase + base + p;
+      if (t + k * kRowBlock < m) {
+        at[k] = s_idx[t + k * kRowBlock];
+        pr[k] = src[at[k]];
       }
     }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (t + k * kRowBlock < m) s_idx[t + k * kRowBlock] = pr[k].idx;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
       if (t + k * kRowBlock < m) {
-        s_phi[pos[k]] = phi[k];
-        s_idx[pos[k]] = idx[k];
+        const int2 r = group(pr[k].phi);
+        int p = r.x;
+        for (int i = r.x; i < r.y; ++i) p += s_idx[i] < pr[k].idx;
+        pos[k] = p;
+        lplace[at[k]] = gbase + base + p;
+        phis[gbase + base + p] = pr[k].phi;
       }
     }
     __syncthreads();
-  };
-  auto put = [&](int s, const RowPair& p, int at) {
-    s_phi[s] = __int_as_float(at);
-    s_idx[s] = p.idx;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (t + k * kRowBlock < m) s_idx[pos[k]] = pr[k].idx;
+    __syncthreads();
   };
   for (int b0 = 0; b0 < kFineBins;) {
     const int base = cur[b0];
@@ -572,14 +544,14 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
       __syncthreads();
       each_pair(0, nt, [&](const RowPair& p, int at) {
         const int b = fine_bin_clamped(p.phi);
-        if (b >= b0 && b < b1) put(atomicAdd(&cur[b], 1) - base, p, at);
+        if (b >= b0 && b < b1) s_idx[atomicAdd(&cur[b], 1) - base] = at;
       });
       __syncthreads();
       order(base, m, [&](float phi) {
         const int b = fine_bin_clamped(phi);
         return make_int2((b > b0 ? cur[b - 1] : base) - base, cur[b] - base);
       });
-      write_out(base, m);
+      write_hits(base, m);
       b0 = b1;
     } else {                             // one bin beyond the capacity
       int done = 0;
@@ -587,12 +559,12 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
         if (t == 0) s_cnt = 0;
         __syncthreads();
         each_pair(i, i + 1, [&](const RowPair& p, int at) {
-          if (fine_bin_clamped(p.phi) == b0) put(atomicAdd(&s_cnt, 1), p, at);
+          if (fine_bin_clamped(p.phi) == b0) s_idx[atomicAdd(&s_cnt, 1)] = at;
         });
         __syncthreads();
         const int m = s_cnt;
         order(base + done, m, [&](float) { return make_int2(0, m); });
-        write_out(base + done, m);
+        write_hits(base + done, m);
         done += m;
         __syncthreads();
       }
