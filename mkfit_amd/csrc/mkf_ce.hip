@@ -73,19 +73,18 @@ __device__ __forceinline__ float key_score(uint64_t key) {
 }
 __device__ __forceinline__ int key_gen(uint64_t key) { return kGenEnd - (int)(unsigned)key; }
 
-// The greatest key of the lane's seed group (lanes g*KS .. g*KS + KS - 1).
+// The greatest key of the lane's seed group (lanes lane0 .. lane0 + KS - 1): after the steps 1, 2 and KS - 4, taken
+// around the group, a lane has seen all of its KS <= 8 keys.
 template <int KS>
-__device__ __forceinline__ uint64_t group_max(uint64_t key, int group_lane0, int c) {
-  uint64_t best = key;
+__device__ __forceinline__ uint64_t group_max(uint64_t key, int lane0, int c) {
+  static_assert(KS > 4 && KS <= 8, "three steps cover the group");
 #pragma unroll
-  for (int o = 1; o < KS; ++o) {
-    const int from = group_lane0 + (c + o >= KS ? c + o - KS : c + o);
-    const uint64_t k = __shfl(key, from, 64);
-    best = k > best ? k : best;
+  for (int o : {1, 2, KS - 4}) {
+    const uint64_t k = __shfl(key, lane0 + (c + o >= KS ? c + o - KS : c + o), 64);
+    key = k > key ? k : key;
   }
-  return best;
+  return key;
 }
-
 constexpr int kCeWavesPerCu = 8, kStdWavesPerCu = 6;   // workgroups whose LDS fits a CU
 
 struct Cand {
