@@ -851,43 +851,55 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
 namespace {
 
 void free_hit_arrays(mkf_event_of_hits* h) {
-  void* ps[] = {h->d_phis, h->d_qs, h->d_shits, h->d_ranks, h->d_inv};
+  void* ps[] = {h->d_phis, h->d_qs, h->d_shits, h->d_ranks, h->d_inv, h->d_sort};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   h->d_ranks = h->d_inv = nullptr;
   h->d_phis = h->d_qs = h->d_shits = nullptr;
+  h->d_sort = nullptr;
   h->cap = 0;
 }
 
-void free_sort_arrays(mkf_event_of_hits* h) {
-  if (h->d_sort) (void)hipFree(h->d_sort);
-  h->d_sort = nullptr;
-  h->sort_bytes = 0;
-}
+size_t aligned(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
-int grow(mkf_event_of_hits* h, size_t total, size_t sort_bytes, hipStream_t st) {
-  if (total <= h->cap && h->cap && sort_bytes <= h->sort_bytes) return MKF_OK;
-  HIP_TRY(hipStreamSynchronize(st));
-  HIP_TRY(hipDeviceSynchronize());
-  if (total > h->cap || !h->cap) {
-    free_hit_arrays(h);
-    const size_t cap = std::max<size_t>(total, 1024);
-    HIP_TRY(hipMalloc(&h->d_phis, (cap + kScanUnroll) * 4));   // the scans read whole kScanUnroll runs
-    HIP_TRY(hipMalloc(&h->d_qs, (cap + kScanUnroll) * 4));
-    HIP_TRY(hipMalloc(&h->d_ranks, cap * 4));
-    HIP_TRY(hipMalloc(&h->d_inv, cap * 4));
-    HIP_TRY(hipMalloc(&h->d_shits, cap * 9 * 4));
-    h->cap = cap;
-  }
-  if (sort_bytes > h->sort_bytes) {
-    free_sort_arrays(h);
-    HIP_TRY(hipMalloc(&h->d_sort, sort_bytes));
-    h->sort_bytes = sort_bytes;
-  }
+// A load's scratch for up to `cap` hits, whichever way they are sorted and however they lie over the layers.
+struct RowScratch {
+  size_t place, pre, bytes;       // offsets of the places and row starts behind the pairs
+};
+RowScratch row_scratch(const mkf_event_of_hits* h, size_t cap) {
+  RowScratch r;
+  r.place = aligned(cap * sizeof(RowPair));
+  r.pre = r.place + aligned(cap * 4);
+  r.bytes = r.pre + (cap / kTile + h->n_layers) * (size_t)(h->max_nq + 1) * sizeof(unsigned short);
+  return r;
+}
+int radix_scratch(size_t cap, size_t* temp, size_t* bytes) {
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, *temp, (uint32_t*)nullptr, (uint32_t*)nullptr, (int*)nullptr,
+                                             (int*)nullptr, (int)cap, 0, 32, (hipStream_t) nullptr));
+  *bytes = 4 * aligned(cap * 4) + *temp;
   return MKF_OK;
 }
 
-size_t aligned(size_t bytes) { return (bytes + 255) / 256 * 256; }
+// Both ways' scratch is taken when the hits outgrow the arrays, so that no later load of as many hits allocates.
+int grow(mkf_event_of_hits* h, size_t total, hipStream_t st) {
+  if (total <= h->cap && h->cap) return MKF_OK;
+  HIP_TRY(hipStreamSynchronize(st));
+  HIP_TRY(hipDeviceSynchronize());
+  free_hit_arrays(h);
+  const size_t cap = std::max<size_t>(total, 1024);
+  size_t temp = 0, bytes = 0;
+  CHECK(radix_scratch(cap, &temp, &bytes));
+  HIP_TRY(hipMalloc(&h->d_phis, (cap + kScanUnroll) * 4));   // the scans read whole kScanUnroll runs
+  HIP_TRY(hipMalloc(&h->d_qs, (cap + kScanUnroll) * 4));
+  HIP_TRY(hipMalloc(&h->d_ranks, cap * 4));
+  HIP_TRY(hipMalloc(&h->d_inv, cap * 4));
+  HIP_TRY(hipMalloc(&h->d_shits, cap * 9 * 4));
+  HIP_TRY(hipMalloc(&h->d_sort, std::max(bytes, row_scratch(h, cap).bytes)));
+  h->sort_temp = temp;
+  h->cap = cap;
+  return MKF_OK;
+}
+
 
 int blocks_for(size_t n, int block) { return (int)std::max<size_t>(1, (n + block - 1) / block); }
 
@@ -964,7 +976,6 @@ int mkf_event_of_hits_destroy(mkf_event_of_hits* h) {
   (void)hipSetDevice(h->device);
   (void)hipDeviceSynchronize();
   free_hit_arrays(h);
-  free_sort_arrays(h);
   if (h->d_tile_off) (void)hipFree(h->d_tile_off);
   if (h->d_ce_nodes) (void)hipFree(h->d_ce_nodes);
   if (h->d_mask_s) (void)hipFree(h->d_mask_s);
@@ -1000,16 +1011,7 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
     tiles += (int)((nl + kTile - 1) / kTile);
   }
   const int pre_stride = h->max_nq + 1;
-  const size_t items = std::max<size_t>(total, 1024);
-  size_t temp = 0, need;
-  if (rows) {
-    need = aligned(items * sizeof(RowPair)) + aligned(items * 4) + (size_t)tiles * pre_stride * sizeof(unsigned short);
-  } else {
-    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, temp, (uint32_t*)nullptr, (uint32_t*)nullptr, (int*)nullptr,
-                                               (int*)nullptr, (int)items, 0, 32, st));
-    need = 4 * aligned(items * 4) + temp;
-  }
-  CHECK(grow(h, total, need, st));
+  CHECK(grow(h, total, st));
   h->has_mask = false;
   h->has_charge = false;
   for (int l = 0; l < L; ++l) {
@@ -1030,9 +1032,11 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
   }
   const int n_rows = h->total_bins / kNPhi;
   if (rows) {
-    RowPair* pairs = static_cast<RowPair*>(h->d_sort);
-    int* place = reinterpret_cast<int*>(static_cast<char*>(h->d_sort) + aligned(items * sizeof(RowPair)));
-    unsigned short* pre = reinterpret_cast<unsigned short*>(reinterpret_cast<char*>(place) + aligned(items * 4));
+    const RowScratch lay = row_scratch(h, h->cap);
+    char* scr = static_cast<char*>(h->d_sort);
+    RowPair* pairs = reinterpret_cast<RowPair*>(scr);
+    int* place = reinterpret_cast<int*>(scr + lay.place);
+    unsigned short* pre = reinterpret_cast<unsigned short*>(scr + lay.pre);
     if (tiles) {
       hipLaunchKernelGGL(k_row_partition, dim3(tiles), dim3(kPartBlock), 0, st, L, h->d_tile_off, h->d_layers, hits,
                          pairs, pre, pre_stride);
@@ -1055,12 +1059,13 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
   const int nt = (int)total;
   char* scr = static_cast<char*>(h->d_sort);
   uint32_t* keys = reinterpret_cast<uint32_t*>(scr);
-  uint32_t* keys_s = reinterpret_cast<uint32_t*>(scr + aligned(items * 4));
-  int* vals = reinterpret_cast<int*>(scr + 2 * aligned(items * 4));
-  int* vals_s = reinterpret_cast<int*>(scr + 3 * aligned(items * 4));
+  uint32_t* keys_s = reinterpret_cast<uint32_t*>(scr + aligned(h->cap * 4));
+  int* vals = reinterpret_cast<int*>(scr + 2 * aligned(h->cap * 4));
+  int* vals_s = reinterpret_cast<int*>(scr + 3 * aligned(h->cap * 4));
   hipLaunchKernelGGL(k_hit_keys, dim3(blocks_for(total, 256)), dim3(256), 0, st, nt, L, hits, h->d_layers, keys, vals);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(scr + 4 * aligned(items * 4), temp, keys, keys_s, vals, vals_s, nt, 0, 32,
+  size_t temp = h->sort_temp;
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(scr + 4 * aligned(h->cap * 4), temp, keys, keys_s, vals, vals_s, nt, 0, 32,
                                              st));
   hipLaunchKernelGGL(k_loh_gather, dim3(blocks_for(total, 256)), dim3(256), 0, st, nt, keys_s, vals_s, h->d_layers,
                      hits, h->d_shits, h->d_phis, h->d_qs);

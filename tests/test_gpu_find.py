@@ -455,3 +455,124 @@ def test_loh_order_for_row_and_tile_sizes(gpu_device, q_bin, is_barrel):
         assert xs.item() == 1 and xa[0, 0].item() == sizes[last] - 1
     eoh.close()
     ctx.close()
+
+
+def test_loh_order_beyond_the_tile_table(gpu_device):
+    """A layer of more tiles (261 of 3072 hits) than a row's block keeps, beside a small one."""
+    import torch
+    rng = np.random.default_rng(77)
+    d = dict(is_barrel=1, rin=19.99, rout=20.01, zmin=-60.0, zmax=60.0, propagate_to=20.0, q_bin=0.5, min_dphi=0.002,
+             max_dphi=0.1, min_dq=0.3, max_dq=2.0, c_dp_sf=1.1, c_dq_sf=1.1, c_c2_sf=1.1)
+    n = 800_000
+    phi, z = rng.uniform(-np.pi, np.pi, n + 10), rng.uniform(-60.0, 60.0, n + 10)
+    h = np.zeros((n + 10, 9), np.float32)
+    h[:, 0], h[:, 1], h[:, 2] = 20 * np.cos(phi), 20 * np.sin(phi), z
+    ctx = mk.Context(bfield=3.8)
+    eoh = mk.EventOfHits(ctx, [d, d])
+    eoh.load(np.array([0, n, n + 10], np.int32), torch.from_numpy(h).to(gpu_device))
+    for l, hl in ((0, h[:n]), (1, h[n:])):
+        ranks, bins, phis, qs, nq = eoh.layer_views(l)
+        ph = np.arctan2(hl[:, 1].astype(np.float64), hl[:, 0].astype(np.float64)).astype(np.float32)
+        lo, extent = np.float32(-60.0), np.float32(120.0)
+        extra = np.float32(0.5) * (np.float32(nq) * np.float32(0.5) - extent)
+        qb = np.clip(((hl[:, 2] - (lo - extra)) * (np.float32(nq) / extent)).astype(np.int64), 0, nq - 1)
+        key = np.floor(F_PHI_FINE * (ph + np.float32(np.pi))).astype(np.int64) + (qb << 16)
+        assert np.array_equal(ranks, np.argsort(key, kind="stable"))
+        assert np.array_equal(phis, ph[ranks]) and np.array_equal(qs, hl[ranks, 2])
+        want = _rows_of_keys(key, nq)
+        full = want[:, 0] < want[:, 1]
+        assert np.array_equal(bins[full], want[full])
+    eoh.close()
+    ctx.close()
+
+
+def _repeat(ev, times):
+    """The event with its seeds repeated: every copy must come out as the first."""
+    out = dict(ev, n_seeds=ev["n_seeds"] * times)
+    for k in ("seed_par", "seed_err", "seed_chg", "seed_hits"):
+        out[k] = np.concatenate([ev[k]] * times, axis=-1)
+    return out
+
+
+def _first(ev, n):
+    return dict(ev, n_seeds=n, **{k: np.ascontiguousarray(ev[k][..., :n])
+                                  for k in ("seed_par", "seed_err", "seed_chg", "seed_hits")})
+
+
+@pytest.mark.parametrize("prop_to_hit", [False, True])
+def test_best_hit_for_every_packing(setup, gpu_device, prop_to_hit):
+    """Seeds per wavefront follow the batch size (1 to 64): the tracks do not depend on it."""
+    ev, descs, ctx, eoh = setup
+    ev = _first(ev, 1100)
+
+    def run(e):
+        b = mk.FindBatch(e, len(descs), 3, device=gpu_device, chi2_cut=15.0, prop_to_hit=prop_to_hit)
+        ctx.find_tracks_best_hit(eoh, b)
+        return b.numpy()
+    whole = run(ev)
+    for n in (1, 63, 1025):
+        part = run(_first(ev, n))
+        assert all(np.array_equal(part[k], whole[k][..., :n], equal_nan=True) for k in whole), n
+    for times in (2, 5, 16, 61):                     # 2 .. 64 seeds per wavefront, the last wavefront part filled
+        many = run(_repeat(ev, times))
+        for k in whole:
+            assert np.array_equal(many[k], np.concatenate([whole[k]] * times, axis=-1), equal_nan=True), (times, k)
+
+
+@pytest.mark.parametrize("finder,max_cands", [("ce", 1), ("ce", 6), ("ce", 8), ("std", 3), ("std", 8)])
+def test_combinatorial_for_every_packing(setup, gpu_device, finder, max_cands):
+    """Seeds per wavefront follow the batch size (1 to 10, or 8 slots' 8): the candidates do not depend on it."""
+    ev, descs, ctx, eoh = setup
+    ev = _first(ev, 900)
+
+    def run(e):
+        b = mk.CEBatch(e, len(descs), 3, device=gpu_device, chi2_cut=30.0, max_cands=max_cands)
+        (ctx.find_tracks_clone_engine if finder == "ce" else ctx.find_tracks_standard)(eoh, b)
+        return b.numpy()
+    whole = run(ev)
+    part = run(_first(ev, 1))
+    assert all(np.array_equal(part[k], whole[k][..., :1], equal_nan=True) for k in whole)
+    for times in (5, 9, 27):
+        many = run(_repeat(ev, times))
+        for k in whole:
+            assert np.array_equal(many[k], np.concatenate([whole[k]] * times, axis=-1), equal_nan=True), (times, k)
+
+
+@pytest.mark.parametrize("min_dphi,min_dq", [(0.01, 1.0), (0.3, 2.0), (1.6, 9.0), (3.1, 300.0)])
+def test_select_for_every_packing_and_window(gpu_device, min_dphi, min_dq):
+    """Windows of one bin to the whole layer (several runs per q row across phi = +-pi, more rows than are read
+    together, more chunks than the work list holds), for 1 to 64 windows per wavefront, against the oracle."""
+    import torch
+    rng = np.random.default_rng(31)
+    d = dict(is_barrel=1, rin=19.99, rout=20.01, zmin=-60.0, zmax=60.0, propagate_to=20.0, q_bin=2.0, min_dphi=min_dphi,
+             max_dphi=3.14, min_dq=min_dq, max_dq=400.0, c_dp_sf=1.1, c_dq_sf=1.1, c_c2_sf=1.1)
+    n_hits, n = 12000, 70000
+    phi, z = rng.uniform(-np.pi, np.pi, n_hits), rng.uniform(-60.0, 60.0, n_hits)
+    h = np.zeros((n_hits, 9), np.float32)
+    h[:, 0], h[:, 1], h[:, 2], h[:, 3], h[:, 5], h[:, 8] = 20 * np.cos(phi), 20 * np.sin(phi), z, 1e-4, 1e-4, 1e-2
+    tp = np.where(rng.random(n) < 0.3, np.pi - rng.uniform(0, 0.05, n), rng.uniform(-np.pi, np.pi, n))
+    par = np.stack([20 * np.cos(tp), 20 * np.sin(tp), rng.uniform(-62.0, 62.0, n), np.full(n, 0.5), tp,
+                    rng.uniform(0.6, 2.5, n)]).astype(np.float32)
+    err = np.zeros((21, n), np.float32)
+    err[[0, 2, 5, 9, 14, 20]] = 1e-4
+    ctx = mk.Context(bfield=3.8)
+    eoh = mk.EventOfHits(ctx, [d])
+    eoh.load(np.array([0, n_hits], np.int32), torch.from_numpy(h).to(gpu_device))
+
+    def run(m):
+        t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu_device)
+        xs, xa, w = t(np.zeros(m, np.int32)), t(np.zeros((16, m), np.int32)), t(np.zeros(m, np.int32))
+        eoh.select_hit_indices(0, t(par[:, :m]), t(err[:, :m]), xs, xa, w)
+        return xs.cpu().numpy(), xa.cpu().numpy(), w.cpu().numpy()
+    whole = run(n)
+    for m in (1, 3, 700, 1025, 9001, 40000):
+        assert all(np.array_equal(a, b[..., :m]) for a, b in zip(run(m), whole)), m
+    m = 400
+    xs, xa, w = oracle.select_hit_indices(d, h, np.ascontiguousarray(par[:, :m]), np.ascontiguousarray(err[:, :m]))
+    # one float rounding of a bin or window edge moves a lane's list: at most a lane in a hundred
+    same = (xs == whole[0][:m]) & (w == whole[2][:m])
+    for k in range(m):
+        same[k] &= np.array_equal(xa[:max(xs[k], 0), k], whole[1][:max(xs[k], 0), k])
+    assert same.mean() >= 0.99, same.mean()
+    eoh.close()
+    ctx.close()

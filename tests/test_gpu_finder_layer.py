@@ -248,3 +248,41 @@ def test_layer_steps_reject_bad_arguments(setup, gpu_device):
     with RawDeviceBuffer(n // 2 * 4) as short:
         with pytest.raises(mk.MkfError, match="hit_idx"):
             ctx.update_with_last_hit(eoh, 3, g, short)
+
+
+@pytest.mark.parametrize("prop_to_hit", [False, True])
+def test_layer_steps_for_every_packing(setup, gpu_device, prop_to_hit):
+    """Candidates per wavefront follow the number of lanes (1 to 64): records and states do not depend on it.  The
+    lists hold entries that are no hit of the layer (-1, beyond the last), which both steps pass over."""
+    import torch
+    ev, descs, ctx, eoh = setup
+    layer = 6
+    ln = _lanes_at(oracle.Oracle(bfield=3.8), ev, descs, layer, seed=layer)
+    xs, xa, w = oracle.select_hit_indices(descs[layer], _layer_hits(ev, layer), ln["prop_par"], ln["prop_err"])
+    n0 = 1100
+    xa, xs = xa[:, :n0].copy(), xs[:n0].copy()
+    xa[2, ::7] = -1
+    xa[0, ::11] = 1 << 29
+    rep = lambda a, idx: np.ascontiguousarray(np.asarray(a)[..., idx])
+
+    def run(idx):
+        g = _gpu_lanes({k: rep(v, idx) for k, v in ln.items() if isinstance(v, np.ndarray)}, gpu_device)
+        n = g.n
+        sel = [_t(rep(v, idx), gpu_device) for v in (xs, xa, w)]
+        ne = torch.zeros(n, dtype=torch.int32, device=gpu_device)
+        ent = torch.zeros(n * mk.CE_ENTRIES_PER_LANE * mk.IDX_CHI2_DTYPE.itemsize, dtype=torch.uint8, device=gpu_device)
+        code = torch.zeros(n, dtype=torch.int32, device=gpu_device)
+        ctx.find_candidates_clone_engine(eoh, layer, g, *sel, ne, ent, prop_to_hit=prop_to_hit)
+        ctx.add_best_hit(eoh, layer, g, *sel, code, prop_to_hit=prop_to_hit)
+        rec = ent.cpu().numpy().view(mk.IDX_CHI2_DTYPE).reshape(n, -1)
+        fields = {k: rec[k].T for k in rec.dtype.names if k != "trk_idx"}
+        return dict(g.numpy(), code=code.cpu().numpy(), ne=ne.cpu().numpy(), **fields)
+    whole = run(np.arange(n0))
+    assert whole["ne"].max() > 4 and (whole["code"] >= 0).mean() > 0.4
+    for n in (1, 63, 1025):
+        part = run(np.arange(n))
+        assert all(np.array_equal(part[k], whole[k][..., :n], equal_nan=True) for k in whole), n
+    for times in (2, 16, 61):
+        many = run(np.tile(np.arange(n0), times))
+        for k in whole:
+            assert np.array_equal(many[k], np.concatenate([whole[k]] * times, axis=-1), equal_nan=True), (times, k)
