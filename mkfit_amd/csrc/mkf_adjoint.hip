@@ -351,7 +351,11 @@ extern "C" int mkf_fit_adjoint(mkf_context* c, const mkf_adjoint_batch* b, void*
   if (b->n_tracks == 0) return adjoint_launch(c, b, 1, nullptr, 0, st);
   std::lock_guard<std::mutex> lk(c->mu);
   CHECK(scratch_acquire(c->adj_done, st));
-  int every = adjoint_spacing(b, sum_bytes, std::max(kAdjScratchFree, c->adj_bytes));
+  // A captured call that fits the scratch at the caller's spacing does not grow it.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &cap));
+  const bool fixed = cap != hipStreamCaptureStatusNone && need <= c->adj_bytes;
+  int every = adjoint_spacing(b, sum_bytes, fixed ? c->adj_bytes : std::max(kAdjScratchFree, c->adj_bytes));
   const size_t want = adjoint_bytes(b, every, sum_bytes);
   if (want > c->adj_bytes) {
     HIP_TRY(hipDeviceSynchronize());
