@@ -217,6 +217,8 @@ constexpr size_t kRowMeanMax = 2 * kRowCap;
 // 5.7M, 1517 / 1559 at 22.7M).
 constexpr size_t kStreamHits = 4000000;
 
+constexpr int kRowWeight = 100;      // a row's fixed cost in hits, for the XCDs' shares
+
 struct RowPair {
   float phi;
   int idx;      // hit index in its layer
@@ -322,6 +324,14 @@ k_row_partition(int n_layers, const int* __restrict__ tile_off, const LayerDev* 
   for (int j = t; j < n; j += kPartBlock) dst[j] = out[j];
 }
 
+// The rows each XCD takes, contiguous so that its L2 keeps the layers it gathers from, and of equal shares of the
+// hits (equal numbers of rows gave the XCD of the outermost layers of one event twice the hits of the first: best-hit
+// step 335 us, against 321 us with the rows dealt out singly and 310 us with equal shares; 50 events 7.21, 7.73 and
+// 7.13 ms).
+struct XcdRows {
+  int first[9];
+};
+
 // One q row per block; see above.  The pairs of a row come in any order within a
 // tile's part, so the order inside a fine phi bin (one to three hits) is set by
 // comparing indices.  A row that fits the LDS is read once; what it reads from
@@ -331,7 +341,7 @@ k_row_partition(int n_layers, const int* __restrict__ tile_off, const LayerDev* 
 // whose indices ascend.
 template <bool NT>
 __global__ void __launch_bounds__(kRowBlock)
-k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, const int* __restrict__ tile_off,
+k_row_sort(XcdRows xr, const int* __restrict__ row_layer, const LayerDev* __restrict__ L, const int* __restrict__ tile_off,
            const unsigned short* __restrict__ pre, int pre_stride, const RowPair* __restrict__ pairs,
            const float* __restrict__ hits, float* __restrict__ shits, float* __restrict__ phis,
            float* __restrict__ qs, int* __restrict__ ranks, int* __restrict__ place, int2* __restrict__ bins) {
@@ -342,7 +352,8 @@ k_row_sort(const int* __restrict__ row_layer, const LayerDev* __restrict__ L, co
   __shared__ int part[kRowBlock / 64];
   __shared__ int s_b1, s_cnt;
   const int t = threadIdx.x;
-  const int row = xcd_major_block();
+  const int row = xr.first[blockIdx.x % 8] + blockIdx.x / 8;
+  if (row >= xr.first[blockIdx.x % 8 + 1]) return;
   const int layer = row_layer[row];
   const LayerDev& d = L[layer];
   const int q = row - d.bin_off / kNPhi;
@@ -603,20 +614,28 @@ k_row_inverse(int n_layers, const int* __restrict__ tile_off, const LayerDev* __
   for (int j = t; j < n; j += kPartBlock) inv[g0 + j] = out[j];
 }
 
-// The iteration's hit mask in sorted order: mask_s[inv[j]] = mask[j] for every event hit j.
+// Per-hit bytes (the iteration's hit mask, as 0 or 1, or the charge codes) in sorted order, one tile of sorted
+// positions per block: out[i] = in[hit of sorted position i].  Gathered, because the bytes of a layer stay in L2 while
+// its outputs are written whole (scattering them by the inverse map: 19 us for 2.8M hits, against 6 us).
+template <bool MASK>
 __global__ void __launch_bounds__(256)
-k_mask_sorted(int total, const int* __restrict__ inv, const unsigned char* __restrict__ mask,
-              unsigned char* __restrict__ mask_s) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < total) mask_s[inv[j]] = mask[j] ? 1 : 0;
-}
-
-// The hits' charge codes in sorted order: charge_s[inv[j]] = code[j] for every event hit j.
-__global__ void __launch_bounds__(256)
-k_charge_sorted(int total, const int* __restrict__ inv, const unsigned char* __restrict__ code,
-                unsigned char* __restrict__ charge_s) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < total) charge_s[inv[j]] = code[j];
+k_bytes_sorted(int n_layers, const int* __restrict__ tile_off, const LayerDev* __restrict__ L,
+               const int* __restrict__ ranks, const unsigned char* __restrict__ in, unsigned char* __restrict__ out) {
+  const int tile = xcd_major_block();
+  const int l = layer_of_tile(tile, n_layers, tile_off);
+  const LayerDev& d = L[l];
+  const int first = (tile - tile_off[l]) * kTile;
+  const int n = min(kTile, d.n_hits - first), g0 = d.hit_off + first;
+  constexpr int kPer = kTile / 256;
+  int r[kPer];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) r[k] = ranks[g0 + min((int)threadIdx.x + k * 256, n - 1)];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int i = threadIdx.x + k * 256;
+    const unsigned char v = in[d.hit_off + r[k]];
+    if (i < n) out[g0 + i] = MASK ? (v ? 1 : 0) : v;
+  }
 }
 
 // One wavefront per workgroup, `lanes` of its lanes with a window each, scanned by all of them (25 -> 14 us for 30k
@@ -901,6 +920,13 @@ int grow(mkf_event_of_hits* h, size_t total, hipStream_t st) {
 }
 
 
+// Tiles of the loaded hits.
+int hit_tiles(const mkf_event_of_hits* h) {
+  int tiles = 0;
+  for (const LayerDev& d : h->layers) tiles += (d.n_hits + kTile - 1) / kTile;
+  return tiles;
+}
+
 int blocks_for(size_t n, int block) { return (int)std::max<size_t>(1, (n + block - 1) / block); }
 
 }  // namespace
@@ -1042,8 +1068,25 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
                          pairs, pre, pre_stride);
       HIP_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL((total > kStreamHits ? k_row_sort<true> : k_row_sort<false>), dim3(n_rows), dim3(kRowBlock), 0, st, h->d_row_layer, h->d_layers, h->d_tile_off,
-                       pre, pre_stride, pairs, hits, h->d_shits, h->d_phis, h->d_qs, h->d_ranks, place, h->d_bins);
+    // a row weighs its layer's mean of hits and a constant for the block itself
+    XcdRows xr;
+    const double all = (double)total + (double)kRowWeight * n_rows;
+    int x = 0, longest = 0;
+    double w = 0.0;
+    for (int l = 0; l < L; ++l) {
+      const LayerDev& d = h->layers[l];
+      const double each = (double)d.n_hits / d.nq + kRowWeight;
+      for (; x < 8 && w + each * d.nq > all * x / 8; ++x)
+        xr.first[x] = std::min(n_rows, d.bin_off / kNPhi + (int)std::max(0.0, std::ceil((all * x / 8 - w) / each)));
+      w += each * d.nq;
+    }
+    for (; x <= 8; ++x) xr.first[x] = n_rows;
+    xr.first[0] = 0;
+    xr.first[8] = n_rows;
+    for (int k = 0; k < 8; ++k) longest = std::max(longest, xr.first[k + 1] - xr.first[k]);
+    hipLaunchKernelGGL((total > kStreamHits ? k_row_sort<true> : k_row_sort<false>), dim3(8 * longest), dim3(kRowBlock), 0,
+                       st, xr, h->d_row_layer, h->d_layers, h->d_tile_off, pre, pre_stride, pairs, hits, h->d_shits,
+                       h->d_phis, h->d_qs, h->d_ranks, place, h->d_bins);
     HIP_TRY(hipGetLastError());
     if (tiles) {
       hipLaunchKernelGGL(k_row_inverse, dim3(tiles), dim3(kPartBlock), 0, st, L, h->d_tile_off, h->d_layers, pairs,
@@ -1100,8 +1143,8 @@ int mkf_event_of_hits_set_hit_mask(mkf_event_of_hits* h, const unsigned char* ma
     h->mask_cap = total;
   }
   if (total) {
-    hipLaunchKernelGGL(k_mask_sorted, dim3(blocks_for(total, 256)), dim3(256), 0, st, (int)total, h->d_inv, mask,
-                       h->d_mask_s);
+    hipLaunchKernelGGL(k_bytes_sorted<true>, dim3(hit_tiles(h)), dim3(256), 0, st, h->n_layers, h->d_tile_off,
+                       h->d_layers, h->d_ranks, mask, h->d_mask_s);
     HIP_TRY(hipGetLastError());
   }
   h->has_mask = true;
@@ -1129,8 +1172,8 @@ int mkf_event_of_hits_set_hit_charge(mkf_event_of_hits* h, const unsigned char* 
     h->charge_cap = total;
   }
   if (total) {
-    hipLaunchKernelGGL(k_charge_sorted, dim3(blocks_for(total, 256)), dim3(256), 0, st, (int)total, h->d_inv, code,
-                       h->d_charge_s);
+    hipLaunchKernelGGL(k_bytes_sorted<false>, dim3(hit_tiles(h)), dim3(256), 0, st, h->n_layers, h->d_tile_off,
+                       h->d_layers, h->d_ranks, code, h->d_charge_s);
     HIP_TRY(hipGetLastError());
   }
   h->has_charge = true;
