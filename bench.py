@@ -11,8 +11,7 @@ resident in HBM, output written out of place.
 
 Two forms of the same fit are timed on the same inputs:
   plain    -- mkf_fit_plain, one kernel launch per hit slot (state round-trips HBM)
-  batched  -- mkf_fit_batched: one fused kernel over all slots, replayed from a
-              cached hipGraph
+  batched  -- mkf_fit_batched: one fused kernel over all slots
 The batch is packed in fit order (hit count, then endcap/barrel slot pattern;
 mkfit_amd.fit_order), as a caller's packer would build it; both forms fit the
 same packed batch.  --unordered packs it in generation order instead.
@@ -246,11 +245,11 @@ def bench_fit(args, mk, torch, dev, uneven):
     ms_p = wall_p * 1e3 / args.steps
     tps_b = n / (ms_b * 1e-3)
     tps_p = n / (ms_p * 1e-3)
-    # one graph per step (with a sort tile: ordering + fused kernel): HIP events on its stream, graphs back to back
+    # one call per step (with a sort tile: ordering + fused kernel): HIP events on its stream, calls back to back
     graph_ms = float(launch_b)
     order_ms = 0.0
     if shape[3] > 0:
-        # the ordering kernel on its own (same kernel the graph replays), so the fused kernel's share is known
+        # the ordering kernel on its own (the same kernel), so the fused kernel's share is known
         order = torch.empty(n, dtype=torch.int32, device=dev)
         _, _, order_ms = timed(lambda: ctx.fit_order(batch, shape[3], order), args.steps, args.warmup)
     kern_b = graph_ms - order_ms

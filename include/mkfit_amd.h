@@ -122,8 +122,7 @@ typedef struct mkf_fit_batch {
 int mkf_fit_plain(mkf_context* ctx, const mkf_fit_batch* batch, void* stream);
 
 /* Batched fit: one persistent fused propagate+update kernel over the whole
- * batch, state kept in registers across slots, replayed from a cached hipGraph
- * when the same batch is fitted again.  Same results as mkf_fit_plain. */
+ * batch, state kept in registers across slots.  Same results as mkf_fit_plain. */
 int mkf_fit_batched(mkf_context* ctx, const mkf_fit_batch* batch, void* stream);
 
 /* Launch shape used by mkf_fit_batched (set by the autotuner or by hand). */

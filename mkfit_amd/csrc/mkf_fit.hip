@@ -10,9 +10,11 @@
 //              round trip through HBM per slot (~270 B per track-slot).
 //   batched -- k_fit launched once over all slots on a persistent grid: the
 //              state is loaded once, stays in VGPRs across the track's slots,
-//              and only the hits stream (~37 B per track-slot).  It is
-//              launched from a cached hipGraph; launch shape and register
-//              budget come from mkf_autotune_batched.
+//              and only the hits stream (~37 B per track-slot).  Launch shape
+//              and register budget come from mkf_autotune_batched.  (Replaying
+//              it from a cached hipGraph cost 4.7 us more per call than the
+//              launch itself, 1003 tracks 49.0 against 44.3 us, and a new
+//              batch the capture, 112 against 83 us for its first pass.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -20,10 +22,8 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <string>
-#include <tuple>
 #include <vector>
 
 #include "../../include/mkfit_amd.h"
@@ -554,14 +554,11 @@ bool shape_ok(const mkf_launch_shape& s) {
          (s.sort_tile == 0 || s.sort_tile == 1024 || s.sort_tile == 4096 || s.sort_tile == 16384);
 }
 
-// Grows the context's track-order buffer to n ints.  Cached graphs hold the
-// old address, so they are dropped (after the device drains) when it moves.
+// Grows the context's track-order buffer to n ints, after the device drains.
 // Called under c->mu.
 int ensure_fit_order(mkf_context* c, int n) {
   if ((size_t)n <= c->fit_order_cap) return MKF_OK;
   HIP_TRY(hipDeviceSynchronize());
-  for (auto& kv : c->graphs) HIP_TRY(hipGraphExecDestroy(kv.second.exec));
-  c->graphs.clear();
   if (c->fit_order) HIP_TRY(hipFree(c->fit_order));
   c->fit_order = nullptr;
   c->fit_order_cap = 0;
@@ -601,7 +598,7 @@ int mkf_context_create(const mkf_config* cfg, mkf_context** out) {
     if (e == hipSuccess) e = hipMemcpy(c->d_rl, cfg->rl_grid, bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->d_xi, cfg->xi_grid, bytes, hipMemcpyHostToDevice);
   }
-  if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->capture_stream, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->tune_stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     int rc = fail(MKF_ERR_HIP, "context setup: %s", hipGetErrorString(e));
     mkf_context_destroy(c);
@@ -619,8 +616,7 @@ int mkf_context_destroy(mkf_context* c) {
   if (!c) return MKF_OK;
   (void)hipSetDevice(c->device);
   (void)hipDeviceSynchronize();
-  for (auto& kv : c->graphs) (void)hipGraphExecDestroy(kv.second.exec);
-  if (c->capture_stream) (void)hipStreamDestroy(c->capture_stream);
+  if (c->tune_stream) (void)hipStreamDestroy(c->tune_stream);
   if (c->adj_scratch) (void)hipFree(c->adj_scratch);
   if (c->adj_done) (void)hipEventDestroy(c->adj_done);
   if (c->fit_order) (void)hipFree(c->fit_order);
@@ -736,44 +732,10 @@ int mkf_fit_batched(mkf_context* c, const mkf_fit_batch* b, void* stream) {
   std::lock_guard<std::mutex> lk(c->mu);
   const bool sorted = c->shape.sort_tile > 0;
   if (sorted) CHECK(ensure_fit_order(c, a.n));
-  GraphKey key;
-  const void* ptrs[12] = {b->par,    b->err,       b->chg,      b->chi2,     b->hit_pos,  b->hit_err,
-                          b->n_hits, b->hit_flags, b->seed_par, b->seed_err, b->seed_chg, nullptr};
-  std::memcpy(key.ptrs, ptrs, sizeof(ptrs));
-  key.n = a.n; key.slots = a.n_slots; key.pflags = a.pflags; key.fflags = a.fit_flags;
-  key.block = c->shape.block; key.bpc = c->shape.blocks_per_cu; key.variant = c->shape.variant;
-  key.pca_pflags = a.pca_pflags;
-  key.tile = c->shape.sort_tile;
-  auto it = c->graphs.find(key);
-  if (it == c->graphs.end()) {
-    if (c->graphs.size() >= mkf_context::kMaxGraphs) {
-      // Evict the least recently launched graph; a launch of it may still be
-      // in flight, so the device drains first (rare: only callers that cycle
-      // through more than kMaxGraphs distinct batches get here).
-      auto lru = c->graphs.begin();
-      for (auto j = c->graphs.begin(); j != c->graphs.end(); ++j)
-        if (j->second.last_use < lru->second.last_use) lru = j;
-      HIP_TRY(hipDeviceSynchronize());
-      HIP_TRY(hipGraphExecDestroy(lru->second.exec));
-      c->graphs.erase(lru);
-    }
-    hipGraph_t g = nullptr;
-    hipGraphExec_t ge = nullptr;
-    HIP_TRY(hipStreamBeginCapture(c->capture_stream, hipStreamCaptureModeThreadLocal));
-    int rc = launch_fused(c, a, c->shape, c->fit_order, c->capture_stream);
-    hipError_t e = hipStreamEndCapture(c->capture_stream, &g);
-    if (rc) { if (g) (void)hipGraphDestroy(g); return rc; }
-    if (e != hipSuccess) return fail(MKF_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
-    e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    if (e != hipSuccess) return fail(MKF_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(e));
-    it = c->graphs.emplace(key, mkf_context::GraphEntry{ge, 0}).first;
-  }
-  it->second.last_use = ++c->graph_tick;
   // The track-order buffer is shared by every call on this context: a call on
-  // another stream waits for the previous call's graph to finish with it.
+  // another stream waits for the previous call to finish with it.
   if (sorted) CHECK(scratch_acquire(c->fit_done, (hipStream_t)stream));
-  HIP_TRY(hipGraphLaunch(it->second.exec, (hipStream_t)stream));
+  CHECK(launch_fused(c, a, c->shape, c->fit_order, (hipStream_t)stream));
   if (sorted) CHECK(scratch_release(c->fit_done, (hipStream_t)stream));
   return MKF_OK;
 }
@@ -816,7 +778,7 @@ int mkf_autotune_batched(mkf_context* c, const mkf_fit_batch* b, float* scratch,
   if (reps < 1) reps = 1;
   const size_t N = a.n;
   CHECK(check_dev(scratch, 29 * N * 4, "scratch_state"));
-  hipStream_t st = c->capture_stream;
+  hipStream_t st = c->tune_stream;
   // Save the state the fit mutates: par, err, chi2, chg.
   auto save = [&](bool restore) -> hipError_t {
     const hipMemcpyKind k = hipMemcpyDeviceToDevice;

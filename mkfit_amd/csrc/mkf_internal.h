@@ -9,10 +9,8 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <string>
-#include <tuple>
 
 #include "../../include/mkfit_amd.h"
 #include "mkf_track_math.h"
@@ -20,17 +18,6 @@
 // ============================================================================
 // Context and error reporting
 // ============================================================================
-
-struct GraphKey {
-  const void* ptrs[12];
-  int n, slots, pflags, fflags, block, bpc, variant, pca_pflags, tile;
-  bool operator<(const GraphKey& o) const {
-    int c = std::memcmp(ptrs, o.ptrs, sizeof(ptrs));
-    if (c) return c < 0;
-    return std::tie(n, slots, pflags, fflags, block, bpc, variant, pca_pflags, tile) <
-           std::tie(o.n, o.slots, o.pflags, o.fflags, o.block, o.bpc, o.variant, o.pca_pflags, o.tile);
-  }
-};
 
 struct mkf_context {
   int device = 0;
@@ -40,17 +27,7 @@ struct mkf_context {
   float* d_xi = nullptr;
   mkf_launch_shape shape{256, 0, 0, 0};
   mkf_find_shape find_shape[2] = {{0, 2}, {0, 2}};   // clone engine, standard finding
-  hipStream_t capture_stream = nullptr;
-  // Instantiated batched-fit graphs by batch (pointers, sizes, flags, shape),
-  // at most kMaxGraphs; the least recently launched one is destroyed to make
-  // room for a new one.
-  struct GraphEntry {
-    hipGraphExec_t exec;
-    unsigned long long last_use;
-  };
-  static constexpr size_t kMaxGraphs = 16;
-  std::map<GraphKey, GraphEntry> graphs;
-  unsigned long long graph_tick = 0;
+  hipStream_t tune_stream = nullptr;
   std::mutex mu;
   void* adj_scratch = nullptr;   // adjoint checkpoints and per-track gradient rows
   size_t adj_bytes = 0;
@@ -58,8 +35,7 @@ struct mkf_context {
   // kernel that touches adj_scratch; the next call's stream waits on it, so
   // calls on different streams take the scratch one after the other.
   hipEvent_t adj_done = nullptr;
-  // Track order of the batched fit (sort tiles), n_tracks ints; the graphs
-  // capture its address, so growing it drops every cached graph.  fit_done
+  // Track order of the batched fit (sort tiles), n_tracks ints.  fit_done
   // orders its users across streams as adj_done does for adj_scratch.
   int* fit_order = nullptr;
   size_t fit_order_cap = 0;
