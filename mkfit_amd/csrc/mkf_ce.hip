@@ -1,6 +1,6 @@
 // mkf_ce.hip -- clone-engine track finding on gfx950.
 //
-// One 64-lane workgroup carries 8 or 10 seeds through every layer: lane
+// One 64-lane workgroup carries up to 8 or 10 seeds through every layer: lane
 // g*KS + c holds candidate c of seed g (KS = 8 slots per seed, or 6 when at most
 // 6 candidates are kept) with its state in VGPRs.
 // Per layer:
@@ -445,7 +445,8 @@ __global__ void __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(WAV
     __syncthreads();
     // ---- (b) CandCloner::ProcessSeedRange.  Each lane's entries are its records, its invalid-hit record and (STD,
     // where find_tracks_handle_missed_layers runs before FindCandidates) itself when held back; K times the group
-    // takes the best of the lanes' best remaining ones.
+    // takes the best of the lanes' best remaining ones.  (One lane per seed merging all records took 28k of a
+    // wavefront's 104k cycles per layer, this and the layout below 10k: 15.7 -> 13.4 ms for 500k seeds.)
     {
       const int l0 = g * kS;
       const int fc = fcode[lane];

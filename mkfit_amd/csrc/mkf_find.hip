@@ -203,14 +203,18 @@ k_loh_fill(int total, int pass, const uint32_t* __restrict__ keys_s, const int* 
 // everything the finders read: the hits, phi, q, ranks, the inverse map and the
 // row's bin ranges.  A hit moves 36 + 8 bytes in the first kernel and 8 + 36 + 52
 // in the second, against 36 + 8, four radix passes of 16, 8 + 36 + 44 and 8 + 16
-// for keys, sort, gather and fill.
+// for keys, sort, gather and fill.  Over 141.7M hits in 850 layers: 1.16 ms (5.4 TB/s) + 3.8 ms (23 GB moved, 15 of
+// them read for 6: a gathered hit's 128-byte line is fetched for three or four rows, and a layer exceeds an XCD's
+// L2) + 0.39 ms for the inverse map, against 10.6 ms.
 constexpr int kTile = 3072;          // hits per tile; also the LDS capacity of k_row_sort, so one tile's part
 constexpr int kRowCap = kTile;       // of a row always fits
 constexpr int kPartBlock = 512, kRowBlock = 256;
 constexpr int kFineBins = 1025;      // fine phi bins 0..1024 (1024: phi == +pi)
 static_assert(kTile % kPartBlock == 0 && kRowCap % kRowBlock == 0 && kTile <= 0xffff, "tile size");
-// Layers with more hits than this per q bin go through the radix sort: one block per row leaves the chip idle.
-constexpr size_t kRowMeanMax = 2 * kRowCap;
+// Layers with more hits than this per q bin go through the radix sort: a block reads a row beyond kRowCap once per
+// run of bins that fits, and few rows leave the chip idle (17 layers of 167k hits, rows / radix sort: 116 / 289 us at
+// 1391 hits per bin, 193 / 290 at 6185, 289 / 287 at 10437, 1760 / 285 at 41750).
+constexpr size_t kRowMeanMax = 3 * kRowCap;
 
 // Beyond this many hits the sorted copies are stored past the caches: the 256 MB last-level cache no longer keeps
 // them for the finder (best-hit step, stored past / through the caches: 562 / 516 us at 2.8M hits, 723 / 742 at
@@ -706,7 +710,9 @@ struct FindArgs {
 // evaluated as (seed, hit) pairs spread over its lanes, so a layer waits for a few
 // batches of loads instead of one per hit of the fullest window.  A wavefront
 // carries `spw` seeds: 64 when there are enough to fill the chip, fewer otherwise,
-// since the lanes without a seed still share the scan and the pairs.
+// since the lanes without a seed still share the scan and the pairs.  (One lane per seed scanning and evaluating its
+// own hits: 241 us for 500 seeds, 2.35 ms for 500k; so 120 us, bound by 8.5 us of dependent work per layer, and
+// 1.8 ms, bound by the gathers' L2 misses.)
 struct BestHitLds {
   ScanLds scan;
   float c2[64][kHitIdxMax];
