@@ -20,6 +20,8 @@
 #ifndef MKFIT_AMD_H
 #define MKFIT_AMD_H
 
+#include <stddef.h>
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -170,8 +172,12 @@ int mkf_num_batched_variants(void);
  *              x' = x - d_rphi y/r, y' = y + d_rphi x/r, z' = z + d_z.
  * The forward states are kept at least every `checkpoint_every` layers and are
  * recomputed between on the way back; more of them are kept (down to every
- * layer, which recomputes none) while the scratch stays within 512 MiB (or
- * what earlier calls on the context took).  The results do not depend on it. */
+ * layer, which recomputes none) while the scratch allows.  The results do not
+ * depend on it.  The context holds the scratch: a call that it cannot hold at
+ * the caller's spacing replaces it (draining the device), by up to
+ * mkf_set_adjoint_scratch_limit bytes (512 MiB by default) or by what that
+ * spacing takes if that is more, or all there is; every other call takes it as
+ * it is, so that a captured call stays valid until a call that does not fit. */
 typedef struct mkf_adjoint_batch {
   int n_tracks, n_layers;
   const float* seed_par;  /* [6][n] */
@@ -193,6 +199,10 @@ typedef struct mkf_adjoint_batch {
 } mkf_adjoint_batch;
 
 int mkf_fit_adjoint(mkf_context* ctx, const mkf_adjoint_batch* batch, void* stream);
+
+/* Bytes up to which a growing scratch of mkf_fit_adjoint keeps more states than checkpoint_every asks for; 0: just
+ * those.  Scratch already held is not given back. */
+int mkf_set_adjoint_scratch_limit(mkf_context* ctx, size_t bytes);
 
 /* mkf_fit_adjoint without any device allocation: no counterpart in the reference.  For callers that cannot
  * allocate device memory -- code under HIP graph capture, tight fit-and-descend loops, harnesses that forbid

@@ -102,7 +102,7 @@ ABI_SYMBOLS = [
     "mkf_add_best_hit", "mkf_find_candidates_clone_engine", "mkf_update_with_last_hit",
     "mkf_fit_adjoint", "mkf_fit_adjoint_noalloc", "mkf_backward_fit", "mkf_find_tracks_standard",
     "mkf_set_find_shape", "mkf_get_find_shape", "mkf_autotune_find", "mkf_event_of_hits_set_hit_mask",
-    "mkf_event_of_hits_set_dead_regions", "mkf_event_of_hits_set_hit_charge",
+    "mkf_event_of_hits_set_dead_regions", "mkf_event_of_hits_set_hit_charge", "mkf_set_adjoint_scratch_limit",
 ]
 CE_MAX_CANDS = 8
 
@@ -204,6 +204,7 @@ def lib():
         L.mkf_find_tracks_best_hit.argtypes = [_c_void_p, _c_void_p, ctypes.POINTER(MkfFindBatch), _c_void_p]
         L.mkf_find_tracks_clone_engine.argtypes = [_c_void_p, _c_void_p, ctypes.POINTER(MkfCEBatch), _c_void_p]
         L.mkf_fit_adjoint.argtypes = [_c_void_p, ctypes.POINTER(MkfAdjointBatch), _c_void_p]
+        L.mkf_set_adjoint_scratch_limit.argtypes = [_c_void_p, ctypes.c_size_t]
         L.mkf_add_best_hit.argtypes = [_c_void_p, _c_void_p, ctypes.c_int, ctypes.POINTER(MkfFinderLanes)] + \
             [_c_void_p] * 3 + [ctypes.c_float, ctypes.c_int, ctypes.c_int, _c_void_p, _c_void_p]
         L.mkf_find_candidates_clone_engine.argtypes = [_c_void_p, _c_void_p, ctypes.c_int,
@@ -867,6 +868,10 @@ class Context:
         s = MkfLaunchShape()
         _check(lib().mkf_get_batched_shape(self.h, ctypes.byref(s)))
         return (s.block, s.blocks_per_cu, s.variant, s.sort_tile)
+
+    def set_adjoint_scratch_limit(self, nbytes):
+        """Bytes up to which a growing scratch of the fit's gradient keeps more states than checkpoint_every asks."""
+        _check(lib().mkf_set_adjoint_scratch_limit(self.h, int(nbytes)))
 
     def set_find_shape(self, standard, slots=0, waves_per_simd=2):
         """Launch shape of the clone-engine (standard=False) or standard finder (mkf_set_find_shape)."""

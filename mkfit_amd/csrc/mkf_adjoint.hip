@@ -227,27 +227,8 @@ static __device__ __align__(256) unsigned char scratch[kAdjNoallocBytes];
 
 namespace {
 
-// Scratch of a batch that keeps every `every`-th state: the sums' partials (sum_bytes, 256-byte aligned),
-// checkpoints, per-track gradient rows.
-size_t adjoint_bytes(const mkf_adjoint_batch* b, int every, size_t sum_bytes) {
-  const size_t N = b->n_tracks, L = b->n_layers, n_ck = (L + every - 1) / every, word = b->fp64 ? 8 : 4;
-  return sum_bytes + (n_ck * 27 + L * 3) * N * word;
-}
-
-// The spacing a call uses: one, so that the reverse sweep recomputes no state, when the scratch for it stays within
-// `limit`; else the shortest that does, and the caller's at least.  The gradient does not depend on it.  Recomputing
-// the states of five-layer segments is two of the seven forward steps' worth of work per layer (100k tracks, 25
-// layers: 804 us at a spacing of 5, 496 us at 1), while a state's store and load are 216 bytes.
-int adjoint_spacing(const mkf_adjoint_batch* b, size_t sum_bytes, size_t limit) {
-  int every = 1;
-  while (every < b->checkpoint_every && adjoint_bytes(b, every, sum_bytes) > limit) ++every;
-  return every;
-}
-constexpr size_t kAdjScratchFree = (size_t)512 << 20;
-
-// Checks the batch; returns through `need` the scratch bytes the call takes at the caller's spacing and through
-// `sum_bytes` the 256-byte aligned size of the sums' partials at its front.
-int adjoint_check(const mkf_adjoint_batch* b, size_t& need, size_t& sum_bytes) {
+// Checks the batch and returns through `z` the scratch it takes.
+int adjoint_check(const mkf_adjoint_batch* b, AdjointSize& z) {
   if (!b) return fail(MKF_ERR_INVALID_ARG, "batch is NULL");
   if (b->n_tracks < 0 || b->n_layers <= 0 || b->n_layers > 1024)
     return fail(MKF_ERR_INVALID_ARG, "need n_tracks >= 0 and 1 <= n_layers <= 1024");
@@ -257,8 +238,6 @@ int adjoint_check(const mkf_adjoint_batch* b, size_t& need, size_t& sum_bytes) {
   const size_t N = b->n_tracks, L = b->n_layers;
   CHECK(check_dev(b->theta, L * 3 * 4, "theta"));
   CHECK(check_dev(b->grad, L * 3 * 4, "grad"));
-  need = 0;
-  sum_bytes = 0;
   if (N == 0) return MKF_OK;
   if (L * 6 * N * 4 >= ((size_t)1 << 32)) return fail(MKF_ERR_INVALID_ARG, "batch too large");
   CHECK(check_dev(b->seed_par, 6 * N * 4, "seed_par"));
@@ -268,13 +247,16 @@ int adjoint_check(const mkf_adjoint_batch* b, size_t& need, size_t& sum_bytes) {
   CHECK(check_dev(b->hit_err, L * 6 * N * 4, "hit_err"));
   CHECK(check_dev(b->n_hits, N * 4, "n_hits"));
   CHECK(check_dev(b->chi2, N * 4, "chi2"));
-  sum_bytes = (L * 3 * kSumParts * sizeof(double) + 255) / 256 * 256;
-  need = adjoint_bytes(b, b->checkpoint_every, sum_bytes);
+  z.n = N;
+  z.layers = L;
+  z.word = b->fp64 ? 8 : 4;
+  z.sum_bytes = (L * 3 * kSumParts * sizeof(double) + 255) / 256 * 256;
+  z.asked = b->checkpoint_every;
   return MKF_OK;
 }
 
 // The forward fit, reverse sweep and sums of a checked batch, states kept every `every` layers, with `scr` holding
-// at least adjoint_bytes.  Every byte of the scratch that a kernel reads is written earlier in the same call.
+// at least AdjointSize::bytes(every).  Every byte of the scratch that a kernel reads is written earlier in the same call.
 int adjoint_launch(const mkf_context* c, const mkf_adjoint_batch* b, int every, void* scr, size_t sum_bytes,
                    hipStream_t st) {
   const size_t N = b->n_tracks, L = b->n_layers;
@@ -345,46 +327,46 @@ int adjoint_noalloc_setup(mkf_context* c) {
 
 extern "C" int mkf_fit_adjoint(mkf_context* c, const mkf_adjoint_batch* b, void* stream) {
   CHECK(set_device(c));
-  size_t need = 0, sum_bytes = 0;
-  CHECK(adjoint_check(b, need, sum_bytes));
+  AdjointSize z;
+  CHECK(adjoint_check(b, z));
   hipStream_t st = (hipStream_t)stream;
   if (b->n_tracks == 0) return adjoint_launch(c, b, 1, nullptr, 0, st);
   std::lock_guard<std::mutex> lk(c->mu);
   CHECK(scratch_acquire(c->adj_done, st));
-  // A captured call that fits the scratch at the caller's spacing does not grow it.
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(st, &cap));
-  const bool fixed = cap != hipStreamCaptureStatusNone && need <= c->adj_bytes;
-  int every = adjoint_spacing(b, sum_bytes, fixed ? c->adj_bytes : std::max(kAdjScratchFree, c->adj_bytes));
-  const size_t want = adjoint_bytes(b, every, sum_bytes);
-  if (want > c->adj_bytes) {
-    HIP_TRY(hipDeviceSynchronize());
-    if (c->adj_scratch) HIP_TRY(hipFree(c->adj_scratch));
-    c->adj_scratch = nullptr;
-    c->adj_bytes = 0;
-    size_t got = want;
-    if (hipMalloc(&c->adj_scratch, want) != hipSuccess) {   // a full device: the caller's spacing
-      (void)hipGetLastError();
-      c->adj_scratch = nullptr;
-      every = b->checkpoint_every;
-      got = need;
-      HIP_TRY(hipMalloc(&c->adj_scratch, need));
-    }
-    c->adj_bytes = got;
-  }
-  CHECK(adjoint_launch(c, b, every, c->adj_scratch, sum_bytes, st));
+  hipError_t e = hipSuccess;
+  const int every = adjoint_ready(
+      c->adj, z,
+      [&](void* p) {
+        e = hipDeviceSynchronize();
+        if (e == hipSuccess && p) e = hipFree(p);
+        return e == hipSuccess;
+      },
+      [&](size_t bytes) {
+        void* p = nullptr;
+        e = hipMalloc(&p, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e == hipSuccess ? p : nullptr;
+      });
+  if (!every) return fail(MKF_ERR_HIP, "adjoint scratch of %zu bytes: %s", z.need(), hipGetErrorString(e));
+  CHECK(adjoint_launch(c, b, every, c->adj.p, z.sum_bytes, st));
   return scratch_release(c->adj_done, st);
+}
+
+extern "C" int mkf_set_adjoint_scratch_limit(mkf_context* c, size_t bytes) {
+  if (!c) return fail(MKF_ERR_INVALID_ARG, "context is NULL");
+  std::lock_guard<std::mutex> lk(c->mu);
+  c->adj.limit = bytes;
+  return MKF_OK;
 }
 
 extern "C" int mkf_fit_adjoint_noalloc(mkf_context* c, const mkf_adjoint_batch* b, void* stream) {
   CHECK(set_device(c));
-  size_t need = 0, sum_bytes = 0;
-  CHECK(adjoint_check(b, need, sum_bytes));
+  AdjointSize z;
+  CHECK(adjoint_check(b, z));
   if (!c->adj_static) return fail(MKF_ERR_HIP, "no-allocation scratch not set up for this context");
-  if (need > c->adj_static_bytes)
+  if (z.need() > c->adj_static_bytes)
     return fail(MKF_ERR_INVALID_ARG,
                 "batch needs %zu bytes of adjoint scratch; mkf_fit_adjoint_noalloc has %zu (fewer tracks, or a "
-                "larger checkpoint_every)", need, c->adj_static_bytes);
-  return adjoint_launch(c, b, adjoint_spacing(b, sum_bytes, c->adj_static_bytes), c->adj_static, sum_bytes,
-                        (hipStream_t)stream);
+                "larger checkpoint_every)", z.need(), c->adj_static_bytes);
+  return adjoint_launch(c, b, z.spacing(c->adj_static_bytes), c->adj_static, z.sum_bytes, (hipStream_t)stream);
 }

@@ -617,7 +617,7 @@ int mkf_context_destroy(mkf_context* c) {
   (void)hipSetDevice(c->device);
   (void)hipDeviceSynchronize();
   if (c->tune_stream) (void)hipStreamDestroy(c->tune_stream);
-  if (c->adj_scratch) (void)hipFree(c->adj_scratch);
+  if (c->adj.p) (void)hipFree(c->adj.p);
   if (c->adj_done) (void)hipEventDestroy(c->adj_done);
   if (c->fit_order) (void)hipFree(c->fit_order);
   if (c->fit_done) (void)hipEventDestroy(c->fit_done);

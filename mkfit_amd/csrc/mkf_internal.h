@@ -13,6 +13,7 @@
 #include <string>
 
 #include "../../include/mkfit_amd.h"
+#include "mkf_adjoint_scratch.h"
 #include "mkf_track_math.h"
 
 // ============================================================================
@@ -29,14 +30,13 @@ struct mkf_context {
   mkf_find_shape find_shape[2] = {{0, 2}, {0, 2}};   // clone engine, standard finding
   hipStream_t tune_stream = nullptr;
   std::mutex mu;
-  void* adj_scratch = nullptr;   // adjoint checkpoints and per-track gradient rows
-  size_t adj_bytes = 0;
+  AdjointScratch adj;            // adjoint checkpoints and per-track gradient rows
   // Recorded on the stream of the last mkf_fit_adjoint call after its last
-  // kernel that touches adj_scratch; the next call's stream waits on it, so
+  // kernel that touches adj; the next call's stream waits on it, so
   // calls on different streams take the scratch one after the other.
   hipEvent_t adj_done = nullptr;
   // Track order of the batched fit (sort tiles), n_tracks ints.  fit_done
-  // orders its users across streams as adj_done does for adj_scratch.
+  // orders its users across streams as adj_done does for adj.
   int* fit_order = nullptr;
   size_t fit_order_cap = 0;
   hipEvent_t fit_done = nullptr;

@@ -124,6 +124,50 @@ def test_kept_and_recomputed_states_agree(gpu_device, n, fp64):
     ctx.close()
 
 
+def test_captured_call_outlives_a_larger_eager_one(gpu_device):
+    """A gradient call recorded in a graph keeps the scratch it was recorded with: an eager call of more tracks that
+    the scratch holds at its own spacing runs in it, and every later replay gives the first call's result."""
+    import torch
+    ev, geo, th = make_event(30000, seed=33)
+    ctx = mk.Context(bfield=3.8)
+    small = mk.AlignmentData(ctx, {k: np.ascontiguousarray(v[..., :20000]) for k, v in ev.items()}, gpu_device)
+    large = mk.AlignmentData(ctx, ev, gpu_device)
+    theta = _theta(th, gpu_device)
+    ref = [x.clone() for x in small.run(theta)]
+    alone = mk.Context(bfield=3.8)
+    want = [x.clone() for x in mk.AlignmentData(alone, ev, gpu_device).run(theta)]
+    torch.cuda.synchronize()
+    g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(g, stream=s):
+        out = small.run(theta)
+    for _ in range(3):
+        got = large.run(theta)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        for x in out:
+            x.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, ref))
+    del g
+    ctx.close()
+    alone.close()
+
+
+@pytest.mark.parametrize("limit", [0, 9 << 20, 1 << 30])
+def test_scratch_limit_does_not_change_the_result(setup, gpu_device, limit):
+    import torch
+    ev, geo, th, ctx = setup
+    theta = _theta(th, gpu_device)
+    ref = mk.AlignmentData(ctx, ev, gpu_device).run(theta)
+    other = mk.Context(bfield=3.8)
+    other.set_adjoint_scratch_limit(limit)
+    got = mk.AlignmentData(other, ev, gpu_device).run(theta)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))
+    other.close()
+
+
 def test_autograd_harness(setup, gpu_device):
     import torch
     from mkfit_amd.autograd import fit_chi2
