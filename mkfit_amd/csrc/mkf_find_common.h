@@ -223,8 +223,15 @@ __device__ __forceinline__ int wave_inclusive(int v) {
 // list is the window's count so far plus the passing hits of the groups before it;
 // the lists hold the same hits in the same order as scan_window's.  One wavefront
 // per workgroup.
+//
+// That reads every hit of the windows, while a lane that scans its own window stops at 16 hits.  So when a window
+// holds more than kScanLaneMax chunks, or all more than the work list, each lane scans its own (k_select of 1000 / 30k
+// / 100k windows in us, always by the wavefront, always by lane, and by this rule: 21 chunks a window 17 / 36 / 96,
+// 42 / 48 / 65, 17 / 36 / 53; 200 chunks 62 / 380 / 1371, 50 / 60 / 72, 25 / 39 / 50; a whole layer of 50k hits 3022 /
+// 87738 / 329678, 20 / 17 / 27, 15 / 19 / 23).
 constexpr int kChunk = 8, kChunkGroups = 64 / kChunk;
 constexpr int kScanDescs = 1024;
+constexpr int kScanLaneMax = 64;
 constexpr int kScanBatch = 4;                 // chunks per group whose loads are in flight together
 constexpr int kScanRows = 4;                  // q rows whose bin ranges are read together
 struct ScanLds {
@@ -239,11 +246,12 @@ __device__ __forceinline__ int wave_scan(bool active, const LayerDev& d, const W
                                          const float* __restrict__ qs, const unsigned char* __restrict__ mask,
                                          ScanLds& S) {
   const int lane = threadIdx.x & 63, group = lane / kChunk, gl = lane % kChunk;
-  // Runs of the window's bins that avoid bin 0, or bin 0 itself, in scan order: run(first position, hits).
-  auto each_run = [&](auto&& run) {
-    for (int qi = w.qb1; qi < w.qb2; ++qi) {
+  // Runs of the window's bins that avoid bin 0, or bin 0 itself, in scan order: run(first position, hits), until
+  // there are too many chunks.
+  auto each_run = [&](const int& chunks, auto&& run) {
+    for (int qi = w.qb1; qi < w.qb2 && chunks <= kScanLaneMax; ++qi) {
       const int2* __restrict__ row = bins + d.bin_off + qi * kNPhi;
-      for (int pi = w.pb1; pi < w.pb2;) {
+      for (int pi = w.pb1; pi < w.pb2 && chunks <= kScanLaneMax;) {
         const int b = pi & 0xff;
         const int b2 = b == 0 ? 0 : min(kNPhi - 1, b + (w.pb2 - 1 - pi));
         const int lo = row[b].x, hi = row[b2].y;
@@ -271,62 +279,66 @@ __device__ __forceinline__ int wave_scan(bool active, const LayerDev& d, const W
     lo[r] += d.hit_off;
     nch += (len[r] + kChunk - 1) / kChunk;
   }
-  if (active && !plain) each_run([&](int, int h) { nch += (h + kChunk - 1) / kChunk; });
-  const int incl = wave_inclusive(nch);
-  const int total = __shfl(incl, 63, 64), first = incl - nch;
+  if (active && !plain) each_run(nch, [&](int, int h) { nch += (h + kChunk - 1) / kChunk; });
+  const bool wide = __any(nch > kScanLaneMax);
+  const int incl = wave_inclusive(min(nch, kScanLaneMax + 1));
+  const int total = __shfl(incl, 63, 64);
   __syncthreads();
+  if (wide || total > kScanDescs) {
+    int c = 0;
+    if (active) scan_window(d, w, bins, phis, qs, mask, [&](int gi) { S.list[lane][c++] = gi; });
+    S.cnt[lane] = c;
+    __syncthreads();
+    return c;
+  }
   if (active) S.win[lane] = make_float4(w.q, w.phi, w.dq, w.dphi);
   S.cnt[lane] = 0;
-  for (int r0 = 0; r0 < total; r0 += kScanDescs) {
-    if (active) {
-      int id = first - r0, k = 0;
-      auto add = [&](int at, int hits) {
-        for (int h = 0; h < hits; h += kChunk, ++id, ++k)
-          if (id >= 0 && id < kScanDescs) S.desc[id] = make_int2(at + h, lane | min(kChunk, hits - h) << 6 | min(k, kChunkGroups) << 10);
-      };
-      if (plain) {
+  if (active) {
+    int id = incl - nch, k = 0;
+    auto add = [&](int at, int hits) {
+      for (int h = 0; h < hits; h += kChunk, ++id, ++k)
+        S.desc[id] = make_int2(at + h, lane | min(kChunk, hits - h) << 6 | min(k, kChunkGroups) << 10);
+    };
+    if (plain) {
 #pragma unroll
-        for (int r = 0; r < kScanRows; ++r) add(lo[r], len[r]);
-      } else {
-        each_run(add);
-      }
+      for (int r = 0; r < kScanRows; ++r) add(lo[r], len[r]);
+    } else {
+      each_run(k, add);
     }
-    __syncthreads();
-    const int m = min(kScanDescs, total - r0);
-    for (int c0 = 0; c0 < m; c0 += kChunkGroups * kScanBatch) {
-      int2 dd[kScanBatch];
-      float hq[kScanBatch], hp[kScanBatch];
-      bool taken[kScanBatch];
+  }
+  __syncthreads();
+  for (int c0 = 0; c0 < total; c0 += kChunkGroups * kScanBatch) {
+    int2 dd[kScanBatch];
+    float hq[kScanBatch], hp[kScanBatch];
+    bool taken[kScanBatch];
 #pragma unroll
-      for (int u = 0; u < kScanBatch; ++u) {
-        const int c = c0 + u * kChunkGroups + group;
-        dd[u] = c < m ? S.desc[c] : make_int2(0, 0);
-        const bool in = gl < ((dd[u].y >> 6) & 0xf);
-        hq[u] = in ? qs[dd[u].x + gl] : 0.f;
-        hp[u] = in ? phis[dd[u].x + gl] : 0.f;
-        taken[u] = in && mask && mask[dd[u].x + gl];
-      }
-#pragma unroll
-      for (int u = 0; u < kScanBatch; ++u) {
-        const int wl = dd[u].y & 63, hits = (dd[u].y >> 6) & 0xf, k = dd[u].y >> 10;
-        const float4 v = S.win[wl];
-        const float ddq = fabsf(v.x - hq[u]);
-        const float ddphi = cdist(fabsf(v.y - hp[u]));
-        const bool pass = gl < hits && !(ddq >= v.z || ddphi >= v.w) && !taken[u];
-        const uint64_t all = __ballot(pass);
-        const int g0 = max(group - k, 0);                    // this window's first group in the step
-        const uint64_t mine = all >> (g0 * kChunk) << (g0 * kChunk);
-        const int before = S.cnt[wl];
-        const int at = before + __popcll(mine & ((1ull << lane) - 1));
-        if (pass && at < kHitIdxMax) S.list[wl][at] = dd[u].x + gl;
-        // the window's last group in the step adds up
-        const int next = __shfl_down(dd[u].y, kChunk, 64);
-        if (gl == 0 && hits && (group == kChunkGroups - 1 || ((next >> 6) & 0xf) == 0 || next >> 10 == 0))
-          S.cnt[wl] = before + __popcll(mine & (~0ull >> (64 - (group + 1) * kChunk)));
-        __syncthreads();
-      }
+    for (int u = 0; u < kScanBatch; ++u) {
+      const int c = c0 + u * kChunkGroups + group;
+      dd[u] = c < total ? S.desc[c] : make_int2(0, 0);
+      const bool in = gl < ((dd[u].y >> 6) & 0xf);
+      hq[u] = in ? qs[dd[u].x + gl] : 0.f;
+      hp[u] = in ? phis[dd[u].x + gl] : 0.f;
+      taken[u] = in && mask && mask[dd[u].x + gl];
     }
-    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kScanBatch; ++u) {
+      const int wl = dd[u].y & 63, hits = (dd[u].y >> 6) & 0xf, k = dd[u].y >> 10;
+      const float4 v = S.win[wl];
+      const float ddq = fabsf(v.x - hq[u]);
+      const float ddphi = cdist(fabsf(v.y - hp[u]));
+      const bool pass = gl < hits && !(ddq >= v.z || ddphi >= v.w) && !taken[u];
+      const uint64_t all = __ballot(pass);
+      const int g0 = max(group - k, 0);                    // this window's first group in the step
+      const uint64_t mine = all >> (g0 * kChunk) << (g0 * kChunk);
+      const int before = S.cnt[wl];
+      const int at = before + __popcll(mine & ((1ull << lane) - 1));
+      if (pass && at < kHitIdxMax) S.list[wl][at] = dd[u].x + gl;
+      // the window's last group in the step adds up
+      const int next = __shfl_down(dd[u].y, kChunk, 64);
+      if (gl == 0 && hits && (group == kChunkGroups - 1 || ((next >> 6) & 0xf) == 0 || next >> 10 == 0))
+        S.cnt[wl] = before + __popcll(mine & (~0ull >> (64 - (group + 1) * kChunk)));
+      __syncthreads();
+    }
   }
   __syncthreads();
   return active ? min(S.cnt[lane], kHitIdxMax) : 0;

@@ -576,3 +576,88 @@ def test_select_for_every_packing_and_window(gpu_device, min_dphi, min_dq):
     assert same.mean() >= 0.99, same.mean()
     eoh.close()
     ctx.close()
+
+
+def _one_layer(n_hits, rng, min_dphi, min_dq):
+    d = dict(is_barrel=1, rin=19.99, rout=20.01, zmin=-60.0, zmax=60.0, propagate_to=20.0, q_bin=2.0, min_dphi=min_dphi,
+             max_dphi=3.14, min_dq=min_dq, max_dq=400.0, c_dp_sf=1.1, c_dq_sf=1.1, c_c2_sf=1.1)
+    phi, z = rng.uniform(-np.pi, np.pi, n_hits), rng.uniform(-60.0, 60.0, n_hits)
+    h = np.zeros((n_hits, 9), np.float32)
+    h[:, 0], h[:, 1], h[:, 2], h[:, 3], h[:, 5], h[:, 8] = 20 * np.cos(phi), 20 * np.sin(phi), z, 1e-4, 1e-4, 1e-2
+    return d, h
+
+
+def _tracks(n, rng):
+    tp = rng.uniform(-np.pi, np.pi, n)
+    par = np.stack([20 * np.cos(tp), 20 * np.sin(tp), rng.uniform(-58.0, 58.0, n), np.full(n, 0.5), tp,
+                    rng.uniform(0.6, 2.5, n)]).astype(np.float32)
+    err = np.zeros((21, n), np.float32)
+    err[[0, 2, 5, 9, 14, 20]] = 1e-4
+    return par, err
+
+
+@pytest.mark.parametrize("min_dphi,min_dq,free", [(3.1, 300.0, 0.0002), (3.1, 300.0, 0.002), (0.3, 3.0, 0.01),
+                                                  (0.3, 3.0, 0.1), (1.0, 25.0, 0.0)])
+def test_select_in_windows_of_many_masked_hits(gpu_device, min_dphi, min_dq, free):
+    """Windows of many hits, nearly all of them masked, so that a list fills late or never, scanned by the wavefront
+    or, where it holds too many, by lane; plain windows and ones of many rows; against the oracle."""
+    import torch
+    rng = np.random.default_rng(int(min_dq * 10 + free * 1e4))
+    d, h = _one_layer(60000, rng, min_dphi, min_dq)
+    mask = (rng.random(len(h)) >= free).astype(np.uint8)
+    n = 4000
+    par, err = _tracks(n, rng)
+    ctx = mk.Context(bfield=3.8)
+    eoh = mk.EventOfHits(ctx, [d])
+    eoh.load(np.array([0, len(h)], np.int32), torch.from_numpy(h).to(gpu_device))
+    eoh.set_hit_mask(torch.from_numpy(mask).to(gpu_device))
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu_device)
+
+    def run(m, times=1):
+        xs, xa, w = (t(np.zeros(m * times, np.int32)), t(np.zeros((16, m * times), np.int32)),
+                     t(np.zeros(m * times, np.int32)))
+        eoh.select_hit_indices(0, t(np.tile(par[:, :m], times)), t(np.tile(err[:, :m], times)), xs, xa, w)
+        return xs.cpu().numpy(), xa.cpu().numpy(), w.cpu().numpy()
+    whole = run(n)
+    for m in (1, 5, 900):
+        assert all(np.array_equal(a, b[..., :m]) for a, b in zip(run(m), whole)), m
+    for a, b in zip(run(n, 17), whole):
+        assert np.array_equal(a, np.concatenate([b] * 17, axis=-1))
+    m = 300
+    xs, xa, w = oracle.select_hit_indices(d, h, np.ascontiguousarray(par[:, :m]), np.ascontiguousarray(err[:, :m]), mask)
+    # one float rounding of a bin or window edge moves a lane's list: at most a lane in a hundred
+    same = (xs == whole[0][:m]) & (w == whole[2][:m])
+    for k in range(m):
+        same[k] &= np.array_equal(xa[:max(xs[k], 0), k], whole[1][:max(xs[k], 0), k])
+    assert same.mean() >= 0.99, same.mean()
+    eoh.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 1000, 70000])
+def test_wide_windows_cost_what_sixteen_hits_cost(gpu_device, n):
+    """A list is full at 16 hits: windows over a whole layer of 50k hits take a few times as long as ordinary ones
+    (reading all of every window took a hundred to ten thousand times as long)."""
+    import torch
+    took = []
+    for min_dphi, min_dq in ((0.01, 1.0), (3.1, 300.0)):
+        rng = np.random.default_rng(5)
+        d, h = _one_layer(50000, rng, min_dphi, min_dq)
+        par, err = _tracks(n, rng)
+        ctx = mk.Context(bfield=3.8)
+        eoh = mk.EventOfHits(ctx, [d])
+        eoh.load(np.array([0, len(h)], np.int32), torch.from_numpy(h).to(gpu_device))
+        t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu_device)
+        a = [t(par), t(err), t(np.zeros(n, np.int32)), t(np.zeros((16, n), np.int32)), t(np.zeros(n, np.int32))]
+        times = []
+        for _ in range(7):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            eoh.select_hit_indices(0, *a)
+            e1.record()
+            torch.cuda.synchronize()
+            times.append(e0.elapsed_time(e1))
+        took.append(float(np.median(times)))
+        eoh.close()
+        ctx.close()
+    assert took[1] < 20 * took[0], took
