@@ -1,8 +1,8 @@
 // mkf_find.hip -- best-hit track finding on gfx950.
 //
-//   LayerOfHits build   k_row_partition -> k_row_sort (hits by q row, then each row in LDS), or, for layers
-//                       of few q bins and many hits, k_hit_keys -> stable LSD radix sort (hipCUB) ->
-//                       k_loh_gather, k_loh_fill
+//   LayerOfHits build   k_row_partition -> k_row_sort (hits by q row, then each row in LDS) -> k_row_tiles ->
+//                       k_row_units (rows that do not fit there), or, with a layer of millions of hits,
+//                       k_hit_keys -> stable LSD radix sort (hipCUB) -> k_loh_gather, k_loh_fill
 //   SelectHitIndices    k_select (per-operation entry point)
 //   FindTracksBestHit   k_find_best_hit: one lane per seed carries its track
 //                       through every layer with the state in VGPRs; hit
@@ -53,8 +53,15 @@ struct OffsetsArg {
   int tile[kOffChunk + 1];      // first tile of k_row_partition per layer
 };
 
-__global__ void k_set_offsets(OffsetsArg o, LayerDev* __restrict__ L, int* __restrict__ tile_off) {
+// What k_row_sort puts off: the entries of the unit table and the histograms taken so far.
+struct PutOff {
+  int units, hists;
+};
+
+__global__ void k_set_offsets(OffsetsArg o, LayerDev* __restrict__ L, int* __restrict__ tile_off,
+                              PutOff* __restrict__ put) {
   const int l = threadIdx.x;
+  if (o.first == 0 && l == 0) *put = PutOff{0, 0};
   if (l < o.count) {
     L[o.first + l].hit_off = o.off[l];
     L[o.first + l].n_hits = o.off[l + 1] - o.off[l];
@@ -209,12 +216,17 @@ k_loh_fill(int total, int pass, const uint32_t* __restrict__ keys_s, const int* 
 constexpr int kTile = 3072;          // hits per tile; also the LDS capacity of k_row_sort, so one tile's part
 constexpr int kRowCap = kTile;       // of a row always fits
 constexpr int kPartBlock = 512, kRowBlock = 256;
+constexpr int kUnitBlock = 512;
 constexpr int kFineBins = 1025;      // fine phi bins 0..1024 (1024: phi == +pi)
-static_assert(kTile % kPartBlock == 0 && kRowCap % kRowBlock == 0 && kTile <= 0xffff, "tile size");
-// Layers with more hits than this per q bin go through the radix sort: a block reads a row beyond kRowCap once per
-// run of bins that fits, and few rows leave the chip idle (17 layers of 167k hits, rows / radix sort: 116 / 289 us at
-// 1391 hits per bin, 193 / 290 at 6185, 289 / 287 at 10437, 1760 / 285 at 41750).
-constexpr size_t kRowMeanMax = 3 * kRowCap;
+constexpr int kBinMax = 64;          // hits of a fine bin ordered by comparing each with each
+static_assert(kTile % kPartBlock == 0 && kRowCap % kRowBlock == 0 && kRowCap % kUnitBlock == 0 && kTile <= 4096,
+              "tile size; a hit's place in its tile takes 12 bits");
+// Hits of a row that one block orders, reading it once per run of bins that fits.
+constexpr int kRowRuns = 3 * kRowCap;
+// A load with a layer of more hits than this goes through the radix sort, because a put off row's units look into every
+// tile of its layer (one layer, evenly filled / all in one q bin / radix sort: 0.5M hits 49 / 128 / 173 us, 1.05M 110 /
+// 202 / 215, 2M 179 / 364 / 276).
+constexpr size_t kRowLayerMax = (size_t)1 << 21;
 
 // Beyond this many hits the sorted copies are stored past the caches: the 256 MB last-level cache no longer keeps
 // them for the finder (best-hit step, stored past / through the caches: 562 / 516 us at 2.8M hits, 723 / 742 at
@@ -227,6 +239,22 @@ struct RowPair {
   float phi;
   int idx;      // hit index in its layer
 };
+
+// A row that k_row_sort does not order -- of more than kRowRuns hits, or with a crowded fine bin -- is put off:
+// k_row_tiles orders the row's part of each tile by fine bin and index and counts the row's bins (`hist`), and
+// k_row_units writes the row, kRowCap positions per block.  What each block takes is found by searching the parts, so
+// the work is linear in the row but for a few probes per unit and tile, in any distribution over q and phi (17 layers of
+// 167k hits, us, with one block per row in runs, and now: one layer 80 % in two q bins 2854 / 196, all in two bins
+// 6080 / 274; 400k hits in one bin 106004 / 126, in one fine bin 211980 / 86; radix sort 300, 304, 170, 152; evenly
+// filled rows of 11133 / 27833 / 83500 hits, put off and radix sort: 271 / 267 / 263 and 304 / 297 / 298).
+struct RowUnit {
+  int row, start, n;      // the q row, its first position in the layer, its hits
+  int first;              // the unit's first position in the row
+  int hist;               // the row's histogram, or -1: the unit is the whole row
+};
+constexpr int kRowPutOff = -2;       // in row_hist: put off without a histogram; -1: not put off
+// A histogram is kept in parts that tiles add to in turn, because additions to one cache line go one after the other.
+constexpr int kHistParts = 4, kHistWords = kHistParts * (kFineBins + 1);
 
 __device__ __forceinline__ int fine_bin_clamped(float phi) {
   return min(max(phi_bin_fine(phi), 0), kFineBins - 1);
@@ -336,25 +364,92 @@ struct XcdRows {
   int first[9];
 };
 
+// cur (LDS): counts of the fine bins to their starts.
+template <int BLOCK>
+__device__ __forceinline__ void scan_bins(int* cur, int* part, int* crowded) {
+  constexpr int kPer = (kFineBins + BLOCK) / BLOCK;
+  int h[kPer], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int b = threadIdx.x * kPer + k;
+    h[k] = b <= kFineBins ? cur[b] : 0;
+    sum += h[k];
+    if (crowded && h[k] > kBinMax) *crowded = 1;
+  }
+  int total;
+  int e = block_exclusive<BLOCK>(sum, part, &total);
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int b = threadIdx.x * kPer + k;
+    if (b <= kFineBins) cur[b] = e;
+    e += h[k];
+  }
+  __syncthreads();
+}
+
+template <bool NT>
+__device__ __forceinline__ void put_out(float* p, float v) {
+  if (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
+// The m hits listed in order in s_idx (LDS) to sorted positions g0..
+template <int BLOCK, bool NT>
+__device__ __forceinline__ void write_hits(const int* s_idx, int m, int g0, bool barrel, const float* __restrict__ lhits,
+                                           float* __restrict__ shits, float* __restrict__ qs, int* __restrict__ ranks) {
+  struct F3 { float a, b, c; };
+  constexpr int kBatch = 6;
+  for (int f0 = threadIdx.x; f0 < m * 3; f0 += BLOCK * kBatch) {
+    F3 v[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int f = min(f0 + u * BLOCK, m * 3 - 1), h = f / 3;
+      __builtin_memcpy(&v[u], lhits + (size_t)s_idx[h] * 9 + (f - h * 3) * 3, 12);
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int f = f0 + u * BLOCK, h = f / 3;
+      if (f < m * 3) {
+        float* o = shits + (size_t)g0 * 9 + (size_t)f * 3;
+        put_out<NT>(o, v[u].a);
+        put_out<NT>(o + 1, v[u].b);
+        put_out<NT>(o + 2, v[u].c);
+        if (f == h * 3) put_out<NT>(qs + g0 + h, barrel ? v[u].c : hit_r(v[u].a, v[u].b));
+      }
+    }
+  }
+  for (int h = threadIdx.x; h < m; h += BLOCK) ranks[g0 + h] = s_idx[h];
+}
+
+// Range of coarse bin b of a row of n hits at position `start`, its places lo .. hi of the row, `regular` hits below
+// phi = +pi (HitStructures.cc:146-171), as k_loh_fill's two passes leave it: an empty bin 1..255 of a row with hits
+// below phi = +pi holds its insertion point, and the phi = +pi run takes over bin 0.
+__device__ __forceinline__ int2 bin_range(int b, int lo, int hi, int regular, int start, int n) {
+  int2 r = make_int2(start + lo, start + hi);
+  if (regular == 0 || (b == 0 && hi == 0)) r = make_int2(0, 0);
+  if (b == 0 && n > regular) r = make_int2(start + regular, start + n);
+  return r;
+}
+
 // One q row per block; see above.  The pairs of a row come in any order within a
 // tile's part, so the order inside a fine phi bin (one to three hits) is set by
 // comparing indices.  A row that fits the LDS is read once; what it reads from
 // memory is issued in batches, as the block waits on memory for most of its time.
 // Rows beyond the LDS capacity (or of layers with more tiles than threads) go
-// through it in runs of whole fine bins, and a single bin beyond it tile by tile,
-// whose indices ascend.
+// through it in runs of whole fine bins.
 template <bool NT>
 __global__ void __launch_bounds__(kRowBlock)
 k_row_sort(XcdRows xr, const int* __restrict__ row_layer, const LayerDev* __restrict__ L, const int* __restrict__ tile_off,
            const unsigned short* __restrict__ pre, int pre_stride, const RowPair* __restrict__ pairs,
            const float* __restrict__ hits, float* __restrict__ shits, float* __restrict__ phis,
-           float* __restrict__ qs, int* __restrict__ ranks, int* __restrict__ place, int2* __restrict__ bins) {
+           float* __restrict__ qs, int* __restrict__ ranks, int* __restrict__ place, int2* __restrict__ bins,
+           PutOff* __restrict__ put, int* __restrict__ row_hist, int* __restrict__ hist, RowUnit* __restrict__ units) {
   __shared__ int s_idx[kRowCap];
   __shared__ int cur[kFineBins + 1];     // fine bin starts, then (as cursors) the ends of the bins placed so far
   __shared__ int s_seg[kRowBlock];       // each tile's part: first place in the tile << 16 | length
   __shared__ int s_dst[kRowBlock];       // and the place of its first pair among the row's
   __shared__ int part[kRowBlock / 64];
-  __shared__ int s_b1, s_cnt;
+  __shared__ int s_crowded, s_unit, s_hist, s_b1;
   const int t = threadIdx.x;
   const int row = xr.first[blockIdx.x % 8] + blockIdx.x / 8;
   if (row >= xr.first[blockIdx.x % 8 + 1]) return;
@@ -367,6 +462,7 @@ k_row_sort(XcdRows xr, const int* __restrict__ row_layer, const LayerDev* __rest
   int* __restrict__ lplace = place + d.hit_off;
   const float* __restrict__ lhits = hits + (size_t)d.hit_off * 9;
   for (int b = t; b <= kFineBins; b += kRowBlock) cur[b] = 0;
+  if (t == 0) s_crowded = 0;
   int c = 0, before = 0;
   for (int i = t; i < nt; i += kRowBlock) {
     const int a = rp[(size_t)i * pre_stride], len = rp[(size_t)i * pre_stride + 1] - a;
@@ -377,72 +473,28 @@ k_row_sort(XcdRows xr, const int* __restrict__ row_layer, const LayerDev* __rest
   int n, start;                          // hits of the row, its first position in the layer
   s_dst[t] = block_exclusive<kRowBlock>(c, part, &n);
   block_exclusive<kRowBlock>(before, part, &start);
-  int2* __restrict__ brow = bins + d.bin_off + q * kNPhi;
   if (n == 0) {
-    brow[t] = make_int2(0, 0);
+    bins[d.bin_off + q * kNPhi + t] = make_int2(0, 0);
+    if (t == 0) row_hist[row] = -1;
     return;
   }
-  // cur: counts to starts
-  auto scan_bins = [&]() {
-    constexpr int kPer = (kFineBins + kRowBlock) / kRowBlock;
-    int h[kPer], sum = 0;
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      const int b = t * kPer + k;
-      h[k] = b <= kFineBins ? cur[b] : 0;
-      sum += h[k];
-    }
-    int total;
-    int e = block_exclusive<kRowBlock>(sum, part, &total);
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      const int b = t * kPer + k;
-      if (b <= kFineBins) cur[b] = e;
-      e += h[k];
+  auto put_off = [&]() {
+    const int m = (n + kRowCap - 1) / kRowCap;
+    if (t == 0) {
+      s_unit = atomicAdd(&put->units, m);
+      s_hist = m > 1 ? atomicAdd(&put->hists, 1) : -1;
+      row_hist[row] = m > 1 ? s_hist : kRowPutOff;
     }
     __syncthreads();
+    for (int i = t; i < m; i += kRowBlock) units[s_unit + i] = RowUnit{row, start, n, i * kRowCap, s_hist};
+    if (m > 1)
+      for (int b = t; b < kHistWords; b += kRowBlock) hist[(size_t)s_hist * kHistWords + b] = 0;
   };
+  if (n > kRowRuns) {
+    put_off();
+    return;
+  }
   const int gbase = d.hit_off + start;
-  const bool barrel = d.is_barrel != 0;
-  auto put_out = [](float* p, float v) {
-    if (NT) __builtin_nontemporal_store(v, p);
-    else *p = v;
-  };
-  // m hits, ordered in s_idx, to row positions base..
-  auto write_hits = [&](int base, int m) {
-    struct F3 { float a, b, c; };
-    const int g0 = gbase + base;
-    constexpr int kBatch = 6;
-    for (int f0 = t; f0 < m * 3; f0 += kRowBlock * kBatch) {
-      F3 v[kBatch];
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const int f = min(f0 + u * kRowBlock, m * 3 - 1), h = f / 3;
-        __builtin_memcpy(&v[u], lhits + (size_t)s_idx[h] * 9 + (f - h * 3) * 3, 12);
-      }
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const int f = f0 + u * kRowBlock, h = f / 3;
-        if (f < m * 3) {
-          float* o = shits + (size_t)g0 * 9 + (size_t)f * 3;
-          put_out(o, v[u].a);
-          put_out(o + 1, v[u].b);
-          put_out(o + 2, v[u].c);
-          if (f == h * 3) put_out(qs + g0 + h, barrel ? v[u].c : hit_r(v[u].a, v[u].b));
-        }
-      }
-    }
-    for (int h = t; h < m; h += kRowBlock) ranks[g0 + h] = s_idx[h];
-  };
-  auto write_bins = [&](auto&& start_of) {
-    // Bin ranges (HitStructures.cc:146-171), as k_loh_fill's two passes leave them: an empty bin 1..255 of a row
-    // with hits below phi = +pi holds its insertion point, and the phi = +pi run takes over bin 0.
-    const int lo = start_of(4 * t), hi = start_of(4 * t + 4), regular = start_of(1024);
-    int2 r = make_int2(start + lo, start + hi);
-    if (regular == 0 || (t == 0 && hi == 0)) r = make_int2(0, 0);
-    if (t == 0 && n > regular) r = make_int2(start + regular, start + n);
-    brow[t] = r;
-  };
   if (n <= kRowCap && nt <= kRowBlock) {
     // the positions of the row's pairs, 32 lanes per tile's part
     constexpr int kGroups = kRowBlock / 32;
@@ -453,7 +505,7 @@ k_row_sort(XcdRows xr, const int* __restrict__ row_layer, const LayerDev* __rest
     __syncthreads();
     constexpr int kPer = kRowCap / kRowBlock;
     RowPair pr[kPer];
-    int at[kPer];                        // fine bin << 16 | place in it; then the place in the row
+    int at[kPer];                          // fine bin << 16 | place in it; then the place in the row
 #pragma unroll
     for (int k = 0; k < kPer; ++k)
       if (t + k * kRowBlock < n) pr[k] = src[s_idx[t + k * kRowBlock]];
@@ -465,8 +517,13 @@ k_row_sort(XcdRows xr, const int* __restrict__ row_layer, const LayerDev* __rest
       }
     }
     __syncthreads();
-    scan_bins();
-    int at0[kPer];                       // the pairs' positions, kept to write their places there
+    scan_bins<kRowBlock>(cur, part, &s_crowded);
+    if (s_crowded) {
+      put_off();
+      return;
+    }
+    if (t == 0) row_hist[row] = -1;
+    int at0[kPer];                         // the pairs' positions, kept to write their places there
 #pragma unroll
     for (int k = 0; k < kPer; ++k) at0[k] = t + k * kRowBlock < n ? s_idx[t + k * kRowBlock] : 0;
     __syncthreads();
@@ -489,27 +546,32 @@ k_row_sort(XcdRows xr, const int* __restrict__ row_layer, const LayerDev* __rest
     for (int k = 0; k < kPer; ++k)
       if (t + k * kRowBlock < n) s_idx[at[k]] = pr[k].idx;
     __syncthreads();
-    write_hits(0, n);
+    write_hits<kRowBlock, NT>(s_idx, n, gbase, d.is_barrel != 0, lhits, shits, qs, ranks);
     __syncthreads();
     float* s_phi = reinterpret_cast<float*>(s_idx);
 #pragma unroll
     for (int k = 0; k < kPer; ++k)
       if (t + k * kRowBlock < n) s_phi[at[k]] = pr[k].phi;
     __syncthreads();
-    for (int h = t; h < n; h += kRowBlock) put_out(phis + gbase + h, s_phi[h]);
-    write_bins([&](int b) { return cur[b]; });
+    for (int h = t; h < n; h += kRowBlock) put_out<NT>(phis + gbase + h, s_phi[h]);
+    bins[d.bin_off + q * kNPhi + t] = bin_range(t, cur[4 * t], cur[4 * t + 4], cur[1024], start, n);
     return;
   }
   // every pair of the row, 16 lanes per tile's part: f(pair, its position)
-  auto each_pair = [&](int i0, int i1, auto&& f) {
-    for (int i = i0 + (t >> 4); i < i1; i += kRowBlock / 16) {
+  auto each_pair = [&](auto&& f) {
+    for (int i = t >> 4; i < nt; i += kRowBlock / 16) {
       const int lo = rp[(size_t)i * pre_stride], hi = rp[(size_t)i * pre_stride + 1];
       for (int j = lo + (t & 15); j < hi; j += 16) f(src[i * kTile + j], i * kTile + j);
     }
   };
-  each_pair(0, nt, [&](const RowPair& p, int) { atomicAdd(&cur[fine_bin_clamped(p.phi)], 1); });
+  each_pair([&](const RowPair& p, int) { atomicAdd(&cur[fine_bin_clamped(p.phi)], 1); });
   __syncthreads();
-  scan_bins();
+  scan_bins<kRowBlock>(cur, part, &s_crowded);
+  if (s_crowded) {
+    put_off();
+    return;
+  }
+  if (t == 0) row_hist[row] = -1;
   // Puts each of the m entries (s_idx: the pairs' positions), whose equal-bin group lies at [x, y) = group(phi), at
   // its place by index, from row position `base` on; then s_idx holds hit indices.
   auto order = [&](int base, int m, auto&& group) {
@@ -553,51 +615,90 @@ k_row_sort(XcdRows xr, const int* __restrict__ row_layer, const LayerDev* __rest
     for (int b = b0 + 1 + t; b <= kFineBins; b += kRowBlock)
       if (cur[b] - base <= kRowCap) atomicMax(&s_b1, b);
     __syncthreads();
-    const int b1 = s_b1;
-    if (b1 > b0) {
-      const int m = cur[b1] - base;      // cur[kFineBins] == n
-      __syncthreads();
-      each_pair(0, nt, [&](const RowPair& p, int at) {
-        const int b = fine_bin_clamped(p.phi);
-        if (b >= b0 && b < b1) s_idx[atomicAdd(&cur[b], 1) - base] = at;
-      });
-      __syncthreads();
-      order(base, m, [&](float phi) {
-        const int b = fine_bin_clamped(phi);
-        return make_int2((b > b0 ? cur[b - 1] : base) - base, cur[b] - base);
-      });
-      write_hits(base, m);
-      b0 = b1;
-    } else {                             // one bin beyond the capacity
-      int done = 0;
-      for (int i = 0; i < nt; ++i) {
-        if (t == 0) s_cnt = 0;
-        __syncthreads();
-        each_pair(i, i + 1, [&](const RowPair& p, int at) {
-          if (fine_bin_clamped(p.phi) == b0) s_idx[atomicAdd(&s_cnt, 1)] = at;
-        });
-        __syncthreads();
-        const int m = s_cnt;
-        order(base + done, m, [&](float) { return make_int2(0, m); });
-        write_hits(base + done, m);
-        done += m;
-        __syncthreads();
-      }
-      if (t == 0) cur[b0] = base + done;
-      ++b0;
-    }
+    const int b1 = s_b1;                 // past b0: a bin holds at most kBinMax
+    const int m = cur[b1] - base;        // cur[kFineBins] == n
+    __syncthreads();
+    each_pair([&](const RowPair& p, int at) {
+      const int b = fine_bin_clamped(p.phi);
+      if (b >= b0 && b < b1) s_idx[atomicAdd(&cur[b], 1) - base] = at;
+    });
+    __syncthreads();
+    order(base, m, [&](float phi) {
+      const int b = fine_bin_clamped(phi);
+      return make_int2((b > b0 ? cur[b - 1] : base) - base, cur[b] - base);
+    });
+    write_hits<kRowBlock, NT>(s_idx, m, gbase + base, d.is_barrel != 0, lhits, shits, qs, ranks);
+    b0 = b1;
     __syncthreads();
   }
-  write_bins([&](int b) { return b > 0 ? cur[b - 1] : 0; });
+  // the cursors stand at the bins' ends
+  const int c0 = t > 0 ? cur[4 * t - 1] : 0, c1 = cur[4 * t + 3], regular = cur[1023];
+  bins[d.bin_off + q * kNPhi + t] = bin_range(t, c0, c1, regular, start, n);
 }
 
-// The inverse map of a tile's hits from their pairs' places, turned into hit order in LDS.  (Scattering it from
+// Place of element i of an array being sorted in LDS: a word of padding after every eight, so that lanes' elements a power
+// of two apart lie in different banks.
+constexpr int kSortWords = 4096 + 4096 / 8;
+__device__ __forceinline__ int padded(int i) { return i + (i >> 3); }
+
+// Bitonic sort steps of strides s << (E - 1) .. s on the 2^E elements of a thread, in the direction of level k (the
+// elements' complements ascend where the elements descend).  WHOLE: s is a multiple of eight.
+template <int BLOCK, int E, bool WHOLE>
+__device__ __forceinline__ void bitonic_trip(unsigned* v, int size, int k, int s) {
+  constexpr int kN = 1 << E;
+  for (int i = threadIdx.x; i < size / kN; i += BLOCK) {
+    const int at = (i & ~(s - 1)) * kN + (i & (s - 1)), first = padded(at);
+    const unsigned flip = (at & k) == 0 ? 0u : ~0u;
+    auto element = [&](int e) -> unsigned& { return v[WHOLE ? first + e * (s + (s >> 3)) : padded(at + e * s)]; };
+    unsigned x[kN];
+#pragma unroll
+    for (int e = 0; e < kN; ++e) x[e] = element(e) ^ flip;
+#pragma unroll
+    for (int j = kN / 2; j > 0; j /= 2) {
+#pragma unroll
+      for (int e = 0; e < kN; ++e) {
+        if (e & j) continue;
+        const unsigned lo = min(x[e], x[e + j]), hi = max(x[e], x[e + j]);
+        x[e] = lo;
+        x[e + j] = hi;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kN; ++e) element(e) = x[e] ^ flip;
+  }
+  __syncthreads();
+}
+
+// Ascending sort of `size` padded elements in LDS, size a power of two: up to three strides per trip through the LDS, 32 trips
+// and barriers for 4096 elements in place of the 78 of one stride each.
+template <int BLOCK>
+__device__ __forceinline__ void bitonic_sort(unsigned* v, int size) {
+  for (int k = 2; k <= size; k *= 2) {
+    for (int j = k / 2; j > 0;) {
+      if (j >= 32) bitonic_trip<BLOCK, 3, true>(v, size, k, j / 4);
+      else if (j >= 4) bitonic_trip<BLOCK, 3, false>(v, size, k, j / 4);
+      else if (j == 2) bitonic_trip<BLOCK, 2, false>(v, size, k, 1);
+      else bitonic_trip<BLOCK, 1, false>(v, size, k, 1);
+      j = j >= 4 ? j / 8 : 0;
+    }
+  }
+}
+__device__ __forceinline__ int pow2_at_least(int n) { return n <= 1 ? 1 : 1 << (32 - __clz(n - 1)); }
+
+// Per tile: the inverse map of its hits from their pairs' places, turned into hit order in LDS (scattering it from
 // k_row_sort writes a 32-byte sector per 4-byte entry: 1.0 ms over 141.7M hits, against 0.1 ms there for the
-// places and this kernel.)
-__global__ void __launch_bounds__(kPartBlock)
-k_row_inverse(int n_layers, const int* __restrict__ tile_off, const LayerDev* __restrict__ L,
-              const RowPair* __restrict__ pairs, const int* __restrict__ place, int* __restrict__ inv) {
-  __shared__ int out[kTile];
+// places and this kernel).  Then, where rows were put off, their parts in this tile are ordered by fine bin and index,
+// in place, and their bins counted; k_row_units writes those hits' inverse map again.
+__global__ void __launch_bounds__(kPartBlock) __attribute__((amdgpu_waves_per_eu(8)))
+k_row_tiles(int n_layers, const int* __restrict__ tile_off, const LayerDev* __restrict__ L, RowPair* __restrict__ pairs,
+            const int* __restrict__ place, int* __restrict__ inv, const unsigned short* __restrict__ pre, int pre_stride,
+            const PutOff* __restrict__ put, const int* __restrict__ row_hist, int* __restrict__ hist) {
+  __shared__ unsigned key[kSortWords];
+  __shared__ unsigned short s_at[kTile];             // hit of the tile -> its pair's position
+  __shared__ unsigned short s_row[kMaxQBins + 1];
+  __shared__ int s_hist[kMaxQBins];
+  __shared__ int s_lo, s_hi;
+  int* out = reinterpret_cast<int*>(key);
   const int t = threadIdx.x, tile = blockIdx.x;
   const int l = layer_of_tile(tile, n_layers, tile_off);
   const LayerDev& d = L[l];
@@ -616,6 +717,199 @@ k_row_inverse(int n_layers, const int* __restrict__ tile_off, const LayerDev* __
     if (t + k * kPartBlock < n) out[idx[k] - first] = p[k];
   __syncthreads();
   for (int j = t; j < n; j += kPartBlock) inv[g0 + j] = out[j];
+  if (put->units == 0) return;
+  for (int q = t; q <= d.nq; q += kPartBlock) {
+    s_row[q] = pre[(size_t)tile * pre_stride + q];
+    if (q < d.nq) s_hist[q] = row_hist[d.bin_off / kNPhi + q];
+  }
+  // Key: q bin (of half of them at a time), then fine bin and hit of a pair to order, or position of one that stays.
+  constexpr int kQHalf = 512;
+  static_assert(2 * kQHalf == kMaxQBins, "9 bits of a key hold half of the q bins");
+  for (int q0 = 0; q0 < d.nq; q0 += kQHalf) {
+    const int q1 = min(q0 + kQHalf, d.nq);
+    __syncthreads();
+    if (t == 0) {
+      s_lo = n;
+      s_hi = 0;
+    }
+    __syncthreads();
+    // the span from the first put off row's part to the last's
+    for (int q = q0 + t; q < q1; q += kPartBlock) {
+      if (s_hist[q] != -1 && s_row[q + 1] > s_row[q]) {
+        atomicMin(&s_lo, (int)s_row[q]);
+        atomicMax(&s_hi, (int)s_row[q + 1]);
+      }
+    }
+    __syncthreads();
+    const int lo = s_lo, m = s_hi - lo;
+    if (m <= 0) continue;
+    const int size = pow2_at_least(m);
+    RowPair* __restrict__ src = pairs + g0 + lo;
+    RowPair pr[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) pr[k] = src[min(t + k * kPartBlock, m - 1)];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int j = t + k * kPartBlock;
+      if (j >= m) continue;
+      int a = q0;                                // the last row that starts at or before the position
+#pragma unroll
+      for (int step = kQHalf / 2; step > 0; step /= 2)
+        if (a + step < q1 && s_row[a + step] <= lo + j) a += step;
+      unsigned in = j;
+      if (s_hist[a] != -1) {
+        in = (unsigned)fine_bin_clamped(pr[k].phi) << 12 | (unsigned)(pr[k].idx - first);
+        s_at[pr[k].idx - first] = (unsigned short)j;
+      }
+      key[padded(j)] = (unsigned)(a - q0) << 23 | in;
+    }
+    for (int j = m + t; j < size; j += kPartBlock) key[padded(j)] = ~0u;
+    __syncthreads();
+    bitonic_sort<kPartBlock>(key, size);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int j = t + k * kPartBlock;
+      if (j < m && s_hist[q0 + (int)(key[padded(j)] >> 23)] != -1) pr[k] = src[s_at[key[padded(j)] & 0xfff]];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int j = t + k * kPartBlock;
+      if (j >= m) continue;
+      const unsigned v = key[padded(j)] >> 12;           // q bin and fine bin
+      const int h = s_hist[q0 + (int)(v >> 11)];
+      if (h == -1) continue;
+      src[j] = pr[k];
+      if (h < 0) continue;
+      // a run of equal bins adds its length
+      const int add = (j + 1 == m || key[padded(j + 1)] >> 12 != v ? j + 1 : 0) - (j == 0 || key[padded(j - 1)] >> 12 != v ? j : 0);
+      if (add) atomicAdd(&hist[(size_t)h * kHistWords + tile % kHistParts * (kFineBins + 1) + (int)(v & 0x7ff)], add);
+    }
+  }
+}
+
+// A put off row's positions first .. first + kRowCap.  Its tiles' parts are ordered by fine bin and index, and tiles
+// follow each other by index, so the position of a part's first pair of a bin is the bin's start plus the bin's pairs
+// in the tiles before: with those of the unit's first and last bin every tile's share of the unit is known.  Ordering
+// the shares, tile by tile in the list, by bin and place in the list gives the row's order.  Each XCD takes a contiguous
+// eighth of the units, so that units of a row, whose hits share lines, share an L2.
+template <bool NT>
+__global__ void __launch_bounds__(kUnitBlock)
+k_row_units(const PutOff* __restrict__ put, const RowUnit* __restrict__ units, const int* __restrict__ hist,
+            const int* __restrict__ row_layer, const LayerDev* __restrict__ L, const int* __restrict__ tile_off,
+            const unsigned short* __restrict__ pre, int pre_stride, const RowPair* __restrict__ pairs,
+            const float* __restrict__ hits, float* __restrict__ shits, float* __restrict__ phis, float* __restrict__ qs,
+            int* __restrict__ ranks, int* __restrict__ inv, int2* __restrict__ bins) {
+  __shared__ unsigned key[kSortWords];   // fine bin << 12 | place in the list; then the hits in order
+  __shared__ int s_pos[kRowCap];         // the list: the pairs' positions
+  __shared__ int cur[kFineBins + 1];     // the row's fine bin starts
+  __shared__ int s_from[kUnitBlock], s_len[kUnitBlock], s_dst[kUnitBlock];
+  __shared__ int part[kUnitBlock / 64];
+  __shared__ int s_b0, s_b1;
+  const int t = threadIdx.x, n_units = put->units;
+  const int share = (n_units + 7) / 8, u1 = min(n_units, (int)(blockIdx.x % 8 + 1) * share);
+  for (int u = blockIdx.x % 8 * share + blockIdx.x / 8; u < u1; u += gridDim.x / 8) {
+    const RowUnit w = units[u];
+    const int layer = row_layer[w.row];
+    const LayerDev& d = L[layer];
+    const int q = w.row - d.bin_off / kNPhi;
+    const int nt = (d.n_hits + kTile - 1) / kTile;
+    const unsigned short* __restrict__ rp = pre + (size_t)tile_off[layer] * pre_stride + q;
+    const RowPair* __restrict__ src = pairs + d.hit_off;
+    const int p0 = w.first, p1 = min(w.n, p0 + kRowCap), m = p1 - p0;
+    const bool whole = w.hist < 0;
+    __syncthreads();                     // the LDS of the unit before is read
+    for (int b = t; b <= kFineBins; b += kUnitBlock) {
+      int sum = 0;
+      for (int c = 0; c < kHistParts && !whole; ++c) sum += hist[(size_t)w.hist * kHistWords + c * (kFineBins + 1) + b];
+      cur[b] = sum;
+    }
+    __syncthreads();
+    int b0 = 0, b1 = 0;
+    if (!whole) {
+      scan_bins<kUnitBlock>(cur, part, nullptr);
+      for (int b = t; b < kFineBins; b += kUnitBlock) {
+        if (cur[b] <= p0 && p0 < cur[b + 1]) s_b0 = b;
+        if (cur[b] < p1 && p1 <= cur[b + 1]) s_b1 = b;
+      }
+      __syncthreads();
+      b0 = s_b0;
+      b1 = s_b1;
+    }
+    int done0 = 0, done1 = 0, listed = 0;        // pairs of bins b0 and b1 in the tiles before; pairs in the list
+    for (int i0 = 0; i0 < nt; i0 += kUnitBlock) {
+      const int i = i0 + t;
+      int from = 0, to = 0;
+      if (i < nt) {
+        from = i * kTile + rp[(size_t)i * pre_stride];
+        to = i * kTile + rp[(size_t)i * pre_stride + 1];
+      }
+      if (!whole) {
+        // the part's first pair at or past bins b0, b0 + 1, b1, b1 + 1
+        int at[4] = {from, from, from, from};
+        for (int step = pow2_at_least(to - from + 1); step > 0; step >>= 1) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const int b = k < 2 ? b0 + k : b1 + k - 2;
+            if (at[k] + step <= to && fine_bin_clamped(src[at[k] + step - 1].phi) < b) at[k] += step;
+          }
+        }
+        int all;
+        const int g0 = cur[b0] + done0 + block_exclusive<kUnitBlock>(at[1] - at[0], part, &all);
+        done0 += all;
+        const int g1 = cur[b1] + done1 + block_exclusive<kUnitBlock>(at[3] - at[2], part, &all);
+        done1 += all;
+        from = at[0] + min(max(p0 - g0, 0), at[1] - at[0]);
+        to = at[2] + min(max(p1 - g1, 0), at[3] - at[2]);
+      }
+      int all;
+      const int dst = listed + block_exclusive<kUnitBlock>(to - from, part, &all);
+      listed += all;
+      s_from[t] = from;
+      s_len[t] = to - from;
+      s_dst[t] = dst;
+      __syncthreads();
+      for (int k = t >> 5; k < min(kUnitBlock, nt - i0); k += kUnitBlock / 32)
+        for (int j = t & 31; j < s_len[k]; j += 32) s_pos[s_dst[k] + j] = s_from[k] + j;
+      __syncthreads();
+    }
+    const int size = b0 == b1 && !whole ? 0 : pow2_at_least(m);
+    constexpr int kPer = kRowCap / kUnitBlock;
+    RowPair pr[kPer];
+    if (size) {
+#pragma unroll
+      for (int k = 0; k < kPer; ++k) pr[k] = src[s_pos[min(t + k * kUnitBlock, m - 1)]];
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int j = t + k * kUnitBlock;
+      if (j >= m) continue;
+      const int b = size ? fine_bin_clamped(pr[k].phi) : 0;
+      if (whole) atomicAdd(&cur[b], 1);
+      key[padded(j)] = (unsigned)(b << 12 | j);
+    }
+    for (int j = m + t; j < size; j += kUnitBlock) key[padded(j)] = ~0u;
+    __syncthreads();
+    bitonic_sort<kUnitBlock>(key, size);
+    const int g = d.hit_off + w.start + p0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (t + k * kUnitBlock < m) pr[k] = src[s_pos[key[padded(t + k * kUnitBlock)] & 0xfff]];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int j = t + k * kUnitBlock;
+      if (j < m) {
+        key[j] = pr[k].idx;
+        put_out<NT>(phis + g + j, pr[k].phi);
+        inv[d.hit_off + pr[k].idx] = g + j;
+      }
+    }
+    if (whole) scan_bins<kUnitBlock>(cur, part, nullptr);
+    __syncthreads();
+    write_hits<kUnitBlock, NT>(reinterpret_cast<const int*>(key), m, g, d.is_barrel != 0, hits + (size_t)d.hit_off * 9, shits, qs, ranks);
+    if (p0 == 0 && t < kNPhi) bins[d.bin_off + q * kNPhi + t] = bin_range(t, cur[4 * t], cur[4 * t + 4], cur[1024], w.start, w.n);
+  }
 }
 
 // Per-hit bytes (the iteration's hit mask, as 0 or 1, or the charge codes) in sorted order, one tile of sorted
@@ -887,15 +1181,20 @@ void free_hit_arrays(mkf_event_of_hits* h) {
 
 size_t aligned(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
-// A load's scratch for up to `cap` hits, whichever way they are sorted and however they lie over the layers.
+// A load's scratch for up to `cap` hits, whichever way they are sorted and however they lie over the layers and rows.
 struct RowScratch {
-  size_t place, pre, bytes;       // offsets of the places and row starts behind the pairs
+  size_t place, pre, put, row_hist, hist, units, bytes;       // offsets behind the pairs
 };
 RowScratch row_scratch(const mkf_event_of_hits* h, size_t cap) {
+  const size_t n_rows = h->total_bins / kNPhi;
   RowScratch r;
   r.place = aligned(cap * sizeof(RowPair));
   r.pre = r.place + aligned(cap * 4);
-  r.bytes = r.pre + (cap / kTile + h->n_layers) * (size_t)(h->max_nq + 1) * sizeof(unsigned short);
+  r.put = r.pre + aligned((cap / kTile + h->n_layers) * (size_t)(h->max_nq + 1) * sizeof(unsigned short));
+  r.row_hist = r.put + aligned(sizeof(PutOff));
+  r.hist = r.row_hist + aligned(n_rows * 4);
+  r.units = r.hist + aligned(cap / (kRowCap + 1) * kHistWords * 4);     // rows of more than kRowCap hits
+  r.bytes = r.units + (n_rows + cap / kRowCap) * sizeof(RowUnit);            // ceil(n / kRowCap) a row
   return r;
 }
 int radix_scratch(size_t cap, size_t* temp, size_t* bytes) {
@@ -1033,13 +1332,12 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
   if (total >= ((size_t)1 << 31) - 1) return fail(MKF_ERR_INVALID_ARG, "too many hits in one event of hits");
   if (total) CHECK(check_dev(hits, total * 9 * 4, "hits"));
   hipStream_t st = (hipStream_t)stream;
-  // Which way the hits are sorted: by q rows, unless a layer has so few q bins for its hits that one block per
-  // row would take longer than the radix sort of all.
-  bool rows = true;
+  bool rows = true, put_off = false;            // put_off: a row may be (its layer holds more than kBinMax hits)
   int tiles = 0;
   for (int l = 0; l < L; ++l) {
     const size_t nl = (size_t)hit_offset[l + 1] - hit_offset[l];
-    rows = rows && nl <= kRowMeanMax * h->layers[l].nq;
+    rows = rows && nl <= kRowLayerMax;
+    put_off = put_off || nl > (size_t)kBinMax;
     tiles += (int)((nl + kTile - 1) / kTile);
   }
   const int pre_stride = h->max_nq + 1;
@@ -1050,6 +1348,9 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
     h->layers[l].hit_off = hit_offset[l];
     h->layers[l].n_hits = hit_offset[l + 1] - hit_offset[l];
   }
+  const RowScratch lay = row_scratch(h, h->cap);
+  char* scr = static_cast<char*>(h->d_sort);
+  PutOff* put = reinterpret_cast<PutOff*>(scr + lay.put);
   for (int f = 0, tile = 0; f < L; f += kOffChunk) {
     OffsetsArg o;
     o.first = f;
@@ -1059,16 +1360,17 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
       o.tile[l] = tile;
       if (l < o.count) tile += (h->layers[f + l].n_hits + kTile - 1) / kTile;
     }
-    hipLaunchKernelGGL(k_set_offsets, dim3(1), dim3(kOffChunk), 0, st, o, h->d_layers, h->d_tile_off);
+    hipLaunchKernelGGL(k_set_offsets, dim3(1), dim3(kOffChunk), 0, st, o, h->d_layers, h->d_tile_off, put);
     HIP_TRY(hipGetLastError());
   }
   const int n_rows = h->total_bins / kNPhi;
   if (rows) {
-    const RowScratch lay = row_scratch(h, h->cap);
-    char* scr = static_cast<char*>(h->d_sort);
     RowPair* pairs = reinterpret_cast<RowPair*>(scr);
     int* place = reinterpret_cast<int*>(scr + lay.place);
     unsigned short* pre = reinterpret_cast<unsigned short*>(scr + lay.pre);
+    int* row_hist = reinterpret_cast<int*>(scr + lay.row_hist);
+    int* hist = reinterpret_cast<int*>(scr + lay.hist);
+    RowUnit* units = reinterpret_cast<RowUnit*>(scr + lay.units);
     if (tiles) {
       hipLaunchKernelGGL(k_row_partition, dim3(tiles), dim3(kPartBlock), 0, st, L, h->d_tile_off, h->d_layers, hits,
                          pairs, pre, pre_stride);
@@ -1092,11 +1394,19 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
     for (int k = 0; k < 8; ++k) longest = std::max(longest, xr.first[k + 1] - xr.first[k]);
     hipLaunchKernelGGL((total > kStreamHits ? k_row_sort<true> : k_row_sort<false>), dim3(8 * longest), dim3(kRowBlock), 0,
                        st, xr, h->d_row_layer, h->d_layers, h->d_tile_off, pre, pre_stride, pairs, hits, h->d_shits,
-                       h->d_phis, h->d_qs, h->d_ranks, place, h->d_bins);
+                       h->d_phis, h->d_qs, h->d_ranks, place, h->d_bins, put, row_hist, hist, units);
     HIP_TRY(hipGetLastError());
     if (tiles) {
-      hipLaunchKernelGGL(k_row_inverse, dim3(tiles), dim3(kPartBlock), 0, st, L, h->d_tile_off, h->d_layers, pairs,
-                         place, h->d_inv);
+      hipLaunchKernelGGL(k_row_tiles, dim3(tiles), dim3(kPartBlock), 0, st, L, h->d_tile_off, h->d_layers, pairs, place,
+                         h->d_inv, pre, pre_stride, put, row_hist, hist);
+      HIP_TRY(hipGetLastError());
+    }
+    if (put_off) {
+      // two blocks per CU (122 VGPRs), whole eights for the XCDs' shares
+      const int grid = (std::min(2 * h->ctx->num_cus, n_rows + (int)(total / kRowCap)) + 7) / 8 * 8;
+      hipLaunchKernelGGL((total > kStreamHits ? k_row_units<true> : k_row_units<false>), dim3(grid), dim3(kUnitBlock), 0,
+                         st, put, units, hist, h->d_row_layer, h->d_layers, h->d_tile_off, pre, pre_stride, pairs, hits,
+                         h->d_shits, h->d_phis, h->d_qs, h->d_ranks, h->d_inv, h->d_bins);
       HIP_TRY(hipGetLastError());
     }
     h->loaded = true;
@@ -1106,7 +1416,6 @@ int mkf_event_of_hits_load(mkf_event_of_hits* h, const int* hit_offset, const fl
                      reinterpret_cast<int*>(h->d_bins), (long)h->total_bins * 2, 0);
   HIP_TRY(hipGetLastError());
   const int nt = (int)total;
-  char* scr = static_cast<char*>(h->d_sort);
   uint32_t* keys = reinterpret_cast<uint32_t*>(scr);
   uint32_t* keys_s = reinterpret_cast<uint32_t*>(scr + aligned(h->cap * 4));
   int* vals = reinterpret_cast<int*>(scr + 2 * aligned(h->cap * 4));

@@ -396,7 +396,7 @@ def _rows_of_keys(key, nq):
 @pytest.mark.parametrize("q_bin,is_barrel", [(0.15, 1), (2.0, 1), (30.0, 1), (120.0, 1), (1.5, 0), (60.0, 0)])
 def test_loh_order_for_row_and_tile_sizes(gpu_device, q_bin, is_barrel):
     """Sizes around the tile and row capacity (3072 hits) and one hit or none, from 800 q bins down to one: rows
-    sorted in one go, rows beyond the capacity, and layers whose few bins send the load through the radix sort."""
+    sorted in one go, in runs, and by several blocks."""
     import torch
     rng = np.random.default_rng(int(q_bin * 100) + is_barrel)
     sizes = [0, 1, 3071, 3072, 3073, 0, 9000, 40000, 2]
@@ -423,36 +423,23 @@ def test_loh_order_for_row_and_tile_sizes(gpu_device, q_bin, is_barrel):
     eoh = mk.EventOfHits(ctx, descs)
     eoh.load(off, torch.from_numpy(flat).to(gpu_device))
     for l, h in enumerate(hits):
-        ranks, bins, phis, qs, nq = eoh.layer_views(l)
-        assert sorted(ranks.tolist()) == list(range(len(h)))
-        phi = np.empty_like(phis); phi[ranks] = phis
-        q = np.empty_like(qs); q[ranks] = qs
-        assert np.array_equal(phi, np.arctan2(h[:, 1].astype(np.float64), h[:, 0].astype(np.float64)).astype(np.float32))
-        r2 = h[:, 0].astype(np.float64) ** 2 + h[:, 1].astype(np.float64) ** 2
-        assert np.array_equal(q, h[:, 2]) if is_barrel else np.allclose(q, np.sqrt(r2), rtol=2e-7, atol=0)
-        d = descs[l]
-        lo, hi = np.float32(d["zmin"] if is_barrel else d["rin"]), np.float32(d["zmax"] if is_barrel else d["rout"])
-        extra = np.float32(0.5) * (np.float32(nq) * np.float32(q_bin) - (hi - lo))
-        qb = np.clip(((q - (lo - extra)) * (np.float32(nq) / (hi - lo))).astype(np.int64), 0, nq - 1)
-        key = np.floor(F_PHI_FINE * (phi + np.float32(np.pi))).astype(np.int64) + (qb << 16)
-        assert np.array_equal(ranks, np.argsort(key, kind="stable")), (l, len(h))
-        want = _rows_of_keys(key, nq)
-        full = want[:, 0] < want[:, 1]
-        assert np.array_equal(bins[full], want[full]) and np.all(bins[~full, 0] == bins[~full, 1]), (l, len(h))
-    # the sorted hits and the inverse map, through a selection mask: every hit masked but one stays found as itself
-    keep = int(off[-1]) - 1
-    mask = np.ones(off[-1], np.uint8); mask[keep] = 0
+        _check_layer_of_hits(ctx, eoh, l, descs[l], h, gpu_device)
+    # the mask in sorted order: with every hit masked but one, a search around it finds that one
+    last = sizes.index(9000)
+    h = hits[last]
+    q = h[:, 2] if is_barrel else np.hypot(h[:, 0], h[:, 1])
+    keep = int(np.nonzero(np.abs(q - (0.0 if is_barrel else 25.0)) < 20.0)[0][3])
+    x, y, z = h[keep, :3]
+    mask = np.ones(off[-1], np.uint8)
+    mask[off[last] + keep] = 0
     eoh.set_hit_mask(torch.from_numpy(mask).to(gpu_device))
-    last, n = len(sizes) - 1, 1
-    x, y, z = flat[keep, :3]
-    if abs(z) < 60.0:
-        par = np.array([[x], [y], [z], [0.5], [np.arctan2(y, x)], [1.2]], np.float32)
-        err = np.zeros((21, 1), np.float32)
-        err[[0, 2, 5, 9, 14, 20], 0] = 1e-4
-        t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu_device)
-        xs, xa, w = t(np.zeros(1, np.int32)), t(np.zeros((16, 1), np.int32)), t(np.zeros(1, np.int32))
-        eoh.select_hit_indices(last, t(par), t(err), xs, xa, w)
-        assert xs.item() == 1 and xa[0, 0].item() == sizes[last] - 1
+    par = np.array([[x], [y], [z], [0.5], [np.arctan2(y, x)], [1.2]], np.float32)
+    err = np.zeros((21, 1), np.float32)
+    err[[0, 2, 5, 9, 14, 20], 0] = 1e-4
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu_device)
+    xs, xa, w = t(np.zeros(1, np.int32)), t(np.zeros((16, 1), np.int32)), t(np.zeros(1, np.int32))
+    eoh.select_hit_indices(last, t(par), t(err), xs, xa, w)
+    assert xs.item() == 1 and xa[0, 0].item() == keep
     eoh.close()
     ctx.close()
 
@@ -661,3 +648,197 @@ def test_wide_windows_cost_what_sixteen_hits_cost(gpu_device, n):
         eoh.close()
         ctx.close()
     assert took[1] < 20 * took[0], took
+
+
+def _layer_desc(q_bin=0.5, is_barrel=1):
+    return dict(is_barrel=is_barrel, rin=19.99 if is_barrel else 2.0, rout=20.01 if is_barrel else 50.0,
+                zmin=-60.0 if is_barrel else 29.99, zmax=60.0 if is_barrel else 30.01,
+                propagate_to=20.0 if is_barrel else 30.0, q_bin=q_bin, min_dphi=0.002, max_dphi=0.1, min_dq=0.3,
+                max_dq=2.0, c_dp_sf=1.1, c_dq_sf=1.1, c_c2_sf=1.1)
+
+
+def _hits_at(phi, q, rng, is_barrel=1):
+    """Hits of a layer at phi and q (z, or r on a disk), in random order, each with its own covariance."""
+    n = len(phi)
+    r = 20.0 if is_barrel else q
+    h = np.zeros((n, 9), np.float32)
+    h[:, 0], h[:, 1], h[:, 2] = r * np.cos(phi), r * np.sin(phi), q if is_barrel else 30.0
+    h[phi == np.pi, 1] = 0.0                               # phi of the stored hit is +pi itself
+    h[:, 3], h[:, 5], h[:, 8] = rng.uniform(1e-4, 1e-2, (3, n))
+    return h[rng.permutation(n)]
+
+
+def _check_layer_of_hits(ctx, eoh, l, d, h, dev):
+    """Everything a load leaves of layer l: order, phi, q, bin ranges, and, hit by hit through the inverse map, the
+    sorted copies (an update with the loaded hit against the same update from the event of hits)."""
+    import torch
+    ranks, bins, phis, qs, nq = eoh.layer_views(l)
+    phi = np.arctan2(h[:, 1].astype(np.float64), h[:, 0].astype(np.float64)).astype(np.float32)
+    assert np.array_equal(np.sort(ranks), np.arange(len(h)))
+    assert np.array_equal(phis, phi[ranks])
+    q = np.empty_like(qs)
+    q[ranks] = qs
+    r2 = h[:, 0].astype(np.float64) ** 2 + h[:, 1].astype(np.float64) ** 2
+    assert np.array_equal(q, h[:, 2]) if d["is_barrel"] else np.allclose(q, np.sqrt(r2), rtol=2e-7, atol=0)
+    lo, hi = (np.float32(d[k]) for k in (("zmin", "zmax") if d["is_barrel"] else ("rin", "rout")))
+    extra = np.float32(0.5) * (np.float32(nq) * np.float32(d["q_bin"]) - (hi - lo))
+    qb = np.clip(((q - (lo - extra)) * (np.float32(nq) / (hi - lo))).astype(np.int64), 0, nq - 1)
+    key = np.floor(F_PHI_FINE * (phi + np.float32(np.pi))).astype(np.int64) + (qb << 16)
+    assert np.array_equal(ranks, np.argsort(key, kind="stable"))
+    want = _rows_of_keys(key, nq)
+    full = want[:, 0] < want[:, 1]
+    assert np.array_equal(bins[full], want[full]) and np.all(bins[~full, 0] == bins[~full, 1])
+    n = len(h)
+    if n == 0:
+        return key
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    par = np.tile(np.array([[20.0], [0.5], [1.0], [0.5], [0.1], [1.4]], np.float32), n)
+    err = np.zeros((21, n), np.float32)
+    err[[0, 2, 5, 9, 14, 20]] = np.array([100.0, 80.0, 60.0, 1e-4, 1e-3, 1e-3], np.float32)[:, None]
+    err[1], err[3], err[4] = 5.0, 3.0, -2.0
+    lanes = mk.FinderLanes(t(par), t(err), t(np.ones(n, np.int32)))
+    ctx.update_with_last_hit(eoh, l, lanes, t(np.arange(n, dtype=np.int32)), prop_to_hit=False)
+    out_err, out_par = t(np.zeros_like(err)), t(np.zeros_like(par))
+    ctx.kalman_operation(2, t(err), t(par), t(h[:, 3:].T), t(h[:, :3].T), out_err, out_par, endcap=not d["is_barrel"])
+    got = lanes.numpy()
+    # the same arithmetic in two kernels, whose fused operations may round differently
+    assert np.allclose(got["par"], out_par.cpu().numpy(), rtol=1e-5, atol=1e-4)
+    assert np.allclose(got["err"], out_err.cpu().numpy(), rtol=1e-4, atol=1e-4)
+    return key
+
+
+@pytest.mark.parametrize("is_barrel", [1, 0])
+def test_loh_order_of_full_rows_and_crowded_bins(gpu_device, is_barrel):
+    """Rows and fine phi bins around and beyond what one block orders: whole rows of 3071 to 20000 hits, one fine bin of
+    64, 65, 3072 and 7000 hits over several tiles with others before and after it, runs at phi = +pi, a layer in
+    one q bin, and layers in one fine bin."""
+    import torch
+    rng = np.random.default_rng(91 + is_barrel)
+    u = lambda n: rng.uniform(-np.pi, np.pi, n)
+    qmid = 10.25
+    spread = lambda n: rng.uniform(3.0, 49.0, n)
+    layers = []
+    for n in (3071, 3072, 3073, 6145, 20000):               # one full row among others
+        layers.append((np.concatenate([u(n), u(5000)]), np.concatenate([np.full(n, qmid), spread(5000)])))
+    for n in (64, 65, 3072, 7000):                          # one crowded fine bin, in a row of others
+        layers.append((np.concatenate([rng.uniform(0.501, 0.502, n), u(1500), u(9000)]),
+                       np.concatenate([np.full(n + 1500, qmid), spread(9000)])))
+    for n in (1, 65, 4000):                                 # phi = +pi, alone in its row and not
+        layers.append((np.concatenate([np.full(n, np.pi), u(4000)]), np.concatenate([np.full(n, qmid), spread(4000)])))
+        layers.append((np.concatenate([np.full(n, np.pi), u(700), u(9)]),
+                       np.concatenate([np.full(n + 700, qmid), spread(9)])))
+    layers.append((u(9000), np.full(9000, qmid)))           # one q bin
+    for n in (65, 3072, 3073, 12000):                       # one fine bin, and nothing else
+        layers.append((rng.uniform(0.501, 0.502, n), np.full(n, qmid)))
+    layers.append((u(40), spread(40)))
+    d = _layer_desc(is_barrel=is_barrel)
+    hits = [_hits_at(phi, q, rng, is_barrel) for phi, q in layers]
+    off = np.concatenate([[0], np.cumsum([len(h) for h in hits])]).astype(np.int32)
+    ctx = mk.Context(bfield=3.8)
+    eoh = mk.EventOfHits(ctx, [d] * len(hits))
+    flat = torch.from_numpy(np.concatenate(hits)).to(gpu_device)
+    for _ in range(2):                                      # a second load finds the first one's tables
+        eoh.load(off, flat)
+        crowd = 0
+        for l, h in enumerate(hits):
+            key = _check_layer_of_hits(ctx, eoh, l, d, h, gpu_device)
+            crowd = max(crowd, np.bincount(key).max())
+        assert crowd >= 12000
+    eoh.close()
+    ctx.close()
+
+
+def test_loh_order_beyond_four_million_hits(gpu_device):
+    """Loads whose sorted copies are stored past the caches, with even layers, a skewed one and one in one fine bin."""
+    import torch
+    rng = np.random.default_rng(92)
+    d, n = _layer_desc(), 170_000
+    hits = [_hits_at(rng.uniform(-np.pi, np.pi, n), rng.uniform(-60.0, 60.0, n), rng) for _ in range(4)]
+    hits.append(_hits_at(rng.uniform(-np.pi, np.pi, n), rng.uniform(3.0, 4.0, n), rng))
+    hits.append(_hits_at(rng.uniform(0.501, 0.502, n), np.full(n, 7.1), rng))
+    copies = 26
+    order = [l % len(hits) for l in range(copies)]
+    ctx = mk.Context(bfield=3.8)
+    eoh = mk.EventOfHits(ctx, [d] * copies)
+    dev = [torch.from_numpy(h).to(gpu_device) for h in hits]
+    eoh.load((np.arange(copies + 1) * n).astype(np.int32), torch.cat([dev[i] for i in order]))
+    for l in (0, 3, 4, 5, 20, 23, 25):
+        _check_layer_of_hits(ctx, eoh, l, d, hits[order[l]], gpu_device)
+    eoh.close()
+    ctx.close()
+
+
+def test_loh_order_of_a_layer_of_millions(gpu_device):
+    """Above 2^21 hits in a layer the load goes through the radix sort; just below, through the rows."""
+    import torch
+    rng = np.random.default_rng(94)
+    d = _layer_desc(q_bin=2.0)
+    ctx = mk.Context(bfield=3.8)
+    eoh = mk.EventOfHits(ctx, [d, d])
+    for n in ((1 << 21) + 1, 1 << 21):
+        hits = [_hits_at(rng.uniform(-np.pi, np.pi, m), np.where(rng.random(m) < 0.3, 7.1, rng.uniform(-60.0, 60.0, m)),
+                         rng) for m in (n, 5000)]
+        eoh.load(np.array([0, n, n + 5000], np.int32), torch.from_numpy(np.concatenate(hits)).to(gpu_device))
+        for l in (0, 1):
+            _check_layer_of_hits(ctx, eoh, l, d, hits[l], gpu_device)
+    eoh.close()
+    ctx.close()
+
+
+def test_captured_load_sorts_what_the_buffer_holds(gpu_device):
+    """A load recorded in a graph and replayed on other hits of the same number: which rows are put off is decided on the
+    device, replay by replay."""
+    import torch
+    rng = np.random.default_rng(95)
+    d, n = _layer_desc(), 15000
+    u = lambda: rng.uniform(-np.pi, np.pi, n)
+    kinds = [(u(), rng.uniform(-60.0, 60.0, n)), (u(), np.full(n, 3.1)), (rng.uniform(0.501, 0.502, n), np.full(n, 3.1)),
+             (u(), rng.uniform(-60.0, 60.0, n))]
+    hits = [_hits_at(phi, q, rng) for phi, q in kinds]
+    ctx = mk.Context(bfield=3.8)
+    eoh = mk.EventOfHits(ctx, [d, d])
+    off = np.array([0, n, 2 * n], np.int32)
+    buf = torch.from_numpy(np.concatenate([hits[0], hits[0]])).to(gpu_device)
+    eoh.load(off, buf)                       # allocates
+    torch.cuda.synchronize()
+    g, st = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(g, stream=st):
+        eoh.load(off, buf)
+    for a, b in ((1, 0), (2, 1), (0, 3), (3, 2)):
+        buf.copy_(torch.from_numpy(np.concatenate([hits[a], hits[b]])).to(gpu_device))
+        g.replay()
+        torch.cuda.synchronize()
+        _check_layer_of_hits(ctx, eoh, 0, d, hits[a], gpu_device)
+        _check_layer_of_hits(ctx, eoh, 1, d, hits[b], gpu_device)
+    del g
+    eoh.close()
+    ctx.close()
+
+
+def test_load_time_does_not_depend_on_the_distribution(gpu_device):
+    """Hits crowded into two q bins, into one, or into one fine bin load within a few times an even layer's time (one
+    block per full row took up to a thousand times as long)."""
+    import torch
+    rng = np.random.default_rng(93)
+    n, d = 150_000, _layer_desc()
+    u = lambda: rng.uniform(-np.pi, np.pi, n)
+    kinds = [(u(), rng.uniform(-60.0, 60.0, n)), (u(), rng.uniform(3.0, 4.0, n)), (u(), np.full(n, 3.1)),
+             (rng.uniform(0.501, 0.502, n), np.full(n, 3.1))]
+    ctx = mk.Context(bfield=3.8)
+    took = []
+    for phi, q in kinds:
+        h = torch.from_numpy(_hits_at(phi, q, rng)).to(gpu_device).repeat(4, 1)
+        eoh = mk.EventOfHits(ctx, [d] * 4)
+        off = (np.arange(5) * n).astype(np.int32)
+        times = []
+        for _ in range(7):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            eoh.load(off, h)
+            e1.record()
+            torch.cuda.synchronize()
+            times.append(e0.elapsed_time(e1))
+        took.append(float(np.median(times)))
+        eoh.close()
+    assert max(took) < 10 * took[0], took
+    ctx.close()
