@@ -85,7 +85,6 @@ __device__ __forceinline__ uint64_t group_max(uint64_t key, int lane0, int c) {
   }
   return key;
 }
-constexpr int kCeWavesPerCu = 8, kStdWavesPerCu = 6;   // workgroups whose LDS fits a CU
 
 struct Cand {
   float par[6], err[21];
@@ -715,7 +714,7 @@ int find_combinatorial(mkf_context* c, mkf_event_of_hits* h, const mkf_ce_batch*
   if (h->ctx != c) return fail(MKF_ERR_INVALID_ARG, "event of hits belongs to another context");
   if (!h->loaded) return fail(MKF_ERR_INVALID_ARG, "event of hits not loaded");
   if (b->n_seeds < 0) return fail(MKF_ERR_INVALID_ARG, "n_seeds < 0");
-  for (const LayerDev& ld : h->layers)                      
+  for (const LayerDev& ld : h->layers)
     if (ld.n_hits > kMaxLayerHits)
       return fail(MKF_ERR_INVALID_ARG, "a layer holds %d hits, above %d", ld.n_hits, kMaxLayerHits);
   const int LE = b->n_layers ? b->n_layers : h->n_layers;   // layers per event
@@ -788,24 +787,22 @@ int find_combinatorial(mkf_context* c, mkf_event_of_hits* h, const mkf_ce_batch*
   const mkf_find_shape sh = c->find_shape[standard ? 1 : 0];
   const int slots = sh.slots ? sh.slots : (b->max_cands <= 6 ? 6 : 8);
   if (slots < b->max_cands) return fail(MKF_ERR_INVALID_ARG, "find shape: %d slots < max_cands %d", slots, b->max_cands);
-  // Seeds per wavefront: as few as put every wavefront on the chip at once.  A lone wavefront leaves its SIMD waiting
-  // for its own results half of the time and its phases grow with its seeds' windows and pairs, but one more than
-  // fit wait for a whole launch (one 10k-seed event, 10 / 9 / 6 / 5 / 4 / 2 seeds per wavefront: 704 / 692 / 627 /
-  // 612 / 889 / 1093 us; standard finding of 5003 seeds, 10 / 4 / 3 / 2: 660 / 594 / 886 / 842 us; 500 seeds, 10 / 1:
-  // 607 / 432 us).
-  const size_t resident = (size_t)c->num_cus * std::min(4 * sh.waves_per_simd, standard ? kStdWavesPerCu : kCeWavesPerCu);
-  a.spw = (int)std::min<size_t>(kLanes / slots, (N + resident - 1) / resident);
-  const int grid = (int)((N + a.spw - 1) / a.spw);
+  using Kernel = void (*)(CeArgs);
+  static const Kernel kernels[8] = {
+      k_find_clone_engine<6, false, 2>, k_find_clone_engine<6, false, 1>, k_find_clone_engine<6, true, 2>,
+      k_find_clone_engine<6, true, 1>,  k_find_clone_engine<8, false, 2>, k_find_clone_engine<8, false, 1>,
+      k_find_clone_engine<8, true, 2>,  k_find_clone_engine<8, true, 1>};
   const int sel = (slots == 8 ? 4 : 0) | (standard ? 2 : 0) | (sh.waves_per_simd == 1 ? 1 : 0);
-  switch (sel) {
-#define MKF_CE_CASE(I, KS, STD, W)                                                                   \
-    case I:                                                                                          \
-      hipLaunchKernelGGL((k_find_clone_engine<KS, STD, W>), dim3(grid), dim3(kLanes), 0, st, a);     \
-      break;
-    MKF_CE_CASE(0, 6, false, 2) MKF_CE_CASE(1, 6, false, 1) MKF_CE_CASE(2, 6, true, 2) MKF_CE_CASE(3, 6, true, 1)
-    MKF_CE_CASE(4, 8, false, 2) MKF_CE_CASE(5, 8, false, 1) MKF_CE_CASE(6, 8, true, 2) MKF_CE_CASE(7, 8, true, 1)
-#undef MKF_CE_CASE
+  // Wavefronts a CU holds, by the registers and LDS the variant was compiled to (8 and, standard, 6; 4 of <8, false, 1>).
+  int per_cu = c->ce_per_cu[sel].load(std::memory_order_relaxed);
+  if (!per_cu) {
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernels[sel], kLanes, 0));
+    per_cu = std::max(1, per_cu);
+    c->ce_per_cu[sel].store(per_cu, std::memory_order_relaxed);
   }
+  a.spw = seeds_per_wave(N, kLanes / slots, c->num_cus, per_cu);
+  const int grid = (int)((N + a.spw - 1) / a.spw);
+  hipLaunchKernelGGL(kernels[sel], dim3(grid), dim3(kLanes), 0, st, a);
   HIP_TRY(hipGetLastError());
   return scratch_release(h->ce_done, st);
 }

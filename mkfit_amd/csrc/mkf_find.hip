@@ -1564,7 +1564,7 @@ int mkf_select_hit_indices(mkf_event_of_hits* h, int layer, int n, const float* 
   CHECK(check_dev(xsize, N * 4, "xsize"));
   CHECK(check_dev(xarr, kHitIdxMax * N * 4, "xarr"));
   CHECK(check_dev(wsr, N * 4, "wsr"));
-  const int lanes = lanes_per_wave(N);
+  const int lanes = lanes_per_wave(N, h->ctx->num_cus);
   hipLaunchKernelGGL(k_select, dim3(blocks_for(N, lanes)), dim3(64), 0, (hipStream_t)stream, h->layers[layer], n, lanes,
                      par, err, h->d_bins, h->d_phis, h->d_qs, h->mask(), h->d_ranks, xsize, xarr, wsr);
   HIP_TRY(hipGetLastError());
@@ -1615,7 +1615,7 @@ int mkf_find_tracks_best_hit(mkf_context* c, mkf_event_of_hits* h, const mkf_fin
   a.bins = h->d_bins;
   a.phis = h->d_phis; a.qs = h->d_qs; a.shits = h->d_shits; a.ranks = h->d_ranks;
   a.mask = h->mask();
-  a.spw = lanes_per_wave(N);
+  a.spw = lanes_per_wave(N, h->ctx->num_cus);
   hipLaunchKernelGGL(k_find_best_hit, dim3(blocks_for(N, a.spw)), dim3(64), 0, (hipStream_t)stream, a);
   HIP_TRY(hipGetLastError());
   return MKF_OK;

@@ -12,6 +12,7 @@
 
 #include "../../include/mkfit_amd.h"
 #include "mkf_track_math.h"
+#include "mkf_waves.h"
 
 namespace mkf_find {
 
@@ -342,16 +343,6 @@ __device__ __forceinline__ int wave_scan(bool active, const LayerDev& d, const W
   }
   __syncthreads();
   return active ? min(S.cnt[lane], kHitIdxMax) : 0;
-}
-
-// Lanes of a one-wavefront workgroup given a seed (or candidate): halved from 64 until there is a wavefront per
-// SIMD.  Below, SIMDs idle; above, wavefronts of half-used lanes take turns (best-hit step at 512 / 1024 / 2048 /
-// 4096 wavefronts: one 10k-seed event 357 / 342 / 432 / 432 us, 4 events - / 858 / 933 / 1020 us, 12 events
-// - / 1950 / 2077 / 2311 us; at 500 seeds 1, 2, 4, 8, 16 seeds per wavefront: 286, 292, 298, 313, 345 us).
-inline int lanes_per_wave(size_t n) {
-  int lanes = 64;
-  while (lanes > 1 && n < (size_t)lanes * 1024) lanes /= 2;
-  return lanes;
 }
 
 // getHitSelDynamicChi2Cut (MkFinder.cc:202-220)

@@ -373,7 +373,7 @@ int mkf_add_best_hit(mkf_context* c, mkf_event_of_hits* h, int layer, const mkf_
   a.prop_to_hit = prop_to_hit;
   a.prop_pflags = intra_pflags;
   a.hit_code = hit_code;
-  a.lanes = lanes_per_wave(ln->n);
+  a.lanes = lanes_per_wave(ln->n, c->num_cus);
   hipLaunchKernelGGL(k_add_best_hit, dim3(blocks_for(ln->n, a.lanes)), dim3(64), 0, (hipStream_t)stream, a);
   HIP_TRY(hipGetLastError());
   return MKF_OK;
@@ -397,7 +397,7 @@ int mkf_find_candidates_clone_engine(mkf_context* c, mkf_event_of_hits* h, int l
   a.max_consec = max_consec_holes;
   a.n_entries = n_entries;
   a.entries = entries;
-  a.lanes = lanes_per_wave(ln->n);
+  a.lanes = lanes_per_wave(ln->n, c->num_cus);
   hipLaunchKernelGGL(k_find_candidates, dim3(blocks_for(ln->n, a.lanes)), dim3(64), 0, (hipStream_t)stream, a);
   HIP_TRY(hipGetLastError());
   return MKF_OK;

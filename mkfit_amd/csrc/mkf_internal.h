@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -28,6 +29,7 @@ struct mkf_context {
   float* d_xi = nullptr;
   mkf_launch_shape shape{256, 0, 0, 0};
   mkf_find_shape find_shape[2] = {{0, 2}, {0, 2}};   // clone engine, standard finding
+  std::atomic<int> ce_per_cu[8] = {};                // wavefronts a CU holds by variant, 0: not asked yet
   hipStream_t tune_stream = nullptr;
   std::mutex mu;
   AdjointScratch adj;            // adjoint checkpoints and per-track gradient rows
