@@ -174,10 +174,11 @@ int mkf_num_batched_variants(void);
  * recomputed between on the way back; more of them are kept (down to every
  * layer, which recomputes none) while the scratch allows.  The results do not
  * depend on it.  The context holds the scratch: a call that it cannot hold at
- * the caller's spacing replaces it (draining the device), by up to
- * mkf_set_adjoint_scratch_limit bytes (512 MiB by default) or by what that
- * spacing takes if that is more, or all there is; every other call takes it as
- * it is, so that a captured call stays valid until a call that does not fit. */
+ * the caller's spacing replaces it (draining the device) by what every state
+ * takes, up to mkf_set_adjoint_scratch_limit bytes (512 MiB by default), or by
+ * what that spacing takes if that is more, or all there is; every other call
+ * takes it as it is, so that a captured call stays valid until a call that does
+ * not fit. */
 typedef struct mkf_adjoint_batch {
   int n_tracks, n_layers;
   const float* seed_par;  /* [6][n] */
@@ -200,7 +201,7 @@ typedef struct mkf_adjoint_batch {
 
 int mkf_fit_adjoint(mkf_context* ctx, const mkf_adjoint_batch* batch, void* stream);
 
-/* Bytes up to which a growing scratch of mkf_fit_adjoint keeps more states than checkpoint_every asks for; 0: just
+/* Bytes that a growing scratch of mkf_fit_adjoint may take to keep more states than checkpoint_every asks for; 0: just
  * those.  Scratch already held is not given back. */
 int mkf_set_adjoint_scratch_limit(mkf_context* ctx, size_t bytes);
 

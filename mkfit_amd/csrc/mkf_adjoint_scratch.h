@@ -2,6 +2,7 @@
 // Host code without HIP, so that the policy runs (and is tested) on the CPU.
 #pragma once
 
+#include <algorithm>
 #include <cstddef>
 
 // A call's scratch: the sums' partials (sum_bytes, 256-byte aligned), checkpoints of 27 values, gradient rows.
@@ -34,7 +35,9 @@ struct AdjointScratch {
 // Readies the scratch for a call and returns the spacing to run it at, 0 when the memory is not to be had.  A scratch
 // that holds the call at the caller's spacing is left where it is, whatever more the call could use: its address may
 // stand in a captured graph, and another stream may be in the middle of a capture that a drain would break.  Only a
-// call that it cannot hold replaces it, by as much as `limit` allows and else by what the call needs.
+// call that it cannot hold replaces it: by what it would use with every state kept, or by all of `limit` where that is
+// less, so that a later call of another type or size finds it too; or by what the call needs, if that is more or all
+// there is.
 // drain_free(p): waits for the device, frees p, true on success; alloc(bytes): NULL on failure.
 template <class DrainFree, class Alloc>
 int adjoint_ready(AdjointScratch& s, const AdjointSize& z, DrainFree&& drain_free, Alloc&& alloc) {
@@ -42,13 +45,10 @@ int adjoint_ready(AdjointScratch& s, const AdjointSize& z, DrainFree&& drain_fre
   if (!drain_free(s.p)) return 0;
   s.p = nullptr;
   s.bytes = 0;
-  int every = z.spacing(s.limit);
-  s.p = alloc(z.bytes(every));
-  if (!s.p && every != z.asked) {
-    every = z.asked;
-    s.p = alloc(z.bytes(every));
-  }
+  size_t take = std::max(z.need(), std::min(z.bytes(1), s.limit));
+  s.p = alloc(take);
+  if (!s.p && take > z.need()) s.p = alloc(take = z.need());
   if (!s.p) return 0;
-  s.bytes = z.bytes(every);
-  return every;
+  s.bytes = take;
+  return z.spacing(take);
 }

@@ -57,11 +57,15 @@ int main() {
     s.limit = 0;
     assert(d.ready(s, z) == 5 && s.bytes == z.need());
     AdjointScratch t;
-    t.limit = z.bytes(2);
-    assert(d.ready(t, z) == 2);
+    t.limit = z.bytes(1) - 1;
+    assert(d.ready(t, z) == 2 && t.bytes == t.limit);
+    AdjointSize w = z;                 // another type, which the rest of the limit serves too
+    w.word = 8;
+    assert(w.need() <= t.bytes && d.ready(t, w) == 3 && t.bytes == t.limit);
     AdjointScratch u;                  // a need above the limit, at a spacing far beyond the layers
     u.limit = 1;
-    assert(d.ready(u, size(100000, INT_MAX)) == INT_MAX);
+    assert(d.ready(u, size(100000, INT_MAX)) == 25 && u.bytes == size(100000, 25).need());
+    assert(size(100000, INT_MAX).spacing(1) == INT_MAX);
     assert(size(1000, INT_MAX).spacing(SIZE_MAX) == 1);
   }
   return 0;
