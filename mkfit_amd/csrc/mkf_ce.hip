@@ -54,7 +54,7 @@ constexpr int kW = 37;                // LDS words per exchanged candidate (36 u
 // propagated phi and theta.  Word 36, which put / get leave alone, holds
 // the score of the lane's invalid-hit record from (a) to the new candidates (c).
 constexpr int kXCut = 28, kXPre = 29, kXOff = 30, kXBar = 31, kXTrig = 32, kXScore = 36;
-constexpr int kMaxLayerHits = (1 << 28) - 1;   // hits per layer the finders take
+constexpr int kMaxLayerHits = (1 << 28) - 1;   // most hits of a layer: a limit of the entry points, not of the kernel
 constexpr int kBsW = 40;              // words per seed of the best short candidate store (36 used)
 
 // Ranking key of an entry: its score, then the earlier place in the reference's

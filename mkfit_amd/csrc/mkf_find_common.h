@@ -444,7 +444,7 @@ struct mkf_event_of_hits {
   float* d_shits = nullptr;
   int* d_ranks = nullptr;
   int* d_inv = nullptr;           // event hit index -> sorted position (inverse of ranks)
-  void* d_sort = nullptr;         // a load's scratch: pairs and row starts, or keys and radix sort buffers
+  void* d_sort = nullptr;         // a load's scratch: pairs, row starts and put off rows, or keys and radix sort buffers
   size_t sort_temp = 0;           // radix sort's share of it
   bool loaded = false;
   void* d_ce_nodes = nullptr;     // clone-engine HitOnTrack node store, then its best short candidates

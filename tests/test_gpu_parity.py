@@ -267,7 +267,7 @@ def test_all_batched_variants_identical(gpu_device, fallback):
                 assert ndiff == 0
 
 
-def test_batched_graph_replay(gpu_device):
+def test_repeated_batched_fits_agree(gpu_device):
     import torch
     geo, p, ev, rl, xi = event(2, 5000, 44)
     ctx = mk.Context(p.bfield, rl, xi)
@@ -279,7 +279,7 @@ def test_batched_graph_replay(gpu_device):
         ctx.fit_batched(b)
         torch.cuda.synchronize()
         outs.append((_np(b.par).copy(), _np(b.err).copy(), _np(b.chi2).copy()))
-        _ = torch.ones(1000, device=gpu_device).sum().item()  # eager work between replays
+        _ = torch.ones(1000, device=gpu_device).sum().item()  # other work between the calls
     for o in outs[1:]:
         for x, y in zip(o, outs[0]):
             np.testing.assert_array_equal(x, y)
