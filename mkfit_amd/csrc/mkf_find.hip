@@ -766,15 +766,17 @@ k_row_tiles(int n_layers, const int* __restrict__ tile_off, const LayerDev* __re
     for (int j = m + t; j < size; j += kPartBlock) key[padded(j)] = ~0u;
     __syncthreads();
     bitonic_sort<kPartBlock>(key, size);
+    int t1 = t;
+    asm volatile("" : "+v"(t1));          // the addresses are formed anew, not kept in registers during the sort
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const int j = t + k * kPartBlock;
+      const int j = t1 + k * kPartBlock;
       if (j < m && s_hist[q0 + (int)(key[padded(j)] >> 23)] != -1) pr[k] = src[s_at[key[padded(j)] & 0xfff]];
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const int j = t + k * kPartBlock;
+      const int j = t1 + k * kPartBlock;
       if (j >= m) continue;
       const unsigned v = key[padded(j)] >> 12;           // q bin and fine bin
       const int h = s_hist[q0 + (int)(v >> 11)];
