@@ -1211,6 +1211,7 @@ int grow(mkf_event_of_hits* h, size_t total, hipStream_t st) {
   if (total <= h->cap && h->cap) return MKF_OK;
   HIP_TRY(hipStreamSynchronize(st));
   HIP_TRY(hipDeviceSynchronize());
+  h->loaded = false;              // until this load is through: a failed allocation leaves nothing to search
   free_hit_arrays(h);
   const size_t cap = std::max<size_t>(total, 1024);
   size_t temp = 0, bytes = 0;
@@ -1454,6 +1455,7 @@ int mkf_event_of_hits_set_hit_mask(mkf_event_of_hits* h, const unsigned char* ma
   if (total > h->mask_cap) {
     HIP_TRY(hipStreamSynchronize(st));
     if (h->d_mask_s) HIP_TRY(hipFree(h->d_mask_s));
+    h->has_mask = false;
     h->d_mask_s = nullptr;
     h->mask_cap = 0;
     HIP_TRY(hipMalloc(&h->d_mask_s, total));
@@ -1483,6 +1485,7 @@ int mkf_event_of_hits_set_hit_charge(mkf_event_of_hits* h, const unsigned char* 
   if (total > h->charge_cap) {
     HIP_TRY(hipStreamSynchronize(st));
     if (h->d_charge_s) HIP_TRY(hipFree(h->d_charge_s));
+    h->has_charge = false;
     h->d_charge_s = nullptr;
     h->charge_cap = 0;
     HIP_TRY(hipMalloc(&h->d_charge_s, total));
