@@ -255,8 +255,8 @@ int adjoint_check(const mkf_adjoint_batch* b, AdjointSize& z) {
   return MKF_OK;
 }
 
-// The forward fit, reverse sweep and sums of a checked batch, states kept every `every` layers, with `scr` holding
-// at least AdjointSize::bytes(every).  Every byte of the scratch that a kernel reads is written earlier in the same call.
+// The forward fit, reverse sweep and sums of a checked batch, states kept every `every` layers, with `scr` holding at
+// least AdjointSize::bytes(every).  Every byte of the scratch that a kernel reads is written earlier in the same call.
 int adjoint_launch(const mkf_context* c, const mkf_adjoint_batch* b, int every, void* scr, size_t sum_bytes,
                    hipStream_t st) {
   const size_t N = b->n_tracks, L = b->n_layers;

@@ -218,10 +218,13 @@ constexpr int kRowCap = kTile;       // of a row always fits
 constexpr int kPartBlock = 512, kRowBlock = 256;
 constexpr int kUnitBlock = 512;
 constexpr int kFineBins = 1025;      // fine phi bins 0..1024 (1024: phi == +pi)
-constexpr int kBinMax = 64;          // hits of a fine bin ordered by comparing each with each
+// Hits of a fine bin ordered by comparing each with each; a row with a bin of more is put off (17 layers of 30k / 167k
+// hits in bins of about 24 / 55 / 90 / 200, compared: 50 / 55 / 62 / 86 and 141 / 162 / 183 / 247 us, put off: 125 and 269).
+constexpr int kBinMax = 256;
 static_assert(kTile % kPartBlock == 0 && kRowCap % kRowBlock == 0 && kRowCap % kUnitBlock == 0 && kTile <= 4096,
               "tile size; a hit's place in its tile takes 12 bits");
-// Hits of a row that one block orders, reading it once per run of bins that fits.
+// Hits of a row that one block orders, reading it once per run of bins that fits; a row of more is put off (17 layers of
+// 167k hits, 4175 / 6958 / 11133 / 15308 a row, in runs: 174 / 216 / 282 / 473 us, put off: 334 / 296 / 267 / 269).
 constexpr int kRowRuns = 3 * kRowCap;
 // A load with a layer of more hits than this goes through the radix sort, because a put off row's units look into every
 // tile of its layer (one layer, evenly filled / all in one q bin / radix sort: 0.5M hits 49 / 128 / 173 us, 1.05M 110 /
@@ -244,9 +247,9 @@ struct RowPair {
 // k_row_tiles orders the row's part of each tile by fine bin and index and counts the row's bins (`hist`), and
 // k_row_units writes the row, kRowCap positions per block.  What each block takes is found by searching the parts, so
 // the work is linear in the row but for a few probes per unit and tile, in any distribution over q and phi (17 layers of
-// 167k hits, us, with one block per row in runs, and now: one layer 80 % in two q bins 2854 / 196, all in two bins
-// 6080 / 274; 400k hits in one bin 106004 / 126, in one fine bin 211980 / 86; radix sort 300, 304, 170, 152; evenly
-// filled rows of 11133 / 27833 / 83500 hits, put off and radix sort: 271 / 267 / 263 and 304 / 297 / 298).
+// 167k hits, us, with one block per row in runs, and now: one layer 80 % in two q bins 2854 / 188, all in two bins
+// 6080 / 263; 400k hits in one bin 106004 / 115, in one fine bin 211980 / 82; radix sort 300, 304, 170, 152; evenly
+// filled rows of 11133 / 27833 / 83500 hits, put off and radix sort: 267 / 267 / 263 and 304 / 297 / 298).
 struct RowUnit {
   int row, start, n;      // the q row, its first position in the layer, its hits
   int first;              // the unit's first position in the row
@@ -636,8 +639,8 @@ k_row_sort(XcdRows xr, const int* __restrict__ row_layer, const LayerDev* __rest
   bins[d.bin_off + q * kNPhi + t] = bin_range(t, c0, c1, regular, start, n);
 }
 
-// Place of element i of an array being sorted in LDS: a word of padding after every eight, so that lanes' elements a power
-// of two apart lie in different banks.
+// Place of element i of an array being sorted in LDS: a word of padding after every eight, so that lanes' elements a
+// power of two apart lie in different banks.
 constexpr int kSortWords = 4096 + 4096 / 8;
 __device__ __forceinline__ int padded(int i) { return i + (i >> 3); }
 
@@ -669,8 +672,8 @@ __device__ __forceinline__ void bitonic_trip(unsigned* v, int size, int k, int s
   __syncthreads();
 }
 
-// Ascending sort of `size` padded elements in LDS, size a power of two: up to three strides per trip through the LDS, 32 trips
-// and barriers for 4096 elements in place of the 78 of one stride each.
+// Ascending sort of `size` padded elements in LDS, size a power of two: up to three strides per trip through the LDS,
+// 32 trips and barriers for 4096 elements in place of the 78 of one stride each.
 template <int BLOCK>
 __device__ __forceinline__ void bitonic_sort(unsigned* v, int size) {
   for (int k = 2; k <= size; k *= 2) {
@@ -784,7 +787,8 @@ k_row_tiles(int n_layers, const int* __restrict__ tile_off, const LayerDev* __re
       src[j] = pr[k];
       if (h < 0) continue;
       // a run of equal bins adds its length
-      const int add = (j + 1 == m || key[padded(j + 1)] >> 12 != v ? j + 1 : 0) - (j == 0 || key[padded(j - 1)] >> 12 != v ? j : 0);
+      const bool first_of = j == 0 || key[padded(j - 1)] >> 12 != v, last_of = j + 1 == m || key[padded(j + 1)] >> 12 != v;
+      const int add = (last_of ? j + 1 : 0) - (first_of ? j : 0);
       if (add) atomicAdd(&hist[(size_t)h * kHistWords + tile % kHistParts * (kFineBins + 1) + (int)(v & 0x7ff)], add);
     }
   }
@@ -909,8 +913,10 @@ k_row_units(const PutOff* __restrict__ put, const RowUnit* __restrict__ units, c
     }
     if (whole) scan_bins<kUnitBlock>(cur, part, nullptr);
     __syncthreads();
-    write_hits<kUnitBlock, NT>(reinterpret_cast<const int*>(key), m, g, d.is_barrel != 0, hits + (size_t)d.hit_off * 9, shits, qs, ranks);
-    if (p0 == 0 && t < kNPhi) bins[d.bin_off + q * kNPhi + t] = bin_range(t, cur[4 * t], cur[4 * t + 4], cur[1024], w.start, w.n);
+    write_hits<kUnitBlock, NT>(reinterpret_cast<const int*>(key), m, g, d.is_barrel != 0, hits + (size_t)d.hit_off * 9,
+                               shits, qs, ranks);
+    if (p0 == 0 && t < kNPhi)
+      bins[d.bin_off + q * kNPhi + t] = bin_range(t, cur[4 * t], cur[4 * t + 4], cur[1024], w.start, w.n);
   }
 }
 

@@ -710,7 +710,7 @@ def _check_layer_of_hits(ctx, eoh, l, d, h, dev):
 @pytest.mark.parametrize("is_barrel", [1, 0])
 def test_loh_order_of_full_rows_and_crowded_bins(gpu_device, is_barrel):
     """Rows and fine phi bins around and beyond what one block orders: whole rows of 3071 to 20000 hits, one fine bin of
-    64, 65, 3072 and 7000 hits over several tiles with others before and after it, runs at phi = +pi, a layer in
+    256, 257, 3072 and 7000 hits over several tiles with others before and after it, runs at phi = +pi, a layer in
     one q bin, and layers in one fine bin."""
     import torch
     rng = np.random.default_rng(91 + is_barrel)
@@ -720,15 +720,15 @@ def test_loh_order_of_full_rows_and_crowded_bins(gpu_device, is_barrel):
     layers = []
     for n in (3071, 3072, 3073, 6145, 20000):               # one full row among others
         layers.append((np.concatenate([u(n), u(5000)]), np.concatenate([np.full(n, qmid), spread(5000)])))
-    for n in (64, 65, 3072, 7000):                          # one crowded fine bin, in a row of others
+    for n in (256, 257, 3072, 7000):                        # one crowded fine bin, in a row of others
         layers.append((np.concatenate([rng.uniform(0.501, 0.502, n), u(1500), u(9000)]),
                        np.concatenate([np.full(n + 1500, qmid), spread(9000)])))
-    for n in (1, 65, 4000):                                 # phi = +pi, alone in its row and not
+    for n in (1, 257, 4000):                                # phi = +pi, alone in its row and not
         layers.append((np.concatenate([np.full(n, np.pi), u(4000)]), np.concatenate([np.full(n, qmid), spread(4000)])))
         layers.append((np.concatenate([np.full(n, np.pi), u(700), u(9)]),
                        np.concatenate([np.full(n + 700, qmid), spread(9)])))
     layers.append((u(9000), np.full(9000, qmid)))           # one q bin
-    for n in (65, 3072, 3073, 12000):                       # one fine bin, and nothing else
+    for n in (256, 257, 3072, 3073, 12000):                 # one fine bin, and nothing else
         layers.append((rng.uniform(0.501, 0.502, n), np.full(n, qmid)))
     layers.append((u(40), spread(40)))
     d = _layer_desc(is_barrel=is_barrel)
