@@ -226,10 +226,10 @@ __device__ __forceinline__ int wave_inclusive(int v) {
 // per workgroup.
 //
 // That reads every hit of the windows, while a lane that scans its own window stops at 16 hits.  So when a window
-// holds more than kScanLaneMax chunks, or all more than the work list, each lane scans its own (k_select of 1000 / 30k
-// / 100k windows in us, always by the wavefront, always by lane, and by this rule: 21 chunks a window 17 / 36 / 96,
-// 42 / 48 / 65, 17 / 36 / 53; 200 chunks 62 / 380 / 1371, 50 / 60 / 72, 25 / 39 / 50; a whole layer of 50k hits 3022 /
-// 87738 / 329678, 20 / 17 / 27, 15 / 19 / 23).
+// holds more than kScanLaneMax chunks, or all more than the work list, each lane scans its own (k_select of 1000 / 10k /
+// 30k / 100k windows in us, by the wavefront and by lane: windows of about 23 chunks 11 / 21 / 30 / 42 and 16 / 24 / 26 /
+// 34, 39 chunks 14 / 30 / 45 / 43 and 18 / 28 / 31 / 42, 66 chunks 18 / 42 / 63 / 47 and 20 / 30 / 36 / 45; with nothing
+// but wavefronts at it, windows over a whole layer of 50k hits took 3.0 ms to 330 ms, by this rule 15 to 23 us).
 constexpr int kChunk = 8, kChunkGroups = 64 / kChunk;
 constexpr int kScanDescs = 1024;
 constexpr int kScanLaneMax = 64;
